@@ -129,6 +129,7 @@ struct DevPattern {
   DevBuf far_ptr, far_src, far_order, far_task, far_split;
   DevBuf near_ptr, near_src, near_run, near_order, near_task, near_split;
   int far_top_target = 0, far_top_source = 0;
+  double near_per_task = 0, far_per_task = 0;
   DevPatternView view(const Pattern &p) const {
     DevPatternView v;
     v.far_top_target = far_top_target;
@@ -149,10 +150,18 @@ struct DevPattern {
     v.near_task = near_task.as<int32_t>();
     v.nnear_split = (int)p.near_split.size();
     v.near_split = near_split.as<int32_t>();
+    v.has_far = p.n_far > 0 ? 1 : 0;
+    v.near_per_task = near_per_task;
+    v.far_per_task = far_per_task;
     return v;
   }
-  hipError_t upload(const Pattern &p) {
+  // cols: the source tree of the pattern
+  hipError_t upload(const Pattern &p, const Tree &cols) {
     hipError_t e;
+    double near_sources = 0;
+    for (int32_t src : p.near_src) near_sources += (double)cols.size[src];
+    near_per_task = near_sources / std::max<size_t>(1, p.near_task.size() / 4);
+    far_per_task = (double)p.far_src.size() / std::max<size_t>(1, p.far_task.size() / 4);
     // first far target and source (INT_MAX: no far blocks at all)
     far_top_target = far_top_source = std::numeric_limits<int>::max();
     for (size_t t = 0; t + 1 < p.far_ptr.size(); ++t)
@@ -177,7 +186,7 @@ struct DevPattern {
 
 template <typename T>
 struct Workspace {
-  DevBuf xs, mom, tlhs;
+  DevBuf xs, mom, tlhs, part;
 };
 
 }  // namespace
@@ -376,7 +385,7 @@ fmca_status ensure_device(fmca_h2_actor *a) {
     HIP_TRY(upload_reals<double>(a->d_cols_64, a->cols(), a->pts_cols, unit, a->trans_cols));
     HIP_TRY(upload_reals<float>(a->d_cols_32, a->cols(), a->pts_cols, unit, a->trans_cols));
   }
-  HIP_TRY(a->d_pat.upload(a->pat));
+  HIP_TRY(a->d_pat.upload(a->pat, a->cols()));
   if (a->ip.scheme == IS_TOTAL_DEGREE) {
     const int q = a->ip.q, d = a->dim;
     std::vector<double> un((size_t)d * q);
@@ -456,6 +465,9 @@ struct Region {
   size_t bytes;
 };
 
+// Most bytes of an action's slabs of partial sums.
+constexpr size_t kPartBytes = size_t(256) << 20;
+
 constexpr size_t align_up(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Enqueue one action on `stream`.  transpose swaps the roles of the trees.
@@ -487,6 +499,7 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
   const size_t b_xs = (size_t)t_src.npts * nrhs * sizeof(T);
   const size_t b_mom = (size_t)t_src.ncl * q * nrhs * sizeof(T);
   const size_t b_tlhs = (size_t)t_tgt.ncl * q * nrhs * sizeof(T);
+  const DevPatternView v_pat = dpat->view(*pat);
   ActionBuffers<T> buf;
   if (fixed) {
     // the caller's region: xs | mom | tlhs, each start aligned to 256 bytes
@@ -497,14 +510,27 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
                       " bytes of workspace, the device scratch holds " +
                       std::to_string(fixed->bytes));
     unsigned char *base = static_cast<unsigned char *>(fixed->base);
-    buf = ActionBuffers<T>{reinterpret_cast<T *>(base), reinterpret_cast<T *>(base + o_mom),
-                           reinterpret_cast<T *>(base + o_tlhs)};
+    buf.xs = reinterpret_cast<T *>(base);
+    buf.mom = reinterpret_cast<T *>(base + o_mom);
+    buf.tlhs = reinterpret_cast<T *>(base + o_tlhs);
+    // what is left of the region holds the slabs of phases cut into parts
+    const size_t o_part = std::min(fixed->bytes, o_tlhs + align_up(b_tlhs));
+    T *slabs = reinterpret_cast<T *>(base + o_part);
+    buf.part_cap = (int64_t)((fixed->bytes - o_part) / sizeof(T));
+    buf.part = [slabs](int64_t) { return slabs; };
   } else {
     HIP_TRY(ws.xs.alloc(b_xs));
     HIP_TRY(ws.mom.alloc(b_mom));
     HIP_TRY(ws.tlhs.alloc(b_tlhs));
-    buf = ActionBuffers<T>{ws.xs.template as<T>(), ws.mom.template as<T>(),
-                           ws.tlhs.template as<T>()};
+    buf.xs = ws.xs.template as<T>();
+    buf.mom = ws.mom.template as<T>();
+    buf.tlhs = ws.tlhs.template as<T>();
+    buf.part_cap = (int64_t)(kPartBytes / sizeof(T));
+    buf.part = [&ws](int64_t elems) -> T * {
+      if (ws.part.alloc((size_t)elems * sizeof(T)) == hipSuccess) return ws.part.template as<T>();
+      (void)hipGetLastError();  // no room: the phase runs uncut
+      return nullptr;
+    };
   }
   PhaseEvents *pe = nullptr;
   if (a->profiling && !fixed) {
@@ -539,7 +565,7 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
   }
   KernelParams<T> kp = kernel_params<T>(a, groups);
   kp.split_bf16 = split_bf16 ? 1 : 0;
-  hipError_t e = launch_action<T>(v_rows, v_cols, l_tgt, l_src, dpat->view(*pat),
+  hipError_t e = launch_action<T>(v_rows, v_cols, l_tgt, l_src, v_pat,
                                   interp_params<T>(a), kp, d_rhs, ld_rhs,
                                   (int)nrhs, d_out, ld_out, natural, buf, stream, pe,
                                   use_stored ? &st : nullptr, grad);
@@ -661,7 +687,7 @@ fmca_status enqueue_any_unordered(fmca_h2_actor *a, const double *d_rhs, int64_t
   }
   if (transpose && !a->shared && !a->have_pat_t) {
     compute_pattern(a->pat_t, a->cols(), a->rows(), a->eta, a->ip.q);
-    HIP_TRY(a->d_pat_t.upload(a->pat_t));
+    HIP_TRY(a->d_pat_t.upload(a->pat_t, a->rows()));
     a->have_pat_t = true;
   }
   if (precision == FMCA_PRECISION_FP64)

@@ -3,8 +3,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <functional>
 
 #include "plan.hpp"
 
@@ -57,6 +59,8 @@ struct DevPatternView {
   // ordered, so the tree passes above their levels carry only zeros); 0: no
   // information, the passes run over every level
   int far_top_target = 0, far_top_source = 0;
+  int has_far = 1;                       // 0: no far block at all
+  double near_per_task = 0, far_per_task = 0;  // mean sources / far blocks of a task
 };
 
 // Interpolation data of the kernels.  Tensor scheme: the per-axis Chebyshev
@@ -138,7 +142,32 @@ struct ActionBuffers {
   T *xs = nullptr;    // npts_src x nrhs (point-major, rhs fastest)
   T *mom = nullptr;   // ncl_src x q x nrhs
   T *tlhs = nullptr;  // ncl_tgt x q x nrhs
+  // room for the slabs of partial sums of a phase cut into parts: up to
+  // part_cap elements, given by part(elements) (null: none, the phase runs
+  // uncut)
+  std::function<T *(int64_t)> part;
+  int64_t part_cap = 0;
 };
+
+// Parts of a phase's lists.  A launch of few or of long workgroups leaves CUs
+// idle, at its end above all (n = 1e6, 1 rhs: 16 leaf workgroups per CU, 8 of
+// them resident, kept the CUs 65 % busy).  So the workgroups take grid.y
+// contiguous parts of every task's list, until the launch has about
+// kFillWaves waves (8 rounds of 8 waves per SIMD) or a part has fewer than
+// `least` sources on average.  Part k writes slab k and the slabs are added
+// in order.  Launches with split tasks (nsplit) already add atomically and
+// are not cut further.
+constexpr int kFillWaves = 65536;
+constexpr int kFillWavesMfma = 12288;  // the matrix-core forms: fewer waves per SIMD
+constexpr int kMaxParts = 16;
+inline int phase_parts(int tasks, int nsplit, int waves, double sources, double least,
+                       int64_t slab, int64_t cap, int fill = kFillWaves) {
+  if (nsplit > 0 || tasks <= 0 || slab <= 0) return 1;
+  const double want = std::ceil((double)fill / ((double)tasks * waves));
+  const double most = std::min(sources / least, (double)(cap / slab));
+  const int k = (int)std::min(std::min(want, most), (double)kMaxParts);
+  return k < 2 ? 1 : k;
+}
 
 // Phases of one action, in launch order (timed with events when profiling).
 enum Phase : int {
@@ -243,6 +272,55 @@ hipError_t launch_stored(bool output, const DevTreeView<T> &rows, const DevTreeV
                          const T *xs, const T *mom, T *tlhs, double *out, int64_t ldo,
                          bool natural, hipStream_t stream);
 
+// Adds the slabs of a phase cut into parts (kernels.hip): the coupling sums of
+// all clusters, or the output rows (natural order through perm, or cluster
+// order).
+template <typename T>
+hipError_t launch_add_parts(bool output, const DevTreeView<T> &rows, int q, int nrhs, int parts,
+                            const T *part, T *tlhs, double *out, int64_t ldo, bool natural,
+                            hipStream_t stream);
+
+// Vector-ALU forms of the coupling (output = false) and the leaf output
+// (output = true), kernels_valu.hpp.
+template <typename T>
+struct PhaseLaunch {
+  DevTreeView<T> rows, cols;
+  DevPatternView pat;
+  InterpParams<T> ip;
+  KernelParams<T> kp;
+  int nrhs;
+  const T *xs, *mom;
+  T *tlhs;
+  double *out;
+  int64_t ldo;
+  bool natural;
+  const std::function<T *(int64_t)> &part;
+  int64_t part_cap;
+  hipStream_t stream;
+};
+template <typename T>
+using ValuLaunch = PhaseLaunch<T>;
+template <typename T>
+using MfmaLaunch = PhaseLaunch<T>;
+template <typename T>
+hipError_t launch_valu(bool output, const ValuLaunch<T> &a);
+
+// Parts of a matrix-core launch (256 threads per task) and their slabs.
+template <typename T>
+inline int launch_parts(bool output, const MfmaLaunch<T> &a, T **slabs) {
+  // a part has at least two staged chunks of 128 sources; 3 rounds of the 4
+  // resident waves per SIMD
+  const int64_t slab =
+      (output ? a.rows.npts : (int64_t)a.rows.ncl * a.ip.q) * (int64_t)a.nrhs;
+  int parts = output ? phase_parts(a.pat.nnear_order, a.pat.nnear_split, 4, a.pat.near_per_task,
+                                   256, slab, a.part_cap, kFillWavesMfma)
+                     : phase_parts(a.pat.nfar_order, a.pat.nfar_split, 4,
+                                   a.pat.far_per_task * a.ip.q, 256, slab, a.part_cap,
+                                   kFillWavesMfma);
+  if (parts > 1 && !(*slabs = a.part(parts * slab))) parts = 1;
+  return parts;
+}
+
 // Matrix-core (MFMA) forms of the coupling (output = false) and the leaf
 // output (output = true), used from kMfmaMinRhs right-hand sides on when
 // their LDS fits (td = 1: total-degree scheme).
@@ -265,17 +343,10 @@ bool bf16_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vma
 // The right operand the launch reads (xs for the leaf output, mom for the
 // coupling) is split into BF16 halves in place first, so it holds hi | lo << 16
 // words afterwards.
-hipError_t launch_bf16(bool output, const DevTreeView<float> &rows,
-                       const DevTreeView<float> &cols, const DevPatternView &pat,
-                       const InterpParams<float> &ip, const KernelParams<float> &kp, int nrhs,
-                       float *xs, float *mom, float *tlhs, double *out, int64_t ldo,
-                       bool natural, hipStream_t stream);
+hipError_t launch_bf16(bool output, const MfmaLaunch<float> &a, float *xs, float *mom);
 
 template <typename T>
-hipError_t launch_mfma(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                       const DevPatternView &pat, const InterpParams<T> &ip,
-                       const KernelParams<T> &kp, int nrhs, const T *xs, const T *mom, T *tlhs,
-                       double *out, int64_t ldo, bool natural, hipStream_t stream);
+hipError_t launch_mfma(bool output, const MfmaLaunch<T> &a);
 
 // Column-batched FP64 vector kernels (blas1.hip); columns of n x nrhs arrays.
 size_t blas1_dot_scratch(int nrhs);

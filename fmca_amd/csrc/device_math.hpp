@@ -117,6 +117,75 @@ __device__ __forceinline__ T exp_neg_scaled(T u, const KernelParams<T> &kp) {
     return Math<T>::exp_(-u * kp.s);
 }
 
+// 2^(j / 64), j < 64, rounded to nearest.
+__constant__ double kExp2Table[64] = {
+    1.0, 1.0108892860517005, 1.0218971486541166, 1.0330248790212284,
+    1.0442737824274138, 1.0556451783605572, 1.0671404006768237, 1.0787607977571199,
+    1.0905077326652577, 1.1023825833078409, 1.1143867425958924, 1.1265216186082418,
+    1.1387886347566916, 1.1511892299529827, 1.1637248587775775, 1.1763969916502812,
+    1.189207115002721, 1.2021567314527031, 1.215247359980469, 1.22848053610687,
+    1.241857812073484, 1.2553807570246911, 1.2690509571917332, 1.2828700160787783,
+    1.2968395546510096, 1.3109612115247644, 1.3252366431597413, 1.3396675240533029,
+    1.3542555469368927, 1.3690024229745905, 1.383909881963832, 1.3989796725383112,
+    1.4142135623730951, 1.42961333839197, 1.4451808069770467, 1.460917794180647,
+    1.4768261459394993, 1.4929077282912648, 1.5091644275934228, 1.5255981507445384,
+    1.5422108254079407, 1.5590044002378369, 1.5759808451078865, 1.593142151342267,
+    1.6104903319492543, 1.6280274218573478, 1.6457554781539649, 1.6636765803267364,
+    1.681792830507429, 1.7001063537185235, 1.7186192981224779, 1.7373338352737062,
+    1.7562521603732995, 1.7753764925265212, 1.7947090750031072, 1.8142521755003989,
+    1.8340080864093424, 1.8539791250833855, 1.8741676341103, 1.8945759815869656,
+    1.9152065613971474, 1.9360617934922943, 1.9571441241754002, 1.9784560263879509,
+};
+
+// Entries of the four common kernels in FP64 (the value form of the kernel
+// loops): a root without the exact-zero select and a table exponential.
+//
+// The loops are bound by vector issue (an FP64 operation takes 4.7-5 cycles
+// of a SIMD, v_rsq_f64 16), so the count of operations is what matters:
+//   root:  rsq seed y, then one step of third order on g = x y,
+//          e = 1 - g y, sqrt(x) = g + g e (1/2 + 3/8 e); 5 operations (8 and a
+//          select for Math<double>::sqrt_).  x > 0 is needed: the squared
+//          distances start from kTinyR2 = 1e-300, which leaves every
+//          r2 > 1e-284 as it was and makes k(0) its value at r = 1e-150.
+//   2^(-t / 64): k = rint(t), f = k - t in [-1/2, 1/2], 2^(f / 64) - 1 by its
+//          Taylor polynomial of degree 5 (remainder < 4e-17), times the table
+//          value of -k mod 64 (LDS), scaled by ldexp; 10 operations instead
+//          of 21 for the reduction by ln 2 and a degree-12 polynomial.  The
+//          result carries the rounding of one fma and of the table value.
+// FP64 action, n = 1e4, 1 rhs: 42 -> 27 vector operations per entry.
+constexpr double kTinyR2 = 1e-300;
+
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double g = x * y;
+  const double e = __builtin_fma(-g, y, 1.0);
+  return __builtin_fma(g * e, __builtin_fma(e, 0.375, 0.5), g);
+}
+
+__device__ __forceinline__ double exp2_neg64(double t, const double *tab) {
+  const double k = __builtin_rint(t);
+  const int n = (int)(-k);
+  const double f = k - t;
+  double p = __builtin_fma(f, 1.24178437017169252822e-12, 5.73285168864040188714e-10);
+  p = __builtin_fma(f, p, 2.11731371554647762752e-07);
+  p = __builtin_fma(f, p, 5.86490495505616996649e-05);
+  p = __builtin_fma(f, p, 1.08304246962491450973e-02);
+  const double s = tab[n & 63];
+  return __builtin_ldexp(__builtin_fma(s, f * p, s), n >> 6);
+}
+
+// Copies the table to LDS (64 doubles); the caller synchronises.
+__device__ __forceinline__ void load_exp2_table(double *tab) {
+  for (int j = threadIdx.x; j < 64; j += blockDim.x) tab[j] = kExp2Table[j];
+}
+
+template <int KT, typename T>
+constexpr bool kTableEntry = sizeof(T) == 8 && (KT == KT_EXPONENTIAL || KT == KT_MATERN32 ||
+                                                KT == KT_MATERN52 || KT == KT_GAUSSIAN);
+// start value of a squared distance
+template <int KT, typename T>
+constexpr T kR2Start = kTableEntry<KT, T> ? T(kTinyR2) : T(0);
+
 // Kernel value from the squared distance (CovarianceKernel.h:56-116) with the
 // scales of KernelParams.  KT < 0 selects the type at run time (uniform
 // branch) for the less common kernels.
@@ -242,24 +311,39 @@ __device__ __forceinline__ T kernel_r2(T r2, const KernelParams<T> &kp) {
 // column tile: where it costs extra work (a division, a separate evaluation)
 // it is skipped and left 0.
 template <int KT, typename T>
-__device__ __forceinline__ void kernel_r2_all(T r2, const KernelParams<T> &kp, T ev[3]) {
+__device__ __forceinline__ void kernel_r2_all(T r2, const KernelParams<T> &kp, const double *tab,
+                                              T ev[3]) {
   using M = Math<T>;
+  // root and exp(-s r) (Gaussian: exp(s r2)); r2 started from kR2Start
+  auto root = [](T x) {
+    if constexpr (kTableEntry<KT, T>)
+      return sqrt_pos(x);
+    else
+      return M::sqrt_(x);
+  };
+  auto expo = [&](T u) {
+    if constexpr (kTableEntry<KT, T>)
+      return exp2_neg64(u * (64.0 * kp.sl2), tab);
+    else
+      return exp_neg_scaled(u, kp);
+  };
   if constexpr (KT == KT_EXPONENTIAL) {
     // s = 1 / l: value e, dk/dl = r e / l^2, phi = -e / (l r)
-    const T r = M::sqrt_(r2), e = exp_neg_scaled(r, kp);
+    const T r = root(r2), e = expo(r);
     ev[KV_VALUE] = e;
     ev[KV_DL] = r * (kp.s * kp.s) * e;
     ev[KV_PHI] = T(0);
-    if (kp.vmask & (1 << KV_PHI)) ev[KV_PHI] = r > T(0) ? -M::div_(kp.s, r) * e : T(0);
+    if (kp.vmask & (1 << KV_PHI))
+      ev[KV_PHI] = r2 > kR2Start<KT, T> ? -M::div_(kp.s, r) * e : T(0);
   } else if constexpr (KT == KT_MATERN32 || KT == KT_MATERN52 || KT == KT_GAUSSIAN) {
     // the shared exponential; dk/dl = -(r^2 / l) phi for these f(r / l)
     T phi;
     if constexpr (KT == KT_GAUSSIAN) {
-      const T e = exp_neg_scaled(-r2, kp);
+      const T e = expo(-r2);
       ev[KV_VALUE] = e;
       phi = -(kp.inv_l * kp.inv_l) * e;
     } else {
-      const T r = M::sqrt_(r2), x = r * kp.s, e = exp_neg_scaled(r, kp);
+      const T r = root(r2), x = r * kp.s, e = expo(r);
       if constexpr (KT == KT_MATERN32) {
         ev[KV_VALUE] = (T(1) + x) * e;
         phi = -kp.s * kp.s * e;
@@ -283,6 +367,26 @@ __device__ __forceinline__ void kernel_r2_all(T r2, const KernelParams<T> &kp, T
       k.kt = base + KT_COUNT * v;
       ev[v] = (kp.vmask & (1 << v)) ? kernel_r2<-1, T>(r2, k) : T(0);
     }
+  }
+}
+
+// Kernel value from a squared distance that was started from kR2Start: the
+// table form above where there is one (tab: the table in LDS), else kernel_r2.
+template <int KT, typename T>
+__device__ __forceinline__ T entry_value(T r2, const KernelParams<T> &kp, const double *tab) {
+  if constexpr (kTableEntry<KT, T>) {
+    const double c = 64.0 * kp.sl2;  // 64 s log2(e)
+    if constexpr (KT == KT_GAUSSIAN) {
+      return exp2_neg64(-c * r2, tab);
+    } else {
+      const double r = sqrt_pos(r2), e = exp2_neg64(r * c, tab);
+      if constexpr (KT == KT_EXPONENTIAL) return e;
+      const double a = r * kp.s;
+      if constexpr (KT == KT_MATERN32) return fmat(a, e, e);
+      return fmat(fmat(a, a * (1. / 3.), a), e, e);
+    }
+  } else {
+    return kernel_r2<KT, T>(r2, kp);
   }
 }
 
@@ -405,9 +509,9 @@ constexpr bool kGramNear = KT == KT_MATERN32 || KT == KT_MATERN52 || KT == KT_GA
 // sigma x, so that the exponential needs no multiply of its own:
 //   MATERN32/52: FP32 sigma = s log2(e), r' = sigma r, s r = r' ln 2,
 //                k = p(r' ln 2) exp2(-r');
-//                FP64 sigma = s, k = p(r') exp(-r')
+//                FP64 sigma = 64 s log2(e), k = p(r' ln 2 / 64) 2^(-r' / 64)
 //   GAUSSIAN:    FP32 sigma^2 = log2(e) / (2 l^2), k = exp2(-r'^2);
-//                FP64 sigma^2 = 1 / (2 l^2), k = exp(-r'^2)
+//                FP64 sigma^2 = 64 log2(e) / (2 l^2), k = 2^(-r'^2 / 64)
 // (the negation is a source modifier).  Other kernels take sigma = 1 and
 // kernel_r2.
 template <int KT, typename T>
@@ -421,18 +525,21 @@ __device__ __forceinline__ T gram_sigma(const KernelParams<T> &kp) {
       return 1.f;
   } else {
     if constexpr (KT == KT_MATERN32 || KT == KT_MATERN52)
-      return kp.s;
+      return 64.0 * kp.sl2;
     else if constexpr (KT == KT_GAUSSIAN)
-      return __builtin_sqrt(-kp.s);
+      return 8.0 * __builtin_sqrt(-kp.sl2);
     else
       return 1.0;
   }
 }
 
-// Kernel value from the squared distance in the coordinates of gram_sigma.
+// Kernel value from the squared distance in the coordinates of gram_sigma, of
+// either sign (tab: the exponential's table in LDS, FP64 only).
 template <int KT, typename T>
-__device__ __forceinline__ T gram_kernel(T r2s, const KernelParams<T> &kp) {
+__device__ __forceinline__ T gram_kernel(T r2g, const KernelParams<T> &kp,
+                                         const double *tab = nullptr) {
   if constexpr (sizeof(T) == 4) {
+    const float r2s = fabsf(r2g);
     constexpr float kLn2 = 0.693147180559945309f;
     if constexpr (KT == KT_MATERN32) {
       const float r = __builtin_amdgcn_sqrtf(r2s);
@@ -446,19 +553,15 @@ __device__ __forceinline__ T gram_kernel(T r2s, const KernelParams<T> &kp) {
     } else {
       return kernel_r2<KT, float>(r2s, kp);
     }
+  } else if constexpr (KT == KT_GAUSSIAN) {
+    return exp2_neg64(__builtin_fabs(r2g), tab);
   } else {
-    using M = Math<double>;
-    if constexpr (KT == KT_MATERN32) {
-      const double a = M::sqrt_(r2s);
-      return (1.0 + a) * M::exp_(-a);
-    } else if constexpr (KT == KT_MATERN52) {
-      const double a = M::sqrt_(r2s);
-      return fmat(a, fmat(a, 1. / 3., 1.0), 1.0) * M::exp_(-a);
-    } else if constexpr (KT == KT_GAUSSIAN) {
-      return M::exp_(-r2s);
-    } else {
-      return kernel_r2<KT, double>(r2s, kp);
-    }
+    static_assert(KT == KT_MATERN32 || KT == KT_MATERN52, "FP64 Gram kernels");
+    constexpr double kLn2By64 = 1.08304246962491450973e-02;
+    const double t = sqrt_pos(__builtin_fabs(r2g) + kTinyR2), e = exp2_neg64(t, tab);
+    const double a = t * kLn2By64;
+    if constexpr (KT == KT_MATERN32) return fmat(a, e, e);
+    return fmat(fmat(a, a * (1. / 3.), a), e, e);
   }
 }
 

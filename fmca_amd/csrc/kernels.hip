@@ -250,151 +250,6 @@ __global__ __launch_bounds__(kBlock) void k_upward_transfer(DevTreeView<T> tr, I
 }
 
 // ---------------------------------------------------------------------------
-// 4. coupling: tlhs[t] = sum_{s in far(t)} K(xi_t, xi_s) mom[s]
-// (unsymmetricNystromEvaluator.h:42-58 with invV = I, H2kernelActor.h:64-66).
-// One workgroup per target cluster; thread <-> target interpolation node.
-// GEO: geodesic entries (KernelParams::geodesic), one source node at a time.
-template <typename T, int D, int KT, int NR, bool GEO = false>
-__global__ __launch_bounds__(kBlock) void k_coupling(DevTreeView<T> rows, DevTreeView<T> cols,
-                                                     DevPatternView pat, InterpParams<T> ip,
-                                                     KernelParams<T> kp, int nrhs,
-                                                     const T *__restrict__ mom,
-                                                     T *__restrict__ tlhs) {
-  extern __shared__ unsigned char smem_raw[];
-  const int P1 = ip.P1, q = ip.q;
-  // source nodes: [D][kMaxP1] per-axis values (tensor) or [D][q] (total degree)
-  const int ys = ip.td ? q : kMaxP1;
-  T *Y = reinterpret_cast<T *>(smem_raw);
-  T *Mv = Y + D * ys;  // [q][NR] source moments
-  const int task = pat.far_order[blockIdx.x];
-  if (task < 0) return;
-  const int t = pat.far_task[4 * task], f0 = pat.far_task[4 * task + 1],
-            f1 = pat.far_task[4 * task + 2];
-  const bool split = (pat.far_task[4 * task + 3] & kTaskSplit) != 0;
-  for (int rc = 0; rc < nrhs; rc += NR) {
-    const int nr = min(NR, nrhs - rc);
-    for (int abase = 0; abase < q; abase += blockDim.x) {
-      const int alpha = abase + threadIdx.x;
-      T x[D];
-      {
-        const int al = alpha < q ? alpha : 0;
-        const int pk = basis_index<T, D>(al, ip);
-#pragma unroll
-        for (int i = 0; i < D; ++i) {
-          const T u = ip.td ? ip.unodes[i * q + al] : ip.xi[(pk >> (8 * i)) & 0xff];
-          x[i] = u * rows.bbsize[t * D + i] + rows.bbmin[t * D + i];
-        }
-      }
-      T acc[NR];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) acc[r] = 0;
-      for (int f = f0; f < f1; ++f) {
-        const int s = pat.far_src[f];
-        __syncthreads();
-        if (ip.td) {
-          for (int e = threadIdx.x; e < D * q; e += blockDim.x) {
-            const int i = e / q;
-            Y[e] = ip.unodes[e] * cols.bbsize[s * D + i] + cols.bbmin[s * D + i];
-          }
-        } else {
-          for (int e = threadIdx.x; e < D * P1; e += blockDim.x) {
-            const int i = e / P1, b = e % P1;
-            Y[i * kMaxP1 + b] = ip.xi[b] * cols.bbsize[s * D + i] + cols.bbmin[s * D + i];
-          }
-        }
-        for (int e = threadIdx.x; e < q * NR; e += blockDim.x) {
-          const int beta = e / NR, r = e % NR;
-          Mv[e] = r < nr ? mom[((int64_t)s * q + beta) * nrhs + rc + r] : T(0);
-        }
-        __syncthreads();
-        if constexpr (GEO) {
-          // source node beta: axis i at Y[i * ys + b_i], b_0 fastest in the
-          // tensor case
-          int b[D];
-#pragma unroll
-          for (int i = 0; i < D; ++i) b[i] = 0;
-          for (int beta = 0; alpha < q && beta < q; ++beta) {
-            T y[D];
-#pragma unroll
-            for (int i = 0; i < D; ++i) y[i] = Y[i * ys + (ip.td ? beta : b[i])];
-            const T kv = kernel_r2<KT, T>(geodesic_r2<T, D>(x, y, 1), kp);
-#pragma unroll
-            for (int r = 0; r < NR; ++r) acc[r] += kv * Mv[beta * NR + r];
-#pragma unroll
-            for (int i = 0; i < D; ++i) {
-              if (++b[i] < P1) break;
-              b[i] = 0;
-            }
-          }
-        } else if (alpha < q && ip.td) {
-          // total degree: nodes without tensor structure
-          for (int beta = 0; beta < q; ++beta) {
-            T r2 = 0;
-#pragma unroll
-            for (int i = 0; i < D; ++i) {
-              const T di = x[i] - Y[i * q + beta];
-              r2 = fmat(di, di, r2);
-            }
-            const T kv = kernel_r2<KT, T>(r2, kp);
-#pragma unroll
-            for (int r = 0; r < NR; ++r) acc[r] += kv * Mv[beta * NR + r];
-          }
-        } else if (alpha < q) {
-          // tensor loop over the source nodes: the squared distance is
-          // accumulated dimension by dimension, one fma per entry innermost
-          int beta = 0;
-          if constexpr (D == 1) {
-            for (int b0 = 0; b0 < P1; ++b0, ++beta) {
-              const T d0 = x[0] - Y[b0];
-              const T kv = kernel_r2<KT, T>(d0 * d0, kp);
-#pragma unroll
-              for (int r = 0; r < NR; ++r) acc[r] += kv * Mv[beta * NR + r];
-            }
-          } else if constexpr (D == 2) {
-            for (int b1 = 0; b1 < P1; ++b1) {
-              const T d1 = x[1] - Y[kMaxP1 + b1];
-              const T t1 = d1 * d1;
-              for (int b0 = 0; b0 < P1; ++b0, ++beta) {
-                const T d0 = x[0] - Y[b0];
-                const T kv = kernel_r2<KT, T>(fmat(d0, d0, t1), kp);
-#pragma unroll
-                for (int r = 0; r < NR; ++r) acc[r] += kv * Mv[beta * NR + r];
-              }
-            }
-          } else {
-            for (int b2 = 0; b2 < P1; ++b2) {
-              const T d2 = x[2] - Y[2 * kMaxP1 + b2];
-              const T t2 = d2 * d2;
-              for (int b1 = 0; b1 < P1; ++b1) {
-                const T d1 = x[1] - Y[kMaxP1 + b1];
-                const T t1 = fmat(d1, d1, t2);
-                for (int b0 = 0; b0 < P1; ++b0, ++beta) {
-                  const T d0 = x[0] - Y[b0];
-                  const T kv = kernel_r2<KT, T>(fmat(d0, d0, t1), kp);
-#pragma unroll
-                  for (int r = 0; r < NR; ++r) acc[r] += kv * Mv[beta * NR + r];
-                }
-              }
-            }
-          }
-        }
-      }
-      if (alpha < q) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-          if (r < nr) {
-            T *p = tlhs + ((int64_t)t * q + alpha) * nrhs + rc + r;
-            if (split)
-              atomic_accumulate(p, acc[r]);
-            else
-              *p = acc[r];
-          }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // 5. downward transfer for the clusters [cbeg, cend) of one level >= 1:
 //    tlhs[c] += (T_c0 (x) ...)^T tlhs[parent(c)]
 template <typename T, int D, int NRC>
@@ -561,266 +416,49 @@ __global__ __launch_bounds__(kBlock) void k_cluster_basis_change(int q, const T 
 }
 
 // ---------------------------------------------------------------------------
-// 6. leaf output: y_t = V_t^T tlhs[t] + sum_{s in near(t)} K(P_t, P_s) xs_s,
-// written to out (natural order through perm, or cluster order).
-// One workgroup per target leaf, thread <-> target point.  LDS holds the
-// thread's Lagrange factors plus one union region used first for tiles of
-// far-field coefficients, then for tiles of source points.
-constexpr int kAlphaTile = 128;
-constexpr int kSrcTile = 64;
-
-template <typename T, int NR>
-__host__ __device__ constexpr size_t leaf_output_union_elems(int D) {
-  return (size_t)kAlphaTile * NR > (size_t)D * kSrcTile + (size_t)kSrcTile * NR
-             ? (size_t)kAlphaTile * NR
-             : (size_t)D * kSrcTile + (size_t)kSrcTile * NR;
+// Sums of the slabs of a phase whose lists were cut into parts (phase_parts),
+// in part order.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_add_parts(int64_t count, int parts,
+                                                      const T *__restrict__ part,
+                                                      T *__restrict__ x) {
+  const int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (e >= count) return;
+  T s = part[e];
+  for (int k = 1; k < parts; ++k) s += part[k * count + e];
+  x[e] = s;
 }
 
-template <typename T, int D, int KT, int NR, bool GEO = false>
-__global__ __launch_bounds__(kBlock) void k_leaf_output(DevTreeView<T> rows, DevTreeView<T> cols,
-                                                        DevPatternView pat, InterpParams<T> ip,
-                                                        KernelParams<T> kp, int nrhs,
-                                                        const T *__restrict__ xs,
-                                                        const T *__restrict__ tlhs,
-                                                        double *__restrict__ out, int64_t ldo,
-                                                        int natural) {
-  extern __shared__ unsigned char smem_raw[];
-  const int P1 = ip.P1, q = ip.q;
-  T *F = reinterpret_cast<T *>(smem_raw);  // [D][P1][kBlock] Lagrange factors
-  T *U = F + D * P1 * kBlock;              // union region
-  T *Mv = U;                               // [kAlphaTile][NR] far-field coefficients
-  T *Ys = U;                               // [D][kSrcTile] source points
-  T *Xs = U + D * kSrcTile;                // [kSrcTile][NR] source rhs
-  const int task = pat.near_order[blockIdx.x];
-  if (task < 0) return;
-  const int li = pat.near_task[4 * task], n0 = pat.near_task[4 * task + 1],
-            n1 = pat.near_task[4 * task + 2], flags = pat.near_task[4 * task + 3];
-  const bool split = (flags & kTaskSplit) != 0, do_far = (flags & kTaskFar) != 0;
-  const int c = rows.leaves[li];
-  const int b0 = rows.begin[c], sz = rows.size[c];
-  for (int rc = 0; rc < nrhs; rc += NR) {
-    const int nr = min(NR, nrhs - rc);
-    for (int pbase = 0; pbase < sz; pbase += kBlock) {
-      const int i = pbase + threadIdx.x;
-      const bool act = i < sz;
-      T x[D];
-#pragma unroll
-      for (int d = 0; d < D; ++d)
-        x[d] = act ? rows.pts[(int64_t)d * rows.npts + b0 + i] : T(0);
-      T acc[NR];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) acc[r] = 0;
-      // far field through the leaf basis (backward_transform_impl.h:30-31),
-      // applied by the first task of the leaf
-      __syncthreads();
-      if (act && do_far) {
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-          basis_1d<T>(rows.unit[(int64_t)d * rows.npts + b0 + i], ip,
-                      F + (d * P1) * kBlock + threadIdx.x, kBlock);
-      }
-      int a[D];
-#pragma unroll
-      for (int d = 0; d < D; ++d) a[d] = 0;
-      for (int at = 0; do_far && at < q; at += kAlphaTile) {
-        const int na = min(kAlphaTile, q - at);
-        __syncthreads();
-        for (int e = threadIdx.x; e < kAlphaTile * NR; e += blockDim.x) {
-          const int al = e / NR, r = e % NR;
-          Mv[e] = (al < na && r < nr) ? tlhs[((int64_t)c * q + at + al) * nrhs + rc + r] : T(0);
-        }
-        __syncthreads();
-        if (act) {
-          for (int al = 0; al < na; ++al) {
-            if (ip.td) {
-              const int pk = ip.midx[at + al];
-#pragma unroll
-              for (int d = 0; d < D; ++d) a[d] = (pk >> (8 * d)) & 0xff;
-            }
-            T v = F[(0 * P1 + a[0]) * kBlock + threadIdx.x];
-#pragma unroll
-            for (int d = 1; d < D; ++d) v *= F[(d * P1 + a[d]) * kBlock + threadIdx.x];
-#pragma unroll
-            for (int r = 0; r < NR; ++r) acc[r] += v * Mv[al * NR + r];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-              if (++a[d] < P1) break;
-              a[d] = 0;
-            }
-          }
-        }
-      }
-      // near field (unsymmetricNystromEvaluator.h:63-73, H2kernelActor.h:68-69);
-      // a run of sources with adjacent point ranges is one source here
-      for (int nb = n0; nb < n1;) {
-        const int run = pat.near_run[nb];
-        const int s = pat.near_src[nb], sl = pat.near_src[nb + run - 1];
-        const int sb = cols.begin[s], ss = cols.begin[sl] + cols.size[sl] - sb;
-        nb += run;
-        for (int j0 = 0; j0 < ss; j0 += kSrcTile) {
-          const int nj = min(kSrcTile, ss - j0);
-          __syncthreads();
-          for (int e = threadIdx.x; e < D * kSrcTile; e += blockDim.x) {
-            const int d = e / kSrcTile, jj = e % kSrcTile;
-            Ys[e] = jj < nj ? cols.pts[(int64_t)d * cols.npts + sb + j0 + jj] : T(0);
-          }
-          for (int e = threadIdx.x; e < kSrcTile * NR; e += blockDim.x) {
-            const int jj = e / NR, r = e % NR;
-            Xs[e] = (jj < nj && r < nr) ? xs[(int64_t)(sb + j0 + jj) * nrhs + rc + r] : T(0);
-          }
-          __syncthreads();
-          if (act) {
-            for (int jj = 0; jj < nj; ++jj) {
-              T r2 = 0;
-              if constexpr (GEO) {
-                r2 = geodesic_r2<T, D>(x, Ys + jj, kSrcTile);
-              } else {
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                  const T dd = x[d] - Ys[d * kSrcTile + jj];
-                  r2 += dd * dd;
-                }
-              }
-              const T kv = kernel_r2<KT, T>(r2, kp);
-#pragma unroll
-              for (int r = 0; r < NR; ++r) acc[r] += kv * Xs[jj * NR + r];
-            }
-          }
-        }
-      }
-      if (act) {
-        const int64_t row = natural ? (int64_t)rows.perm[b0 + i] : (int64_t)(b0 + i);
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-          if (r < nr) {
-            double *p = out + row + (int64_t)(rc + r) * ldo;
-            if (split)
-              atomic_accumulate(p, (double)acc[r]);
-            else
-              *p = (double)acc[r];
-          }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-template <typename T, int NR>
-size_t output_lds(int D, int P1) {
-  return ((size_t)D * P1 * kBlock + leaf_output_union_elems<T, NR>(D)) * sizeof(T);
-}
-
-template <typename T, int NR>
-size_t coupling_lds(int D, int q, bool td) {
-  return ((size_t)D * (td ? q : kMaxP1) + (size_t)q * NR) * sizeof(T);
-}
-
-template <typename T, int D, int KT, int NR, bool GEO = false>
-hipError_t launch_far_near(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                           const DevPatternView &pat, const InterpParams<T> &ip,
-                           const KernelParams<T> &kp, int nrhs, ActionBuffers<T> buf,
-                           double *out, int64_t ldo, bool natural, hipStream_t stream) {
-  const int q = ip.q;
-  const int threads = q <= 64 ? 64 : (q <= 128 ? 128 : kBlock);
-  const size_t lds = coupling_lds<T, NR>(D, q, ip.td != 0);
-  hipLaunchKernelGGL((k_coupling<T, D, KT, NR, GEO>), dim3(pat.nfar_order), dim3(threads), lds, stream, rows,
-                     cols, pat, ip, kp, nrhs, buf.mom, buf.tlhs);
-  return hipGetLastError();
-}
-
-template <typename T, int D, int KT, int NR, bool GEO = false>
-hipError_t launch_output(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                         const DevPatternView &pat, const InterpParams<T> &ip,
-                         const KernelParams<T> &kp, int nrhs, ActionBuffers<T> buf, double *out,
-                         int64_t ldo, bool natural, hipStream_t stream) {
-  const size_t lds = output_lds<T, NR>(D, ip.P1);
-  hipLaunchKernelGGL((k_leaf_output<T, D, KT, NR, GEO>), dim3(pat.nnear_order), dim3(kBlock), lds,
-                     stream, rows, cols, pat, ip, kp, nrhs, buf.xs, buf.tlhs, out, ldo,
-                     natural ? 1 : 0);
-  return hipGetLastError();
-}
-
-template <typename T, int D, int NR>
-hipError_t dispatch_kt(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                       const DevPatternView &pat, const InterpParams<T> &ip,
-                       const KernelParams<T> &kp, int nrhs, ActionBuffers<T> buf, double *out,
-                       int64_t ldo, bool natural, hipStream_t stream) {
-#define FMCA_KT_CASE(K)                                                                 \
-  case K:                                                                               \
-    return output ? launch_output<T, D, K, NR>(rows, cols, pat, ip, kp, nrhs, buf, out, \
-                                               ldo, natural, stream)                    \
-                  : launch_far_near<T, D, K, NR>(rows, cols, pat, ip, kp, nrhs, buf, out, \
-                                                 ldo, natural, stream);
-  if (kp.geodesic) {
-    // geodesic entries: FP64 only, the kernel type switched at run time
-    if constexpr (sizeof(T) == 8)
-      return output ? launch_output<T, D, -1, NR, true>(rows, cols, pat, ip, kp, nrhs, buf, out,
-                                                        ldo, natural, stream)
-                    : launch_far_near<T, D, -1, NR, true>(rows, cols, pat, ip, kp, nrhs, buf,
-                                                          out, ldo, natural, stream);
-    return hipErrorInvalidValue;
-  }
-  switch (kp.kt) {
-    FMCA_KT_CASE(KT_EXPONENTIAL)
-    FMCA_KT_CASE(KT_MATERN32)
-    FMCA_KT_CASE(KT_MATERN52)
-    FMCA_KT_CASE(KT_GAUSSIAN)
-    default:
-      return output ? launch_output<T, D, -1, NR>(rows, cols, pat, ip, kp, nrhs, buf, out, ldo,
-                                                  natural, stream)
-                    : launch_far_near<T, D, -1, NR>(rows, cols, pat, ip, kp, nrhs, buf, out,
-                                                    ldo, natural, stream);
-  }
-#undef FMCA_KT_CASE
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_add_parts_out(int64_t n, int nrhs, int parts,
+                                                          const uint32_t *__restrict__ perm,
+                                                          const T *__restrict__ part,
+                                                          double *__restrict__ out, int64_t ldo) {
+  const int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (e >= n * nrhs) return;
+  double s = (double)part[e];
+  for (int k = 1; k < parts; ++k) s += (double)part[k * n * nrhs + e];
+  const int64_t i = e / nrhs, r = e - i * nrhs;
+  out[(perm ? (int64_t)perm[i] : i) + r * ldo] = s;
 }
 
 constexpr size_t kLdsLimit = 64 * 1024;
-
-// Largest rhs tile (32, 8 or 1) whose LDS footprint fits one workgroup.
-template <typename T>
-int pick_nr(bool output, int D, int P1, int q, int nrhs, bool td) {
-  auto fits = [&](int nr) {
-    const size_t b = output ? (nr == 32   ? output_lds<T, 32>(D, P1)
-                               : nr == 8 ? output_lds<T, 8>(D, P1)
-                                         : output_lds<T, 1>(D, P1))
-                            : (nr == 32   ? coupling_lds<T, 32>(D, q, td)
-                               : nr == 8 ? coupling_lds<T, 8>(D, q, td)
-                                         : coupling_lds<T, 1>(D, q, td));
-    return b <= kLdsLimit;
-  };
-  if (nrhs > 8 && fits(32)) return 32;
-  if (nrhs > 1 && fits(8)) return 8;
-  return 1;
-}
 
 template <typename T, int D>
 hipError_t dispatch_nr(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                        const DevPatternView &pat, const InterpParams<T> &ip,
                        const KernelParams<T> &kp, int nrhs, ActionBuffers<T> buf, double *out,
                        int64_t ldo, bool natural, hipStream_t stream) {
+  const PhaseLaunch<T> a{rows, cols, pat,  ip,      kp,       nrhs,         buf.xs, buf.mom, buf.tlhs,
+                         out,  ldo,  natural, buf.part, buf.part_cap, stream};
   if constexpr (sizeof(T) == 4) {
     if (kp.geodesic) return hipErrorInvalidValue;
     if (kp.split_bf16 && bf16_supported(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask))
-      return launch_bf16(output, rows, cols, pat, ip, kp, nrhs, buf.xs, buf.mom, buf.tlhs, out,
-                         ldo, natural, stream);
+      return launch_bf16(output, a, buf.xs, buf.mom);
   }
   if (!kp.geodesic && mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td))
-    return launch_mfma<T>(output, rows, cols, pat, ip, kp, nrhs, buf.xs, buf.mom, buf.tlhs, out,
-                          ldo, natural, stream);
-  // the VALU forms evaluate one variant per launch (kp.kt)
-  if ((kp.vmask & (kp.vmask - 1)) != 0) return hipErrorInvalidValue;
-  const bool td = ip.td != 0;
-  const int nr = pick_nr<T>(output, D, ip.P1, ip.q, nrhs, td);
-  if (output ? output_lds<T, 1>(D, ip.P1) > kLdsLimit : coupling_lds<T, 1>(D, ip.q, td) > kLdsLimit)
-    return hipErrorInvalidConfiguration;
-  if (nr == 1)
-    return dispatch_kt<T, D, 1>(output, rows, cols, pat, ip, kp, nrhs, buf, out, ldo, natural,
-                                stream);
-  if (nr == 8)
-    return dispatch_kt<T, D, 8>(output, rows, cols, pat, ip, kp, nrhs, buf, out, ldo, natural,
-                                stream);
-  return dispatch_kt<T, D, 32>(output, rows, cols, pat, ip, kp, nrhs, buf, out, ldo, natural,
-                               stream);
+    return launch_mfma<T>(output, a);
+  return launch_valu<T>(output, a);
 }
 
 template <typename T, int D>
@@ -842,9 +480,12 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
     hipLaunchKernelGGL((k_permute_in<T>), dim3((unsigned)grid), dim3(kBlock), 0, stream, rhs,
                        ld_rhs, nrhs, cols.npts, natural ? cols.pinv : nullptr, buf.xs);
   }
+  // without far blocks (and without stored leaf bases or a gradient job that
+  // read the moments) the tree passes and the coupling have nothing to do
+  const bool tree = pat.has_far || stored || grad;
   // 2. leaf moments
   mark(PH_UPWARD_LEAF);
-  {
+  if (tree) {
     // FP64: column groups, as many as leave kBlock / G >= q threads per group
     // (n = 1e6, q = 125, 32 rhs: 0.79 -> 0.64 ms); FP32 is faster with one
     // group (0.36 against 0.40 ms: the shared basis values then cover twice
@@ -895,7 +536,7 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
   };
   const int top_src = first_level(lcols, pat.far_top_source);
   const int top_tgt = first_level(lrows, pat.far_top_target);
-  if (top_src > 0) {
+  if (tree && top_src > 0) {
     const int64_t count = (int64_t)lcols.level_ptr[std::min(top_src, lcols.depth + 1)] * q * nrhs;
     hipLaunchKernelGGL((k_zero_range<T>), dim3((unsigned)std::min<int64_t>(
                            1024, std::max<int64_t>(1, (count + kBlock - 1) / kBlock))),
@@ -924,7 +565,7 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
     return dense_lds(arrays, nrc) +
            (mats_fit(arrays, nrc) ? (size_t)arrays * q * q * sizeof(T) : 0);
   };
-  if (ip.td) {
+  if (tree && ip.td) {
     const int nu = dense_nrc(2);
     if (dense_lds(2, nu) > kLdsLimit) return hipErrorInvalidConfiguration;
     const int se = mats_fit(2, nu) ? 1 : 0;
@@ -951,7 +592,7 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
   const int nrc_up = transfer_nrc(3), nrc_dn = transfer_nrc(2);
   if (!ip.td && (transfer_lds(3, nrc_up) > kLdsLimit || transfer_lds(2, nrc_dn) > kLdsLimit))
     return hipErrorInvalidConfiguration;
-  for (int L = lcols.depth - 1; !ip.td && L >= top_src; --L) {
+  for (int L = lcols.depth - 1; tree && !ip.td && L >= top_src; --L) {
     const int cb = lcols.level_ptr[L], nc = lcols.level_ptr[L + 1] - cb;
     const size_t lds = transfer_lds(3, nrc_up);
     if (nrc_up == 8)
@@ -964,13 +605,13 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
   if ((err = hipGetLastError()) != hipSuccess) return err;
   // 4. coupling (every target cluster is written, empty far lists give zeros)
   mark(PH_COUPLING);
-  if (ip.td) basis_change(cols.ncl, 1, buf.mom);
+  if (tree && ip.td) basis_change(cols.ncl, 1, buf.mom);
   if (stored) {
     // stored coupling matrices; one workgroup per target writes all of it
     if ((err = launch_stored<T>(false, rows, cols, pat, *stored, q, nrhs, buf.xs, buf.mom,
                                 buf.tlhs, out, ld_out, natural, stream)) != hipSuccess)
       return err;
-  } else {
+  } else if (tree) {
     if (pat.nfar_split > 0)
       hipLaunchKernelGGL((k_zero_clusters<T>), dim3(pat.nfar_split), dim3(kBlock), 0, stream,
                          pat.far_split, (int64_t)q * nrhs, buf.tlhs);
@@ -984,12 +625,12 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                                       stream)) != hipSuccess)
       return err;
   }
-  if (ip.td) basis_change(rows.ncl, 0, buf.tlhs);
+  if (tree && ip.td) basis_change(rows.ncl, 0, buf.tlhs);
   // 5. downward transfers, top level first, from the level below the first
   // far target on (every cluster above it holds zeros after the coupling)
   mark(PH_DOWNWARD_TRANSFER);
   const int first_dn = std::max(1, top_tgt + 1);
-  if (ip.td) {
+  if (tree && ip.td) {
     const int nd = dense_nrc(1);
     const int se = mats_fit(1, nd) ? 1 : 0;
     for (int L = first_dn; L <= lrows.depth; ++L) {
@@ -1002,7 +643,7 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                            with_mats(1, 1), stream, rows, q, cb, nrhs, se, buf.tlhs);
     }
   }
-  for (int L = first_dn; !ip.td && L <= lrows.depth; ++L) {
+  for (int L = first_dn; tree && !ip.td && L <= lrows.depth; ++L) {
     const int cb = lrows.level_ptr[L], nc = lrows.level_ptr[L + 1] - cb;
     const size_t lds = transfer_lds(2, nrc_dn);
     if (nrc_dn == 8)
@@ -1065,6 +706,27 @@ hipError_t launch_math_probe(int fn, const double *x, double *y, int64_t n, hipS
     return hipErrorInvalidValue;
   return hipGetLastError();
 }
+
+template <typename T>
+hipError_t launch_add_parts(bool output, const DevTreeView<T> &rows, int q, int nrhs, int parts,
+                            const T *part, T *tlhs, double *out, int64_t ldo, bool natural,
+                            hipStream_t stream) {
+  const int64_t count = (output ? rows.npts : (int64_t)rows.ncl * q) * nrhs;
+  const unsigned grid = (unsigned)((count + kBlock - 1) / kBlock);
+  if (output)
+    hipLaunchKernelGGL((k_add_parts_out<T>), dim3(grid), dim3(kBlock), 0, stream, rows.npts, nrhs,
+                       parts, natural ? rows.perm : nullptr, part, out, ldo);
+  else
+    hipLaunchKernelGGL((k_add_parts<T>), dim3(grid), dim3(kBlock), 0, stream, count, parts, part,
+                       tlhs);
+  return hipGetLastError();
+}
+template hipError_t launch_add_parts<float>(bool, const DevTreeView<float> &, int, int, int,
+                                            const float *, float *, double *, int64_t, bool,
+                                            hipStream_t);
+template hipError_t launch_add_parts<double>(bool, const DevTreeView<double> &, int, int, int,
+                                             const double *, double *, double *, int64_t, bool,
+                                             hipStream_t);
 
 template <typename T>
 hipError_t launch_action(const DevTreeView<T> &rows, const DevTreeView<T> &cols,

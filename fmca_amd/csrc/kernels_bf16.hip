@@ -58,6 +58,15 @@ __device__ __forceinline__ f32x4 mma_f32(float a, float b, f32x4 c) {
 
 __device__ __forceinline__ f32x4 splat4(float v) { return f32x4{v, v, v, v}; }
 
+// The part of a task's list that this workgroup takes (grid.y parts).
+__device__ __forceinline__ void list_part(int &lo, int &hi) {
+  if (gridDim.y == 1) return;
+  const int64_t cnt = hi - lo;
+  const int lo0 = lo;
+  lo = lo0 + (int)(cnt * blockIdx.y / gridDim.y);
+  hi = lo0 + (int)(cnt * (blockIdx.y + 1) / gridDim.y);
+}
+
 __device__ __forceinline__ int unpack(int p, int d) { return (p >> (8 * d)) & 0xff; }
 
 // hi = bf16(v) rounded to nearest even, lo = bf16(v - hi)
@@ -119,7 +128,8 @@ template <int D, int KT, int NT>
 __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
     DevTreeView<float> rows, DevTreeView<float> cols, DevPatternView pat,
     InterpParams<float> ip, KernelParams<float> kp, int nrhs, const float *__restrict__ xs,
-    const float *__restrict__ tlhs, double *__restrict__ out, int64_t ldo, int natural) {
+    const float *__restrict__ tlhs, double *__restrict__ out, int64_t ldo, int natural,
+    float *__restrict__ part) {
   constexpr int NC = 16 * NT;
   constexpr int NCP = NC + 16;  // padded stride of the staged far moments
   constexpr bool kGram = kGramNear<KT>;
@@ -140,9 +150,11 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
   const int lr = lane & 15, lk = lane >> 4;
   const int task = pat.near_order[blockIdx.x];
   if (task < 0) return;
-  const int li = pat.near_task[4 * task], n0 = pat.near_task[4 * task + 1],
-            n1 = pat.near_task[4 * task + 2], flags = pat.near_task[4 * task + 3];
-  const bool split = (flags & kTaskSplit) != 0, do_far = (flags & kTaskFar) != 0;
+  const int li = pat.near_task[4 * task], flags = pat.near_task[4 * task + 3];
+  int n0 = pat.near_task[4 * task + 1], n1 = pat.near_task[4 * task + 2];
+  const bool split = (flags & kTaskSplit) != 0;
+  const bool do_far = (flags & kTaskFar) != 0 && pat.has_far && blockIdx.y == 0;
+  list_part(n0, n1);
   const int c = rows.leaves[li];
   const int b0 = rows.begin[c], sz = rows.size[c];
   for (int e = threadIdx.x; e < qpad; e += blockDim.x)
@@ -240,7 +252,7 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
       float py[KY], px[KX];
       int nb = n0, j0 = 0, pnj = 0;
       auto fetch = [&]() {
-        const int run = pat.near_run[nb];
+        const int run = min(pat.near_run[nb], n1 - nb);
         const int s = pat.near_src[nb], sl = pat.near_src[nb + run - 1];
         const int sb = cols.begin[s], ss = cols.begin[sl] + cols.size[sl] - sb;
         pnj = min(kChunk, ss - j0);
@@ -349,8 +361,8 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
               float ev[8];
 #pragma unroll
               for (int v = 0; v < 4; ++v) {
-                ev[v] = gram_kernel<KT>(fabsf(c0[v]), kp);
-                ev[4 + v] = gram_kernel<KT>(fabsf(c1[v]), kp);
+                ev[v] = gram_kernel<KT>(c0[v], kp);
+                ev[4 + v] = gram_kernel<KT>(c1[v], kp);
               }
               bf16x8 ah, al;
               split8(ev, ah, al);
@@ -470,6 +482,10 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
           for (int v = 0; v < 4; ++v) {
             const int i = pbase + (wave + kWaves * rt) * 16 + 4 * lk + v;
             if (i < sz && col < nrhs) {
+              if (gridDim.y > 1) {
+                part[((int64_t)blockIdx.y * rows.npts + b0 + i) * nrhs + col] = acc[rt][nt][v];
+                continue;
+              }
               const int64_t row = natural ? (int64_t)rows.perm[b0 + i] : (int64_t)(b0 + i);
               double *p = out + row + (int64_t)col * ldo;
               if (split)
@@ -496,7 +512,7 @@ template <int D, int KT, int NT>
 __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
     DevTreeView<float> rows, DevTreeView<float> cols, DevPatternView pat,
     InterpParams<float> ip, KernelParams<float> kp, int nrhs, const float *__restrict__ mom,
-    float *__restrict__ tlhs) {
+    float *__restrict__ tlhs, float *__restrict__ part) {
   constexpr int NC = 16 * NT;
   extern __shared__ unsigned char smem_raw[];
   const int q = ip.q;
@@ -515,8 +531,11 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
   const int lr = lane & 15, lk = lane >> 4;
   const int task = pat.far_order[blockIdx.x];
   if (task < 0) return;
-  const int t = pat.far_task[4 * task], f0 = pat.far_task[4 * task + 1],
-            f1 = pat.far_task[4 * task + 2];
+  const int t = pat.far_task[4 * task];
+  int f0 = pat.far_task[4 * task + 1], f1 = pat.far_task[4 * task + 2];
+  list_part(f0, f1);
+  // sums of this part: its slab, or the coupling sums themselves
+  float *dst_all = gridDim.y > 1 ? part + (int64_t)blockIdx.y * rows.ncl * ip.q * nrhs : tlhs;
   const bool split = (pat.far_task[4 * task + 3] & kTaskSplit) != 0;
   const int R = (q + 15) / 16;
   const int kspl = R <= kRT ? 4 : (R <= 2 * kRT ? 2 : 1);
@@ -602,8 +621,8 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
           float ev[8];
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            ev[v] = gram_kernel<KT>(fabsf(c0[v]), kp);
-            ev[4 + v] = gram_kernel<KT>(fabsf(c1[v]), kp);
+            ev[v] = gram_kernel<KT>(c0[v], kp);
+            ev[4 + v] = gram_kernel<KT>(c1[v], kp);
           }
           bf16x8 ah, al;
           split8(ev, ah, al);
@@ -735,7 +754,7 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
       for (int e = threadIdx.x; e < q * NC; e += blockDim.x) {
         const int alpha = e / NC, cc = e - alpha * NC;
         if (cc < 16 * ntl && rc + cc < nrhs) {
-          float *p = tlhs + ((int64_t)t * q + alpha) * nrhs + rc + cc;
+          float *p = dst_all + ((int64_t)t * q + alpha) * nrhs + rc + cc;
           if (split)
             atomic_accumulate(p, Red[e]);
           else
@@ -754,7 +773,7 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
           for (int v = 0; v < 4; ++v) {
             const int alpha = (rg + wrows * rt) * 16 + 4 * lk + v;
             if (alpha < q && col < nrhs) {
-              float *p = tlhs + ((int64_t)t * q + alpha) * nrhs + col;
+              float *p = dst_all + ((int64_t)t * q + alpha) * nrhs + col;
               if (split)
                 atomic_accumulate(p, acc[rt][nt][v]);
               else
@@ -787,52 +806,46 @@ size_t coupling_bf16_lds(int D, int q) {
 }
 
 template <int D, int NT>
-hipError_t launch_bf16_nt(bool output, const DevTreeView<float> &rows,
-                          const DevTreeView<float> &cols, const DevPatternView &pat,
-                          const InterpParams<float> &ip, const KernelParams<float> &kp, int nrhs,
-                          const float *xs, const float *mom, float *tlhs, double *out,
-                          int64_t ldo, bool natural, hipStream_t stream) {
-  const size_t lds_out = leaf_output_bf16_lds<NT>(D, ip.P1, ip.q);
-  const size_t lds_cpl = coupling_bf16_lds<NT>(D, ip.q);
-#define FMCA_BF16_CASE(K)                                                                   \
-  case K:                                                                                   \
-    if (output)                                                                             \
-      hipLaunchKernelGGL((k_leaf_output_bf16<D, K, NT>), dim3(pat.nnear_order), dim3(256),  \
-                         lds_out, stream, rows, cols, pat, ip, kp, nrhs, xs, tlhs, out, ldo, \
-                         natural ? 1 : 0);                                                  \
-    else                                                                                    \
-      hipLaunchKernelGGL((k_coupling_bf16<D, K, NT>), dim3(pat.nfar_order), dim3(256),      \
-                         lds_cpl, stream, rows, cols, pat, ip, kp, nrhs, mom, tlhs);        \
-    break;
-  switch (kp.kt) {
-    FMCA_BF16_CASE(KT_EXPONENTIAL)
-    FMCA_BF16_CASE(KT_MATERN32)
-    FMCA_BF16_CASE(KT_MATERN52)
-    FMCA_BF16_CASE(KT_GAUSSIAN)
+hipError_t launch_bf16_nt(bool output, const MfmaLaunch<float> &a) {
+  const size_t lds_out = leaf_output_bf16_lds<NT>(D, a.ip.P1, a.ip.q);
+  const size_t lds_cpl = coupling_bf16_lds<NT>(D, a.ip.q);
+  float *slabs = nullptr;
+  const int parts = launch_parts(output, a, &slabs);
+  const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
+#define FMCA_BF16_LAUNCH(K)                                                                   \
+  if (output)                                                                                 \
+    hipLaunchKernelGGL((k_leaf_output_bf16<D, K, NT>), grid, dim3(256), lds_out, a.stream,    \
+                       a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs, a.tlhs, a.out, a.ldo, \
+                       a.natural ? 1 : 0, slabs);                                             \
+  else                                                                                        \
+    hipLaunchKernelGGL((k_coupling_bf16<D, K, NT>), grid, dim3(256), lds_cpl, a.stream,       \
+                       a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs, slabs)
+  switch (a.kp.kt) {
+    case KT_EXPONENTIAL:
+      FMCA_BF16_LAUNCH(KT_EXPONENTIAL);
+      break;
+    case KT_MATERN32:
+      FMCA_BF16_LAUNCH(KT_MATERN32);
+      break;
+    case KT_MATERN52:
+      FMCA_BF16_LAUNCH(KT_MATERN52);
+      break;
+    case KT_GAUSSIAN:
+      FMCA_BF16_LAUNCH(KT_GAUSSIAN);
+      break;
     default:
-      if (output)
-        hipLaunchKernelGGL((k_leaf_output_bf16<D, -1, NT>), dim3(pat.nnear_order), dim3(256),
-                           lds_out, stream, rows, cols, pat, ip, kp, nrhs, xs, tlhs, out, ldo,
-                           natural ? 1 : 0);
-      else
-        hipLaunchKernelGGL((k_coupling_bf16<D, -1, NT>), dim3(pat.nfar_order), dim3(256),
-                           lds_cpl, stream, rows, cols, pat, ip, kp, nrhs, mom, tlhs);
+      FMCA_BF16_LAUNCH(-1);
   }
-#undef FMCA_BF16_CASE
-  return hipGetLastError();
+#undef FMCA_BF16_LAUNCH
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || parts == 1) return e;
+  return launch_add_parts<float>(output, a.rows, a.ip.q, a.nrhs, parts, slabs, a.tlhs, a.out,
+                                 a.ldo, a.natural, a.stream);
 }
 
 template <int D>
-hipError_t launch_bf16_d(bool output, const DevTreeView<float> &rows,
-                         const DevTreeView<float> &cols, const DevPatternView &pat,
-                         const InterpParams<float> &ip, const KernelParams<float> &kp, int nrhs,
-                         const float *xs, const float *mom, float *tlhs, double *out, int64_t ldo,
-                         bool natural, hipStream_t stream) {
-  if (nrhs <= 16)
-    return launch_bf16_nt<D, 1>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                                natural, stream);
-  return launch_bf16_nt<D, 2>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                              natural, stream);
+hipError_t launch_bf16_d(bool output, const MfmaLaunch<float> &a) {
+  return a.nrhs <= 16 ? launch_bf16_nt<D, 1>(output, a) : launch_bf16_nt<D, 2>(output, a);
 }
 
 }  // namespace
@@ -849,31 +862,24 @@ bool bf16_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vma
   return (nt == 1 ? coupling_bf16_lds<1>(D, q) : coupling_bf16_lds<2>(D, q)) <= limit;
 }
 
-hipError_t launch_bf16(bool output, const DevTreeView<float> &rows,
-                       const DevTreeView<float> &cols, const DevPatternView &pat,
-                       const InterpParams<float> &ip, const KernelParams<float> &kp, int nrhs,
-                       float *xs, float *mom, float *tlhs, double *out, int64_t ldo,
-                       bool natural, hipStream_t stream) {
+hipError_t launch_bf16(bool output, const MfmaLaunch<float> &a, float *xs, float *mom) {
   {
     // the right operand this launch stages, split once here (rewritten by
     // the next action's permutation / upward pass)
     float *x = output ? xs : mom;
-    const int64_t n = (output ? cols.npts : (int64_t)cols.ncl * ip.q) * nrhs;
+    const int64_t n = (output ? a.cols.npts : (int64_t)a.cols.ncl * a.ip.q) * a.nrhs;
     if (n > 0) {
       const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, 8192);
-      hipLaunchKernelGGL(k_split_inplace, dim3(grid), dim3(256), 0, stream, x, n);
+      hipLaunchKernelGGL(k_split_inplace, dim3(grid), dim3(256), 0, a.stream, x, n);
     }
   }
-  switch (rows.dim) {
+  switch (a.rows.dim) {
     case 1:
-      return launch_bf16_d<1>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                              natural, stream);
+      return launch_bf16_d<1>(output, a);
     case 2:
-      return launch_bf16_d<2>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                              natural, stream);
+      return launch_bf16_d<2>(output, a);
     case 3:
-      return launch_bf16_d<3>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                              natural, stream);
+      return launch_bf16_d<3>(output, a);
   }
   return hipErrorInvalidValue;
 }

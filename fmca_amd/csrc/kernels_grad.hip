@@ -96,6 +96,8 @@ __global__ __launch_bounds__(256) void k_grad_near(
   __shared__ T Ys[D][kGChunk];
   __shared__ T Xs[kGChunk * XSP];
   __shared__ T red[kWaves];
+  __shared__ double tab[kTableEntry<KT, T> ? 64 : 1];
+  if constexpr (kTableEntry<KT, T>) load_exp2_table(tab);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lk = lane >> 4;
@@ -164,14 +166,14 @@ __global__ __launch_bounds__(256) void k_grad_near(
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
               const int j = jb + M::crow(lk, v);
-              T r2 = 0, dd[D];
+              T r2 = kR2Start<KT, T>, dd[D];
 #pragma unroll
               for (int d = 0; d < D; ++d) {
                 dd[d] = x[rt][d] - Ys[d][j];
                 r2 = fmat(dd[d], dd[d], r2);
               }
               T ev[3];
-              kernel_r2_all<KT, T>(r2, kp, ev);
+              kernel_r2_all<KT, T>(r2, kp, tab, ev);
               const T wv = w[v];
               dls = fmat(ev[KV_DL], wv, dls);
               const T u = ev[KV_PHI] * wv;

@@ -76,20 +76,29 @@ template <typename T, int NT, int KT, bool MULTI>
 constexpr int kMinWavesGram =
     (sizeof(T) == 8 && !MULTI && kGramNear<KT>) ? 2 : kMinWaves<T, NT, KT, MULTI>;
 
+// The part of a task's list that this workgroup takes (grid.y parts).
+__device__ __forceinline__ void list_part(int &lo, int &hi) {
+  if (gridDim.y == 1) return;
+  const int64_t cnt = hi - lo;
+  const int lo0 = lo;
+  lo = lo0 + (int)(cnt * blockIdx.y / gridDim.y);
+  hi = lo0 + (int)(cnt * (blockIdx.y + 1) / gridDim.y);
+}
+
 // Packed tensor index of every moment: a0 | a1 << 8 | a2 << 16.
 __device__ __forceinline__ int unpack(int p, int d) { return (p >> (8 * d)) & 0xff; }
 
 // ---------------------------------------------------------------------------
 // Leaf output on MFMA: one workgroup per target leaf, 4 waves, each wave owns
-// row tiles {wave, wave+4, wave+8, wave+12} of the current 256-row pass and
-// 16*NT rhs columns.
+// row tiles {wave, wave+4, wave+8, wave+12} of the current 256-row pass (with
+// fewer than 9 tiles the waves split the K-steps too) and 16*NT rhs columns.
 // MULTI: the rhs columns carry different kernel variants (kp.tv per 16-column
 // tile); every entry is evaluated once for all three variants.
 template <typename T, int D, int KT, int NT, bool MULTI>
 __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf_output_mfma(
     DevTreeView<T> rows, DevTreeView<T> cols, DevPatternView pat, InterpParams<T> ip,
     KernelParams<T> kp, int nrhs, const T *__restrict__ xs, const T *__restrict__ tlhs,
-    double *__restrict__ out, int64_t ldo, int natural) {
+    double *__restrict__ out, int64_t ldo, int natural, T *__restrict__ part) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int NC = 16 * NT;
@@ -99,6 +108,8 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
   // the matrix cores (kGramNear), 16 sources per distance MFMA
   constexpr bool kGram = sizeof(T) == 8 && !MULTI && kGramNear<KT> && D <= 3;
   extern __shared__ unsigned char smem_raw[];
+  __shared__ double tab[kTableEntry<KT, T> ? 64 : 1];
+  if constexpr (kTableEntry<KT, T>) load_exp2_table(tab);
   const int P1 = ip.P1, q = ip.q;
   const int qpad = (q + 3) & ~3;
   T *F = reinterpret_cast<T *>(smem_raw);              // [D][P1][kRowsP] factors of the rows
@@ -113,9 +124,11 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
   const int lr = lane & 15, lk = lane >> 4;
   const int task = pat.near_order[blockIdx.x];
   if (task < 0) return;
-  const int li = pat.near_task[4 * task], n0 = pat.near_task[4 * task + 1],
-            n1 = pat.near_task[4 * task + 2], flags = pat.near_task[4 * task + 3];
-  const bool split = (flags & kTaskSplit) != 0, do_far = (flags & kTaskFar) != 0;
+  const int li = pat.near_task[4 * task], flags = pat.near_task[4 * task + 3];
+  int n0 = pat.near_task[4 * task + 1], n1 = pat.near_task[4 * task + 2];
+  const bool split = (flags & kTaskSplit) != 0;
+  const bool do_far = (flags & kTaskFar) != 0 && pat.has_far && blockIdx.y == 0;
+  list_part(n0, n1);
   const int c = rows.leaves[li];
   const int b0 = rows.begin[c], sz = rows.size[c];
   for (int e = threadIdx.x; e < qpad; e += blockDim.x)
@@ -143,12 +156,18 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           for (int a = 0; a < P1; ++a) F[(d * P1 + a) * kRowsP + threadIdx.x] = T(0);
       }
     }
-    // this lane's A rows: tile (wave + 4 rt), row lr
+    // K-split: with at most 8 row tiles, kspl groups of waves share the
+    // K-steps, so that every wave holds up to kRT row tiles (their B operands
+    // are read once); the groups' sums are added in LDS in group order
+    const int R = (min(kRows, sz - pbase) + 15) / 16;
+    const int kspl = R <= kRT ? 4 : (R <= 2 * kRT ? 2 : 1);
+    const int wrows = kWaves / kspl, rg = wave % wrows, sg = wave / wrows;
+    // this lane's A rows: tile (rg + wrows rt), row lr
     T x[kRT][D];
     bool tile_on[kRT];
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) {
-      const int tile_row0 = pbase + (wave + kWaves * rt) * 16;
+      const int tile_row0 = pbase + (rg + wrows * rt) * 16;
       tile_on[rt] = tile_row0 < sz;
       const int i = tile_row0 + lr;
 #pragma unroll
@@ -197,7 +216,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
                                  : T(0);
         }
         __syncthreads();
-        for (int ks = 0; ks < na; ks += 4) {
+        for (int ks = 4 * sg; ks < na; ks += 4 * kspl) {
           const int al = ks + lk;
           const int pk = aidx[a0 + al];
           T b[NT];
@@ -206,7 +225,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
 #pragma unroll
           for (int rt = 0; rt < kRT; ++rt) {
             if (!tile_on[rt]) continue;
-            const int row = (wave + kWaves * rt) * 16 + lr;
+            const int row = (rg + wrows * rt) * 16 + lr;
             T v = F[(0 * P1 + unpack(pk, 0)) * kRowsP + row];
 #pragma unroll
             for (int d = 1; d < D; ++d) v *= F[(d * P1 + unpack(pk, d)) * kRowsP + row];
@@ -228,7 +247,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
       int nb = n0, j0 = 0, pnj = 0;
       // a run of sources with adjacent point ranges is staged as one source
       auto fetch = [&]() {
-        const int run = pat.near_run[nb];
+        const int run = min(pat.near_run[nb], n1 - nb);
         const int s = pat.near_src[nb], sl = pat.near_src[nb + run - 1];
         const int sb = cols.begin[s], ss = cols.begin[sl] + cols.size[sl] - sb;
         pnj = min(kChunk, ss - j0);
@@ -314,20 +333,20 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
 #pragma unroll
               for (int v = 0; v < 4; ++v) {
                 if (!decltype(full)::value && s0 + 4 * v >= nj) break;
-                const T e = gram_kernel<KT>(__builtin_fabs(r2[v]), kp);
+                const T e = gram_kernel<KT>(r2[v], kp, tab);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
                   if (nt < ntl) acc[rt][nt] = M::mma(e, bv[v][nt], acc[rt][nt]);
               }
             }
           };
-          int s0 = 0;
-          for (; s0 + 16 <= nj; s0 += 16) group(s0, std::true_type{});
+          int s0 = 16 * sg;
+          for (; s0 + 16 <= nj; s0 += 16 * kspl) group(s0, std::true_type{});
           if (s0 < nj) group(s0, std::false_type{});
         } else {
           const int nsteps = (nj + 3) & ~3;
 #pragma unroll 2
-          for (int ks = 0; ks < nsteps; ks += 4) {
+          for (int ks = 4 * sg; ks < nsteps; ks += 4 * kspl) {
             const int sj = ks + lk;
             T y[D];
 #pragma unroll
@@ -338,7 +357,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
 #pragma unroll
             for (int rt = 0; rt < kRT; ++rt) {
               if (!tile_on[rt]) continue;
-              T r2 = 0;
+              T r2 = kR2Start<KT, T>;
 #pragma unroll
               for (int d = 0; d < D; ++d) {
                 const T dd = x[rt][d] - y[d];
@@ -346,12 +365,12 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
               }
               if constexpr (MULTI) {
                 T ev[3];
-                kernel_r2_all<KT, T>(r2, kp, ev);
+                kernel_r2_all<KT, T>(r2, kp, tab, ev);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
                   if (nt < ntl) acc[rt][nt] = M::mma(pick_variant(ev, tv[nt]), b[nt], acc[rt][nt]);
               } else {
-                const T e = kernel_r2<KT, T>(r2, kp);
+                const T e = entry_value<KT, T>(r2, kp, tab);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
                   if (nt < ntl) acc[rt][nt] = M::mma(e, b[nt], acc[rt][nt]);
@@ -360,17 +379,44 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           }
         }
       }
-      // store: C row crow(lk, v) of tile (wave + 4 rt), column lr of rhs tile nt
+      if (kspl > 1) {
+        T *Red = U;  // [16 R][16], one column tile at a time
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          for (int g = 1; g <= kspl; ++g) {
+            __syncthreads();
+            if (sg != g % kspl) continue;
+#pragma unroll
+            for (int rt = 0; rt < kRT; ++rt) {
+              if (!tile_on[rt]) continue;
+#pragma unroll
+              for (int v = 0; v < 4; ++v) {
+                T *dst = Red + ((rg + wrows * rt) * 16 + M::crow(lk, v)) * 16 + lr;
+                const T sum = (g == 1 ? T(0) : *dst) + acc[rt][nt][v];
+                if (g < kspl)
+                  *dst = sum;
+                else
+                  acc[rt][nt][v] = sum;
+              }
+            }
+          }
+        }
+      }
+      // store: C row crow(lk, v) of tile (rg + wrows rt), column lr of rhs tile nt
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
-        if (!tile_on[rt]) continue;
+        if (!tile_on[rt] || sg != 0) continue;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const int col = rc + nt * 16 + lr;
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int i = pbase + (wave + kWaves * rt) * 16 + M::crow(lk, v);
+            const int i = pbase + (rg + wrows * rt) * 16 + M::crow(lk, v);
             if (i < sz && col < nrhs) {
+              if (gridDim.y > 1) {
+                part[((int64_t)blockIdx.y * rows.npts + b0 + i) * nrhs + col] = acc[rt][nt][v];
+                continue;
+              }
               const int64_t row = natural ? (int64_t)rows.perm[b0 + i] : (int64_t)(b0 + i);
               double *p = out + row + (int64_t)col * ldo;
               if (split)
@@ -397,7 +443,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
                                                        DevPatternView pat, InterpParams<T> ip,
                                                        KernelParams<T> kp, int nrhs,
                                                        const T *__restrict__ mom,
-                                                       T *__restrict__ tlhs) {
+                                                       T *__restrict__ tlhs, T *__restrict__ part) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int NC = 16 * NT;
@@ -407,6 +453,8 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
   // matrix cores, as in the leaf output (16 source nodes per distance MFMA)
   constexpr bool kGram = sizeof(T) == 8 && !MULTI && kGramNear<KT> && D <= 3;
   extern __shared__ unsigned char smem_raw[];
+  __shared__ double tab[kTableEntry<KT, T> ? 64 : 1];
+  if constexpr (kTableEntry<KT, T>) load_exp2_table(tab);
   const int q = ip.q;
   const int qpad = (q + 3) & ~3;
   T *U = reinterpret_cast<T *>(smem_raw);  // [D][qpad] unit coordinates of the nodes
@@ -420,8 +468,11 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
   const int lr = lane & 15, lk = lane >> 4;
   const int task = pat.far_order[blockIdx.x];
   if (task < 0) return;
-  const int t = pat.far_task[4 * task], f0 = pat.far_task[4 * task + 1],
-            f1 = pat.far_task[4 * task + 2];
+  const int t = pat.far_task[4 * task];
+  int f0 = pat.far_task[4 * task + 1], f1 = pat.far_task[4 * task + 2];
+  list_part(f0, f1);
+  // sums of this part: its slab, or the coupling sums themselves
+  T *dst_all = gridDim.y > 1 ? part + (int64_t)blockIdx.y * rows.ncl * ip.q * nrhs : tlhs;
   const bool split = (pat.far_task[4 * task + 3] & kTaskSplit) != 0;
   // K-split: with R row tiles, kspl groups of waves (4 for R <= kRT, 2 for
   // R <= 2 kRT, else 1) share the K-steps, so that every wave holds up to kRT
@@ -521,7 +572,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
             const acc_t r2 = M::mma(ga, gx[rt], acc_t{gxx[rt], gxx[rt], gxx[rt], gxx[rt]});
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-              const T e = gram_kernel<KT>(__builtin_fabs(r2[v]), kp);
+              const T e = gram_kernel<KT>(r2[v], kp, tab);
 #pragma unroll
               for (int nt = 0; nt < NT; ++nt)
                 if (nt < ntl) acc[rt][nt] = M::mma(e, bv[v][nt], acc[rt][nt]);
@@ -542,7 +593,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt) {
           if (!tile_on[rt]) continue;
-          T r2 = 0;
+          T r2 = kR2Start<KT, T>;
 #pragma unroll
           for (int d = 0; d < D; ++d) {
             const T dd = x[rt][d] - y[d];
@@ -550,12 +601,12 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
           }
           if constexpr (MULTI) {
             T ev[3];
-            kernel_r2_all<KT, T>(r2, kp, ev);
+            kernel_r2_all<KT, T>(r2, kp, tab, ev);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
               if (nt < ntl) acc[rt][nt] = M::mma(pick_variant(ev, tv[nt]), b[nt], acc[rt][nt]);
           } else {
-            const T e = kernel_r2<KT, T>(r2, kp);
+            const T e = entry_value<KT, T>(r2, kp, tab);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
               if (nt < ntl) acc[rt][nt] = M::mma(e, b[nt], acc[rt][nt]);
@@ -732,7 +783,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
       for (int e = threadIdx.x; e < q * NC; e += blockDim.x) {
         const int alpha = e / NC, c = e - alpha * NC;
         if (c < 16 * ntl && rc + c < nrhs) {
-          T *p = tlhs + ((int64_t)t * q + alpha) * nrhs + rc + c;
+          T *p = dst_all + ((int64_t)t * q + alpha) * nrhs + rc + c;
           if (split)
             atomic_accumulate(p, Red[e]);
           else
@@ -751,7 +802,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
           for (int v = 0; v < 4; ++v) {
             const int alpha = (rg + wrows * rt) * 16 + M::crow(lk, v);
             if (alpha < q && col < nrhs) {
-              T *p = tlhs + ((int64_t)t * q + alpha) * nrhs + col;
+              T *p = dst_all + ((int64_t)t * q + alpha) * nrhs + col;
               if (split)
                 atomic_accumulate(p, acc[rt][nt][v]);
               else
@@ -896,43 +947,46 @@ inline bool mfma_multi(int kt, int vmask) {
 }
 
 template <typename T, int D, int NT, bool MULTI>
-hipError_t launch_mfma_nt(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                          const DevPatternView &pat, const InterpParams<T> &ip,
-                          const KernelParams<T> &kp, int nrhs, const T *xs, const T *mom,
-                          T *tlhs, double *out, int64_t ldo, bool natural, hipStream_t stream) {
-  const size_t lds_out = leaf_output_mfma_lds<T, NT>(D, ip.P1, ip.q);
-  const size_t lds_cpl = coupling_mfma_lds<T, NT>(D, ip.q, ip.td != 0);
-  const int base = kp.kt % KT_COUNT;
+hipError_t launch_mfma_nt(bool output, const MfmaLaunch<T> &a) {
+  const size_t lds_out = leaf_output_mfma_lds<T, NT>(D, a.ip.P1, a.ip.q);
+  const size_t lds_cpl = coupling_mfma_lds<T, NT>(D, a.ip.q, a.ip.td != 0);
+  const int base = a.kp.kt % KT_COUNT;
   // MULTI kernels take the base kernel; single-variant kernels take kp.kt
   // (a derivative variant there goes to the run-time switch, K = -1)
-  const int key = MULTI ? base : kp.kt;
-#define FMCA_MFMA_CASE(K)                                                                  \
-  case K:                                                                                  \
-    if (output)                                                                            \
-      hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI>), dim3(pat.nnear_order),  \
-                         dim3(256), lds_out, stream, rows, cols, pat, ip, kp, nrhs, xs,    \
-                         tlhs, out, ldo, natural ? 1 : 0);                                 \
-    else                                                                                   \
-      hipLaunchKernelGGL((k_coupling_mfma<T, D, K, NT, MULTI>), dim3(pat.nfar_order),      \
-                         dim3(256), lds_cpl, stream, rows, cols, pat, ip, kp, nrhs, mom,   \
-                         tlhs);                                                            \
-    break;
+  const int key = MULTI ? base : a.kp.kt;
+  T *slabs = nullptr;
+  const int parts = launch_parts(output, a, &slabs);
+  const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
+#define FMCA_MFMA_LAUNCH(K)                                                                   \
+  if (output)                                                                                 \
+    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI>), grid, dim3(256), lds_out,    \
+                       a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs, a.tlhs,     \
+                       a.out, a.ldo, a.natural ? 1 : 0, slabs);                               \
+  else                                                                                        \
+    hipLaunchKernelGGL((k_coupling_mfma<T, D, K, NT, MULTI>), grid, dim3(256), lds_cpl,       \
+                       a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs,    \
+                       slabs)
   switch (key) {
-    FMCA_MFMA_CASE(KT_EXPONENTIAL)
-    FMCA_MFMA_CASE(KT_MATERN32)
-    FMCA_MFMA_CASE(KT_MATERN52)
-    FMCA_MFMA_CASE(KT_GAUSSIAN)
+    case KT_EXPONENTIAL:
+      FMCA_MFMA_LAUNCH(KT_EXPONENTIAL);
+      break;
+    case KT_MATERN32:
+      FMCA_MFMA_LAUNCH(KT_MATERN32);
+      break;
+    case KT_MATERN52:
+      FMCA_MFMA_LAUNCH(KT_MATERN52);
+      break;
+    case KT_GAUSSIAN:
+      FMCA_MFMA_LAUNCH(KT_GAUSSIAN);
+      break;
     default:
-      if (output)
-        hipLaunchKernelGGL((k_leaf_output_mfma<T, D, -1, NT, MULTI>), dim3(pat.nnear_order),
-                           dim3(256), lds_out, stream, rows, cols, pat, ip, kp, nrhs, xs, tlhs,
-                           out, ldo, natural ? 1 : 0);
-      else
-        hipLaunchKernelGGL((k_coupling_mfma<T, D, -1, NT, MULTI>), dim3(pat.nfar_order),
-                           dim3(256), lds_cpl, stream, rows, cols, pat, ip, kp, nrhs, mom, tlhs);
+      FMCA_MFMA_LAUNCH(-1);
   }
-#undef FMCA_MFMA_CASE
-  return hipGetLastError();
+#undef FMCA_MFMA_LAUNCH
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || parts == 1) return e;
+  return launch_add_parts<T>(output, a.rows, a.ip.q, a.nrhs, parts, slabs, a.tlhs, a.out, a.ldo,
+                             a.natural, a.stream);
 }
 
 // rhs columns per pass: 16 or 32.  Wider passes (64 columns) take fewer
@@ -945,28 +999,14 @@ int mfma_nt(int nrhs, bool multi) {
   return nrhs <= 16 ? 1 : 2;
 }
 
-template <typename T, int D, bool MULTI>
-hipError_t launch_mfma_dm(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                          const DevPatternView &pat, const InterpParams<T> &ip,
-                          const KernelParams<T> &kp, int nrhs, const T *xs, const T *mom,
-                          T *tlhs, double *out, int64_t ldo, bool natural, hipStream_t stream) {
-  if (mfma_nt<T>(nrhs, MULTI) == 1)
-    return launch_mfma_nt<T, D, 1, MULTI>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs,
-                                          out, ldo, natural, stream);
-  return launch_mfma_nt<T, D, 2, MULTI>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs,
-                                        out, ldo, natural, stream);
-}
-
 template <typename T, int D>
-hipError_t launch_mfma_d(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                         const DevPatternView &pat, const InterpParams<T> &ip,
-                         const KernelParams<T> &kp, int nrhs, const T *xs, const T *mom, T *tlhs,
-                         double *out, int64_t ldo, bool natural, hipStream_t stream) {
-  if (mfma_multi(kp.kt, kp.vmask))
-    return launch_mfma_dm<T, D, true>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out,
-                                      ldo, natural, stream);
-  return launch_mfma_dm<T, D, false>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out,
-                                     ldo, natural, stream);
+hipError_t launch_mfma_d(bool output, const MfmaLaunch<T> &a) {
+  const bool multi = mfma_multi(a.kp.kt, a.kp.vmask);
+  if (mfma_nt<T>(a.nrhs, multi) == 1)
+    return multi ? launch_mfma_nt<T, D, 1, true>(output, a)
+                 : launch_mfma_nt<T, D, 1, false>(output, a);
+  return multi ? launch_mfma_nt<T, D, 2, true>(output, a)
+               : launch_mfma_nt<T, D, 2, false>(output, a);
 }
 
 }  // namespace
@@ -1000,7 +1040,8 @@ hipError_t launch_upward_leaf_mfma(const DevTreeView<float> &tr, const InterpPar
 template <typename T>
 bool mfma_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vmask, int td) {
   if (nrhs < kMfmaMinRhs) return false;  // the VALU forms are faster there
-  const size_t limit = 64 * 1024;
+  // less the exponential's table of the FP64 forms
+  const size_t limit = 64 * 1024 - (sizeof(T) == 8 ? 512 : 16);
   const int nt = mfma_nt<T>(nrhs, mfma_multi(kt, vmask));
   if (output)
     return (nt == 1 ? leaf_output_mfma_lds<T, 1>(D, P1, q)
@@ -1011,35 +1052,21 @@ bool mfma_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vma
 }
 
 template <typename T>
-hipError_t launch_mfma(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
-                       const DevPatternView &pat, const InterpParams<T> &ip,
-                       const KernelParams<T> &kp, int nrhs, const T *xs, const T *mom, T *tlhs,
-                       double *out, int64_t ldo, bool natural, hipStream_t stream) {
-  switch (rows.dim) {
+hipError_t launch_mfma(bool output, const MfmaLaunch<T> &a) {
+  switch (a.rows.dim) {
     case 1:
-      return launch_mfma_d<T, 1>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                                 natural, stream);
+      return launch_mfma_d<T, 1>(output, a);
     case 2:
-      return launch_mfma_d<T, 2>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                                 natural, stream);
+      return launch_mfma_d<T, 2>(output, a);
     case 3:
-      return launch_mfma_d<T, 3>(output, rows, cols, pat, ip, kp, nrhs, xs, mom, tlhs, out, ldo,
-                                 natural, stream);
+      return launch_mfma_d<T, 3>(output, a);
   }
   return hipErrorInvalidValue;
 }
 
 template bool mfma_supported<float>(bool, int, int, int, int, int, int, int);
 template bool mfma_supported<double>(bool, int, int, int, int, int, int, int);
-template hipError_t launch_mfma<float>(bool, const DevTreeView<float> &,
-                                       const DevTreeView<float> &, const DevPatternView &,
-                                       const InterpParams<float> &, const KernelParams<float> &,
-                                       int, const float *, const float *, float *, double *,
-                                       int64_t, bool, hipStream_t);
-template hipError_t launch_mfma<double>(bool, const DevTreeView<double> &,
-                                        const DevTreeView<double> &, const DevPatternView &,
-                                        const InterpParams<double> &, const KernelParams<double> &,
-                                        int, const double *, const double *, double *, double *,
-                                        int64_t, bool, hipStream_t);
+template hipError_t launch_mfma<float>(bool, const MfmaLaunch<float> &);
+template hipError_t launch_mfma<double>(bool, const MfmaLaunch<double> &);
 
 }  // namespace fmca_amd
