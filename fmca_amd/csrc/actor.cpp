@@ -1459,6 +1459,348 @@ constexpr int kBasisChunk = 8;  // slot pairs per basis allocation
 // 10 more iterations, the same FP64 actions).
 constexpr double kInnerTarget = 0.5;
 
+// T and T a of one block (32 x 32, row-major) from its Gram matrix G = Y^T Y
+// and H = Y^T R: with G = D L L^T D in pivoted order on its columns (D = diag
+// ||y_b||), T = D^-1 L^-T makes Y T orthonormal and a = T^T H are the
+// coefficients of the residuals on it.  Left out are columns whose pivot falls
+// below kBlockRank of the largest (they depend on the others) and columns of
+// which the window took all but a share `lost` of the norm (sq: the squared
+// norms taken): what is left of those is the rounding of the stored pairs and
+// of the matvec, and no longer an image of its direction.  Returns the rank.
+constexpr double kBlockRank = 1e-8;
+int block_factor(const double *G, const double *H, const double *sq, double lost, double *T,
+                 double *Ta) {
+  constexpr int N = kBlockCols;
+  std::fill(T, T + N * N, 0.0);
+  std::fill(Ta, Ta + N * N, 0.0);
+  double d[N], M[N][N], L[N][N] = {{0}};
+  int idx[N], m = 0;
+  for (int b = 0; b < N; ++b)
+    if (G[b * N + b] > lost * lost * sq[b] && std::isfinite(G[b * N + b])) {
+      d[m] = std::sqrt(G[b * N + b]);
+      idx[m++] = b;
+    }
+  for (int i = 0; i < m; ++i)
+    for (int j = 0; j < m; ++j) M[i][j] = G[idx[i] * N + idx[j]] / (d[i] * d[j]);
+  int piv[N], rank = 0;
+  std::iota(piv, piv + N, 0);
+  double top = 0;
+  for (int k = 0; k < m; ++k) {
+    int best = k;
+    for (int i = k + 1; i < m; ++i)
+      if (M[piv[i]][piv[i]] > M[piv[best]][piv[best]]) best = i;
+    std::swap(piv[k], piv[best]);
+    const double p = M[piv[k]][piv[k]];
+    if (k == 0) top = p;
+    if (!(p > kBlockRank * top)) break;
+    const double r = std::sqrt(p);
+    L[piv[k]][k] = r;
+    for (int i = k + 1; i < m; ++i) L[piv[i]][k] = M[piv[i]][piv[k]] / r;
+    for (int i = k + 1; i < m; ++i)
+      for (int j = k + 1; j < m; ++j) M[piv[i]][piv[j]] -= L[piv[i]][k] * L[piv[j]][k];
+    ++rank;
+  }
+  // column c of L^-T (rank x rank, pivot order): back substitution
+  for (int c = 0; c < rank; ++c) {
+    double x[N] = {0};
+    for (int i = c; i >= 0; --i) {
+      double v = i == c ? 1.0 : 0.0;
+      for (int j = i + 1; j <= c; ++j) v -= L[piv[j]][i] * x[j];
+      x[i] = v / L[piv[i]][i];
+    }
+    for (int i = 0; i <= c; ++i) T[idx[piv[i]] * N + c] = x[i] / d[piv[i]];
+  }
+  double A[N][N] = {{0}};
+  for (int c = 0; c < rank; ++c)
+    for (int b = 0; b < N; ++b) {
+      double v = 0;
+      for (int k = 0; k < m; ++k) v += T[idx[k] * N + c] * H[idx[k] * N + b];
+      A[c][b] = v;  // H is zero in inactive columns
+    }
+  for (int k = 0; k < m; ++k)
+    for (int b = 0; b < N; ++b) {
+      double v = 0;
+      for (int c = 0; c < rank; ++c) v += T[idx[k] * N + c] * A[c][b];
+      Ta[idx[k] * N + b] = v;
+    }
+  return rank;
+}
+
+// Block GCR, the form of FMCA_SOLVER_GCR for two columns or more: the columns
+// of a block of up to 32 share one Krylov space.  Each iteration multiplies
+// the residuals (scaled to unit norm), orthogonalises the image block against
+// the stored ones (one classical Gram-Schmidt pass, applied to the direction
+// block as well), makes it orthonormal through its Gram matrix, and removes
+// from every residual of the block its component on the whole new image
+// block: ||r|| is minimised over the directions of all columns, so the
+// iterations fall with the block size (n = 1e6, 32 columns: 58 -> 14; one
+// iteration costs one action either way).  Pairs stay consistent with their
+// own matvec as in gcr_solve, and the residual replacement is the same.
+// A block whose columns are all below their target, or have dropped by
+// refine_factor, gives no further directions until the next replacement: the
+// recurrence with FP32 pairs stalls at about 3e-8 of a cycle's start, and pairs
+// made from there on are rounding.  When no column has a new direction left (rank 0: the window
+// spans the space to rounding) the residual is replaced and projected, which
+// still reduces it by the rounding of the stored pairs; the solve stops when
+// that no longer halves it.  One column is served by gcr_solve, whose kernels
+// read each stored pair once in vector form.
+template <typename S>
+fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr, double *d_x,
+                            int64_t ld_x, const fmca_cg_options *opts, fmca_cg_result *res,
+                            hipStream_t sm, std::chrono::steady_clock::time_point t0) {
+  const int64_t n = a->n, ld = (n + 63) / 64 * 64;
+  const double ridge = opts->ridge;
+  const bool cl = a->shared;
+  const uint32_t *perm = a->d_rows_i.perm.as<uint32_t>();
+  const size_t vec = (size_t)ld * nr;
+  const int prec = opts->precision;
+  const int max_iter = opts->max_iter > 0 ? opts->max_iter : 100000;
+  const int max_updates = opts->max_outer > 0 ? opts->max_outer : 1000;
+  const double delta = (opts->refine_factor > 0 && opts->refine_factor < 1) ? opts->refine_factor
+                                                                              : 0.1;
+  const int ng = block_groups(nr), bs = block_cols(nr);
+  constexpr int kMat = kBlockCols * kBlockCols;
+  // window size
+  const size_t pair_bytes = 2 * vec * sizeof(S);
+  int m = opts->max_basis;
+  if (m < 0 || m > kBasisMax)
+    return fail(FMCA_ERR_INVALID_ARGUMENT, "max_basis must be in [0, 256]");
+  if (m == 0) {
+    size_t free_b = 0, total_b = 0;
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    size_t budget = free_b / 2;
+    const int64_t cap = g_dev_limit.load();
+    if (cap > 0) {
+      const int64_t left = cap - g_dev_live.load() - (int64_t)(5 * vec * sizeof(double));
+      budget = std::min<size_t>(budget, left > 0 ? (size_t)left / 2 : 0);
+    }
+    m = (int)std::min<size_t>((size_t)kBasisMax, budget / pair_bytes);
+    m = std::min(m, max_iter + 1);
+  }
+  if (m < 2) return fail(FMCA_ERR_OUT_OF_MEMORY, "GCR needs room for two basis pairs");
+  HIP_TRY(a->cg_ws.alloc(5 * vec * sizeof(double)));
+  // scalars: rr, small matrices (window coefficients; Gram; T and T a), partial
+  // sums, active flags
+  const size_t n_coef = (size_t)ng * m * kMat, n_small = (size_t)ng * 2 * kMat,
+               n_sq = (size_t)ng * kBlockCols;
+  const size_t n_scratch =
+      std::max(block_scratch(ld, nr, m), blas1_dot_scratch(nr)) / sizeof(double);
+  const size_t nd = (size_t)nr + n_coef + 2 * n_small + n_sq + n_scratch;
+  HIP_TRY(a->cg_scal.alloc(nd * sizeof(double) + 2 * (size_t)nr * sizeof(int)));
+  double *w = a->cg_ws.as<double>();
+  double *B = w, *X = w + vec, *R = w + 2 * vec, *Y = w + 3 * vec, *W = w + 4 * vec;
+  double *sc = a->cg_scal.as<double>();
+  // d_sq follows d_gram: one download
+  double *d_coef = sc, *d_gram = d_coef + n_coef, *d_sq = d_gram + n_small,
+         *d_mats = d_sq + n_sq, *d_scratch = d_mats + n_small, *d_rr = d_scratch + n_scratch;
+  int *d_active = reinterpret_cast<int *>(d_rr + nr), *d_live = d_active + nr;
+  // least share of an image that the window may leave (see block_factor): well
+  // above the rounding of the matvec (4e-6 for the FP32 forms)
+  const double lost = prec == FMCA_PRECISION_FP64 ? 1e-10 : 1e-3;
+  auto chk = [&](hipError_t e, const char *what) { return from_hip(e, what); };
+#define GCR_TRY(expr)                                 \
+  do {                                                \
+    fmca_status _s = chk((expr), #expr);              \
+    if (_s != FMCA_OK) return _s;                     \
+  } while (0)
+  auto matvec = [&](const double *in, double *out, int p) -> fmca_status {
+    if (p == FMCA_PRECISION_FP64) res->matvecs_fp64++; else res->matvecs_fp32++;
+    return enqueue_any(a, in, ld, nr, out, ld, p, !cl, false, sm);
+  };
+  std::vector<double> rn2(nr), bn2(nr), target(nr), rmax(nr), gram(n_small + n_sq),
+      mats(n_small);
+  std::vector<int> flags(2 * (size_t)nr);  // active columns, live ones
+  int *active = flags.data(), *live = active + nr;
+  auto read_norms = [&](const double *v) -> fmca_status {
+    GCR_TRY(blas1_dot(n, nr, v, ld, v, ld, d_rr, d_scratch, sm));
+    GCR_TRY(hipMemcpyAsync(rn2.data(), d_rr, nr * sizeof(double), hipMemcpyDeviceToHost, sm));
+    GCR_TRY(hipStreamSynchronize(sm));
+    return FMCA_OK;
+  };
+  auto push_flags = [&]() -> hipError_t {
+    return hipMemcpyAsync(d_active, active, 2 * nr * sizeof(int), hipMemcpyHostToDevice, sm);
+  };
+  auto residual = [&]() -> fmca_status {  // R = B - (K + ridge I) X, FP64
+    fmca_status s = matvec(X, Y, FMCA_PRECISION_FP64);
+    if (s != FMCA_OK) return s;
+    GCR_TRY(blas1_residual(n, nr, ridge, B, ld, Y, ld, X, ld, R, ld, sm));
+    return read_norms(R);
+  };
+  // basis slots: chunks allocated as the window grows, released at the end
+  std::vector<const S *> qtab(m, nullptr), ptab(m, nullptr);
+  a->basis.clear();
+  HIP_TRY(a->basis_tab.alloc(2 * (size_t)m * sizeof(void *)));
+  const S *const *d_qtab = reinterpret_cast<const S *const *>(a->basis_tab.p);
+  const S *const *d_ptab = d_qtab + m;
+  int allocated = 0;
+  auto ensure_slot = [&](int slot) -> fmca_status {
+    if (slot < allocated) return FMCA_OK;
+    auto buf = std::make_unique<DevBuf>();
+    const int k = std::min(kBasisChunk, m - allocated);
+    hipError_t e = buf->alloc((size_t)k * pair_bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(FMCA_ERR_OUT_OF_MEMORY, "GCR basis allocation failed (lower max_basis)");
+    }
+    S *base = buf->as<S>();
+    for (int j = 0; j < k; ++j) {
+      ptab[allocated + j] = base + (size_t)j * vec;
+      qtab[allocated + j] = base + (size_t)(k + j) * vec;
+    }
+    a->basis.push_back(std::move(buf));
+    allocated += k;
+    GCR_TRY(hipMemcpyAsync(a->basis_tab.p, qtab.data(), m * sizeof(void *),
+                           hipMemcpyHostToDevice, sm));
+    GCR_TRY(hipMemcpyAsync(reinterpret_cast<char *>(a->basis_tab.p) + m * sizeof(void *),
+                           ptab.data(), m * sizeof(void *), hipMemcpyHostToDevice, sm));
+    // the host tables change when the next chunk arrives
+    GCR_TRY(hipStreamSynchronize(sm));
+    return FMCA_OK;
+  };
+  fmca_status st;
+  // zero rows from n on, in every vector
+  GCR_TRY(blas1_fill(5 * (int64_t)vec, 1, 0.0, w, 5 * (int64_t)vec, sm));
+  if (cl) {
+    GCR_TRY(blas1_permute(n, nr, perm, true, d_b, ld_b, B, ld, sm));
+    GCR_TRY(blas1_permute(n, nr, perm, true, d_x, ld_x, X, ld, sm));
+  } else {
+    const size_t row = n * sizeof(double);
+    GCR_TRY(hipMemcpy2DAsync(B, ld * sizeof(double), d_b, ld_b * sizeof(double), row, nr,
+                             hipMemcpyDeviceToDevice, sm));
+    GCR_TRY(hipMemcpy2DAsync(X, ld * sizeof(double), d_x, ld_x * sizeof(double), row, nr,
+                             hipMemcpyDeviceToDevice, sm));
+  }
+  if ((st = read_norms(B)) != FMCA_OK) return st;
+  bn2 = rn2;
+  for (int j = 0; j < nr; ++j)
+    if (bn2[j] == 0) bn2[j] = 1;  // zero rhs: absolute residual
+  // r = b - (K + ridge I) x, FP64; exactly b when x = 0
+  if ((st = read_norms(X)) != FMCA_OK) return st;
+  if (std::all_of(rn2.begin(), rn2.end(), [](double v) { return v == 0; })) {
+    GCR_TRY(hipMemcpyAsync(R, B, vec * sizeof(double), hipMemcpyDeviceToDevice, sm));
+    if ((st = read_norms(R)) != FMCA_OK) return st;
+  } else if ((st = residual()) != FMCA_OK) {
+    return st;
+  }
+  bool any = false;
+  double worst = 0;
+  for (int j = 0; j < nr; ++j) {
+    rmax[j] = std::sqrt(rn2[j]);
+    target[j] = opts->tol * std::sqrt(bn2[j]);
+    active[j] = live[j] = rmax[j] > target[j];
+    any = any || active[j];
+    worst = std::max(worst, rmax[j] / std::sqrt(bn2[j]));
+  }
+  res->rel_residual = worst;
+  GCR_TRY(push_flags());
+  int first = 0, count = 0;
+  double stuck_at = std::numeric_limits<double>::infinity();  // residual of the last rank 0
+  while (any && res->iterations < max_iter && res->outer < max_updates) {
+    // the image block (K + ridge I) r of the unit residuals, orthogonal to the
+    // window (Y), and its directions (W)
+    if ((st = matvec(R, Y, prec)) != FMCA_OK) return st;
+    GCR_TRY(block_prep(ld, nr, ridge, R, d_rr, d_live, Y, W, sm));
+    if (count == m) {  // full: drop the oldest pair, whose slot takes the new one
+      first = (first + 1) % m;
+      --count;
+    }
+    const int slot = (first + count) % m;
+    if ((st = ensure_slot(slot)) != FMCA_OK) return st;
+    GCR_TRY(block_dots<S>(ld, nr, Y, d_qtab, first, count, m, d_active, d_coef, d_scratch, sm));
+    GCR_TRY(block_combine<S>(ld, nr, d_qtab, d_ptab, first, count, m, d_coef, d_active, Y, -1.0,
+                             W, -1.0, sm));
+    GCR_TRY(block_gram(ld, nr, Y, R, d_active, d_gram, d_scratch, sm));
+    GCR_TRY(block_coef_norms(nr, count, d_coef, d_sq, sm));
+    GCR_TRY(hipMemcpyAsync(gram.data(), d_gram, gram.size() * sizeof(double),
+                           hipMemcpyDeviceToHost, sm));
+    GCR_TRY(hipStreamSynchronize(sm));
+    int rank = 0;
+    for (int g = 0; g < ng; ++g)
+      rank += block_factor(&gram[(size_t)2 * g * kMat], &gram[(size_t)(2 * g + 1) * kMat],
+                           &gram[n_small + (size_t)g * kBlockCols], lost,
+                           &mats[(size_t)2 * g * kMat], &mats[(size_t)(2 * g + 1) * kMat]);
+    GCR_TRY(hipMemcpyAsync(d_mats, mats.data(), n_small * sizeof(double), hipMemcpyHostToDevice,
+                           sm));
+    GCR_TRY(block_apply<S>(ld, nr, Y, W, d_mats, d_active, const_cast<S *>(qtab[slot]),
+                           const_cast<S *>(ptab[slot]), R, X, sm));
+    ++count;
+    if ((st = read_norms(R)) != FMCA_OK) return st;
+    res->iterations++;
+    bool all_ready = true, all_done = true, changed = false;
+    double top = 0;
+    for (int g = 0; g < ng; ++g) {
+      bool ready = true;  // every column of the block
+      const int c0 = g * bs, c1 = std::min(nr, c0 + bs);
+      for (int j = c0; j < c1; ++j) {
+        if (!active[j]) continue;
+        const double rn = std::sqrt(rn2[j]);
+        if (!std::isfinite(rn)) return fail(FMCA_ERR_NONFINITE, "GCR residual is not finite");
+        // lower precision: the iterated residual runs to kInnerTarget tol
+        const bool done = rn <= (prec == FMCA_PRECISION_FP64 ? 1.0 : kInnerTarget) * target[j];
+        all_done = all_done && done;
+        ready = ready && (done || (prec != FMCA_PRECISION_FP64 && rn < delta * rmax[j]));
+        top = std::max(top, rn / std::sqrt(bn2[j]));
+      }
+      all_ready = all_ready && ready;
+      // a block that is ready waits for the others: further directions would
+      // only come from the rounding of its recurrence
+      for (int j = c0; j < c1; ++j) {
+        const int on = active[j] && !ready;
+        changed = changed || live[j] != on;
+        live[j] = on;
+      }
+    }
+    const bool update = prec == FMCA_PRECISION_FP64 ? all_done : all_ready;
+    if (!update && rank > 0) {
+      if (changed) GCR_TRY(push_flags());
+      continue;
+    }
+    if (rank == 0) {
+      if (!(top < 0.5 * stuck_at)) break;
+      stuck_at = top;
+    }
+    // FP64 residual; columns that meet tol stop, the others are projected
+    if ((st = residual()) != FMCA_OK) return st;
+    res->outer++;
+    worst = 0;
+    any = false;
+    for (int j = 0; j < nr; ++j) {
+      const double rn = std::sqrt(rn2[j]);
+      worst = std::max(worst, rn / std::sqrt(bn2[j]));
+      if (active[j] && rn <= target[j]) active[j] = 0;
+      live[j] = active[j];
+      any = any || active[j];
+    }
+    res->rel_residual = worst;
+    GCR_TRY(push_flags());
+    if (!any) break;
+    GCR_TRY(block_dots<S>(ld, nr, R, d_qtab, first, count, m, d_active, d_coef, d_scratch, sm));
+    GCR_TRY(block_combine<S>(ld, nr, d_qtab, d_ptab, first, count, m, d_coef, d_active, R, -1.0,
+                             X, 1.0, sm));
+    if ((st = read_norms(R)) != FMCA_OK) return st;
+    for (int j = 0; j < nr; ++j)
+      if (active[j]) rmax[j] = std::sqrt(rn2[j]);
+  }
+  res->converged = !any;
+  if (any) {  // stopped by a cap: report the FP64 residual of the returned x
+    if ((st = residual()) != FMCA_OK) return st;
+    worst = 0;
+    for (int j = 0; j < nr; ++j) worst = std::max(worst, std::sqrt(rn2[j] / bn2[j]));
+    res->rel_residual = worst;
+  }
+  if (cl)
+    GCR_TRY(blas1_permute(n, nr, perm, false, X, ld, d_x, ld_x, sm));
+  else
+    GCR_TRY(hipMemcpy2DAsync(d_x, ld_x * sizeof(double), X, ld * sizeof(double),
+                             n * sizeof(double), nr, hipMemcpyDeviceToDevice, sm));
+  GCR_TRY(hipStreamSynchronize(sm));
+#undef GCR_TRY
+  a->basis.clear();
+  a->basis_tab.release();
+  res->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  return res->converged ? FMCA_OK : fail(FMCA_ERR_NOT_CONVERGED, "GCR did not reach tol");
+}
+
 // GCR with FP64 residual replacement, the method FMCA_SOLVER_GCR of
 // fmca_h2_cg_device (no FMCA counterpart).  GCR (Eisenstat, Elman & Schultz
 // 1983): each iteration multiplies the residual, q0 = (K + ridge I) r,
@@ -1713,8 +2055,11 @@ fmca_status fmca_h2_cg_device(fmca_h2_actor *a, const double *d_b, int64_t ld_b,
     return fail(FMCA_ERR_INVALID_ARGUMENT, "unknown solver method");
   if (opts->method == FMCA_SOLVER_GCR) {
     *res = fmca_cg_result{};
-    return opts->precision == FMCA_PRECISION_FP64
-               ? gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
+    const bool f64 = opts->precision == FMCA_PRECISION_FP64;
+    if (nrhs > 1)
+      return f64 ? block_gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
+                 : block_gcr_solve<float>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0);
+    return f64 ? gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
                : gcr_solve<float>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0);
   }
   const int64_t n = a->n;

@@ -396,6 +396,45 @@ hipError_t basis_project(int64_t n, int nrhs, const double *coef, const S *const
                          const S *const *ptab, int first, int count, int cap, double *x, double *r,
                          const int *active, double *rr, double *scratch, hipStream_t stream);
 
+// Block GCR (block_krylov.hip): blocks of up to kBlockCols columns in one
+// Krylov space; vectors with a leading dimension ld, a multiple of 64, rows
+// from n on zero.  Small matrices are 32 x 32, row-major.
+constexpr int kBlockCols = 32;
+// blocks, and columns of a block: blocks of about equal size (33 columns: 17
+// and 16, not 32 and 1, whose single column would converge four times slower)
+__host__ __device__ inline int block_groups(int nrhs) {
+  return (nrhs + kBlockCols - 1) / kBlockCols;
+}
+__host__ __device__ inline int block_cols(int nrhs) {
+  const int g = block_groups(nrhs);
+  return (nrhs + g - 1) / g;
+}
+size_t block_scratch(int64_t ld, int nrhs, int count);
+// y = (y + ridge r) / ||r||, w = r / ||r|| per live column, else zero (rr = r.r)
+hipError_t block_prep(int64_t ld, int nrhs, double ridge, const double *r, const double *rr,
+                      const int *live, double *y, double *w, hipStream_t stream);
+// out[g * count + j] = Q_j^T V of block g (zero columns for inactive rhs)
+template <typename S>
+hipError_t block_dots(int64_t ld, int nrhs, const double *v, const S *const *qtab, int first,
+                      int count, int cap, const int *active, double *out, double *scratch,
+                      hipStream_t stream);
+// sq[32 g + b]: squared norm of column b of all coefficient matrices of block g
+hipError_t block_coef_norms(int nrhs, int count, const double *coef, double *sq,
+                            hipStream_t stream);
+// out[2 g] = Y^T Y, out[2 g + 1] = Y^T R of block g
+hipError_t block_gram(int64_t ld, int nrhs, const double *y, const double *r, const int *active,
+                      double *out, double *scratch, hipStream_t stream);
+// out0 += sign0 sum_j Q_j C_j, out1 += sign1 sum_j P_j C_j (active columns)
+template <typename S>
+hipError_t block_combine(int64_t ld, int nrhs, const S *const *qtab, const S *const *ptab,
+                         int first, int count, int cap, const double *coef, const int *active,
+                         double *out0, double sign0, double *out1, double sign1,
+                         hipStream_t stream);
+// qk = Y T, pk = W T, r -= Y (T a), x += W (T a); mats: per block T, then T a
+template <typename S>
+hipError_t block_apply(int64_t ld, int nrhs, const double *y, const double *w, const double *mats,
+                       const int *active, S *qk, S *pk, double *r, double *x, hipStream_t stream);
+
 // Evaluates the device exp (fn 0 / 2) or sqrt (fn 1 / 3) used by the kernel
 // loops, in FP64 (fn 0, 1) or FP32 (fn 2, 3), on n device values.
 hipError_t launch_math_probe(int fn, const double *x, double *y, int64_t n, hipStream_t stream);
