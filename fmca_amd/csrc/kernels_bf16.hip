@@ -10,16 +10,27 @@
 // product carries about the error of an FP32 evaluation of the entry; the sum
 // accumulates in FP32 as in the FP32 forms.  One 16x16x32 BF16 instruction
 // does 8 times the multiply-adds of a 16x16x4 FP32 one in half the cycles, so
-// the three of them cost 3/16 of the FP32 matrix-core time per entry and the
-// kernels become bound by the VALU work of generating the entries.
+// the three of them cost 3/16 of the FP32 matrix-core time per entry.  The
+// squared distances come from the same instruction on three-term splits (24
+// bits, see source_operand).
+//
+// What bounds them: the vector ALU work of an entry (root, exponential,
+// polynomial, split: about 60 cycles per 64 entries) plus the part of the
+// matrix-core time that it does not hide.  Measured (ms, n = 1e6, MATERN32,
+// degree 4; before: FP32 distance MFMAs, four row tiles on each of four waves
+// at two waves per SIMD, 32 columns a pass):
+//   columns            16             32             64
+//   leaf output   7.29 -> 6.52   8.44 -> 7.70   16.6 -> 12.9
+//   coupling      5.14 -> 4.65   6.60 -> 5.76   13.2 -> 11.0
 //
 // Operand layout (gfx950): lane l supplies A[l % 16][k] and B[k][l % 16] for
 // the eight k of K-slot group l / 16; the two operands use the same k <-> (lane
 // group, element) map, so the contraction pairs them whatever that map is.
-// Lane l's eight A values are this lane's row and eight consecutive sources
-// (or source nodes) of the K-step; B is read as 16 bytes from LDS, where the
-// staged right operand is held transposed (column-major over sources).  The
-// accumulator layout is that of the 16x16 FP32 forms: item v of lane l is
+// Lane l's eight A values are this lane's row and eight sources (or source
+// nodes) of the K-step, in the order of gram_pos where the distances come from
+// the matrix cores; B is read as 16 bytes from LDS, where the staged right
+// operand is held transposed (column-major over sources).  The accumulator
+// layout is that of the 16x16 FP32 forms: item v of lane l is
 // C[4 (l / 16) + v][l % 16].
 #include <hip/hip_runtime.h>
 
@@ -40,8 +51,12 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16;
 
-constexpr int kWaves = 4;                // waves per workgroup
-constexpr int kRT = 4;                   // 16-row tiles per wave -> 256 rows per pass
+constexpr int kWaves = 8;                // waves per workgroup
+constexpr int kThreads = 64 * kWaves;
+// Row tiles per wave: two, so that four waves share a SIMD (128 registers).
+// With four tiles and two waves the entries' transcendentals, the distance
+// MFMAs and the LDS reads were exposed (n = 1e6, 32 rhs: leaf output 8.4 ms).
+constexpr int kRT = 2;                   // 16-row tiles per wave -> 256 rows per pass
 constexpr int kRows = kWaves * kRT * 16;
 constexpr int kRowsP = kRows + 16;       // padded LDS row stride of the basis factors
 constexpr int kKB = 32;                  // sources per BF16 K-step
@@ -102,6 +117,14 @@ __device__ __forceinline__ int gram_pos(int jj) {
   return (jj & ~31) | (((jj & 15) >> 2) << 3) | ((jj & 16) >> 2) | (jj & 3);
 }
 
+// The hi | lo << 16 words of two neighbouring sources (even position at) as one
+// 32-bit store to each of the two staged halves.
+__device__ __forceinline__ void store_pair(u16 *h, u16 *l, int at, float w0, float w1) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, w0), b = __builtin_bit_cast(uint32_t, w1);
+  *reinterpret_cast<uint32_t *>(h + at) = (a & 0xffffu) | (b << 16);
+  *reinterpret_cast<uint32_t *>(l + at) = (a >> 16) | (b & 0xffff0000u);
+}
+
 // the 8 bf16 values at p (16-byte aligned) as one operand
 __device__ __forceinline__ bf16x8 load8(const u16 *p) {
   return *reinterpret_cast<const bf16x8 *>(p);
@@ -119,13 +142,175 @@ __global__ __launch_bounds__(256) void k_split_inplace(float *__restrict__ x, in
   }
 }
 
+// Waves per SIMD: 4 up to 32 columns; 64 columns hold twice the accumulators
+// (leaf output n = 1e6, 64 columns: 12.9 ms at 2, 21 ms with spills at 4).
+template <int NT>
+constexpr int kOcc = NT <= 2 ? 4 : 2;
+
+// K-split of R row tiles: with fewer than 9 tiles, groups of waves share the
+// K-steps, so that every wave holds up to kRT row tiles; the groups' sums are
+// added in LDS in group order.  wave = rg + wrows sg.
+__device__ __forceinline__ int k_split(int R) {
+  return R <= kRT ? 8 : (R <= 2 * kRT ? 4 : (R <= 4 * kRT ? 2 : 1));
+}
+
+// Adds the wave groups' accumulators over LDS, one column tile at a time; the
+// sums end in group 0.  Red: [16 R][16].
+template <int NT>
+__device__ __forceinline__ void add_groups(f32x4 (&acc)[kRT][NT], float *Red, int kspl, int wrows,
+                                           int rg, int sg, const bool (&tile_on)[kRT], int lr,
+                                           int lk) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    for (int g = 1; g <= kspl; ++g) {
+      __syncthreads();
+      if (sg != g % kspl) continue;
+#pragma unroll
+      for (int rt = 0; rt < kRT; ++rt) {
+        if (!tile_on[rt]) continue;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float *dst = Red + ((rg + wrows * rt) * 16 + 4 * lk + v) * 16 + lr;
+          const float sum = (g == 1 ? 0.f : *dst) + acc[rt][nt][v];
+          if (g < kspl)
+            *dst = sum;
+          else
+            acc[rt][nt][v] = sum;
+        }
+      }
+    }
+  }
+}
+
+// acc += A B for one K-step: A = ah + al per row tile, B = Bh + Bl (LDS) per
+// column tile, the three leading products.
+template <int NT, bool ALL>
+__device__ __forceinline__ void contract(const bf16x8 (&ah)[kRT], const bf16x8 (&al)[kRT],
+                                         const u16 *Bh, const u16 *Bl,
+                                         const bool (&tile_on)[kRT], int ntl,
+                                         f32x4 (&acc)[kRT][NT]) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    if (!ALL && nt >= ntl) continue;
+    const bf16x8 bh = load8(Bh + nt * 16 * kChunkP), bl = load8(Bl + nt * 16 * kChunkP);
+#pragma unroll
+    for (int rt = 0; rt < kRT; ++rt)
+      if (ALL || tile_on[rt]) acc[rt][nt] = mma_bf16(ah[rt], bh, acc[rt][nt]);
+#pragma unroll
+    for (int rt = 0; rt < kRT; ++rt)
+      if (ALL || tile_on[rt]) acc[rt][nt] = mma_bf16(al[rt], bh, acc[rt][nt]);
+#pragma unroll
+    for (int rt = 0; rt < kRT; ++rt)
+      if (ALL || tile_on[rt]) acc[rt][nt] = mma_bf16(ah[rt], bl, acc[rt][nt]);
+  }
+}
+
+// Distance operands.  r^2 = |y|^2 - 2 x.y + |x|^2 of 16 sources and 16 targets
+// comes from one v_mfma_f32_16x16x32_bf16: every coordinate and squared norm is
+// split into three BF16 terms (24 bits), and its k-slots hold, per axis, the
+// six products down to 2^-16 (slots 6 d .. 6 d + 5: y1x1 y1x2 y2x1 y2x2 y1x3
+// y3x1), then |y|^2 against 1 (18-20) and 1 against |x|^2 (21-23); the last
+// eight are zero on the target side.  FP32 products and sums of the
+// instruction: error 0.9-1.0 of 2^-24 (|x|^2 + |y|^2) rms, against 0.7-0.8 for
+// v_mfma_f32_16x16x4, whose 41 cycles do not overlap with the vector ALU (19
+// cycles here, partly hidden).
+struct Split3 {
+  __bf16 t[3];
+  __device__ __forceinline__ explicit Split3(float v) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      t[i] = (__bf16)v;
+      v -= (float)t[i];
+    }
+  }
+};
+constexpr int kDistGroups = 3;  // eight k-slots each; the fourth group is zero
+
+// the source operand of -2 y' and |y'|^2: group g of this source
+template <int D>
+__device__ __forceinline__ void source_operand(const float (&y)[D], float s2,
+                                               bf16x8 (&out)[kDistGroups]) {
+  const __bf16 zero = (__bf16)0.f, one = (__bf16)1.f;
+  __bf16 a[24];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const Split3 u(d < D ? y[d < D ? d : 0] : 0.f);
+    a[6 * d] = a[6 * d + 1] = a[6 * d + 4] = d < D ? u.t[0] : zero;
+    a[6 * d + 2] = a[6 * d + 3] = d < D ? u.t[1] : zero;
+    a[6 * d + 5] = d < D ? u.t[2] : zero;
+  }
+  const Split3 u(s2);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    a[18 + i] = u.t[i];
+    a[21 + i] = one;
+  }
+#pragma unroll
+  for (int g = 0; g < kDistGroups; ++g)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) out[g][i] = a[8 * g + i];
+}
+
+// the target operand of x' and |x'|^2: the k-slots of lane group lk
+template <int D>
+__device__ __forceinline__ bf16x8 target_operand(const float (&x)[D], float s2, int lk) {
+  const __bf16 zero = (__bf16)0.f, one = (__bf16)1.f;
+  __bf16 b[32];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const Split3 v(d < D ? x[d < D ? d : 0] : 0.f);
+    b[6 * d] = b[6 * d + 2] = b[6 * d + 5] = d < D ? v.t[0] : zero;
+    b[6 * d + 1] = b[6 * d + 3] = d < D ? v.t[1] : zero;
+    b[6 * d + 4] = d < D ? v.t[2] : zero;
+  }
+  const Split3 v(s2);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    b[18 + i] = one;
+    b[21 + i] = v.t[i];
+  }
+#pragma unroll
+  for (int i = 24; i < 32; ++i) b[i] = zero;
+  bf16x8 out;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    out[i] = lk == 0 ? b[i] : (lk == 1 ? b[8 + i] : (lk == 2 ? b[16 + i] : zero));
+  return out;
+}
+
+// One K-step of 32 sources for the row tiles of a wave, distances from the
+// matrix cores: ya, yb are this lane's source operands of the two 16-source
+// halves, xb its target operands, Bh, Bl the right operands.
+template <int KT, int NT, bool ALL>
+__device__ __forceinline__ void gram_step(bf16x8 ya, bf16x8 yb, const u16 *Bh, const u16 *Bl,
+                                          const bf16x8 (&xb)[kRT], const bool (&tile_on)[kRT], int ntl,
+                                          const KernelParams<float> &kp, f32x4 (&acc)[kRT][NT]) {
+  // the entries of every row tile first, then the right operands one column
+  // tile at a time: few registers are live at once
+  bf16x8 ah[kRT], al[kRT];
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    if (!ALL && !tile_on[rt]) continue;
+    const f32x4 g0 = mma_bf16(ya, xb[rt], splat4(0.f));
+    const f32x4 g1 = mma_bf16(yb, xb[rt], splat4(0.f));
+    float ev[8];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      ev[v] = gram_kernel<KT>(g0[v], kp);
+      ev[4 + v] = gram_kernel<KT>(g1[v], kp);
+    }
+    split8(ev, ah[rt], al[rt]);
+  }
+  contract<NT, ALL>(ah, al, Bh, Bl, tile_on, ntl, acc);
+}
+
 // ---------------------------------------------------------------------------
-// Leaf output: one workgroup per target-leaf task, 4 waves, each wave owns row
-// tiles {wave, wave + 4, wave + 8, wave + 12} of the current 256-row pass and
-// 16 NT rhs columns.  Far field: A = V_t^T (rows x q) on FP32 MFMA as in the
-// FP32 form (a small share of the work); near field on BF16 MFMA.
+// Leaf output: one workgroup per target-leaf task, 8 waves, each wave owns row
+// tiles {rg, rg + wrows} of the current 256-row pass and 16 NT rhs columns.
+// Far field: A = V_t^T (rows x q) on FP32 MFMA as in the FP32 form (a small
+// share of the work); near field on BF16 MFMA.
 template <int D, int KT, int NT>
-__global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
+__global__ __launch_bounds__(kThreads, kOcc<NT>) void k_leaf_output_bf16(
     DevTreeView<float> rows, DevTreeView<float> cols, DevPatternView pat,
     InterpParams<float> ip, KernelParams<float> kp, int nrhs, const float *__restrict__ xs,
     const float *__restrict__ tlhs, double *__restrict__ out, int64_t ldo, int natural,
@@ -133,17 +318,18 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
   constexpr int NC = 16 * NT;
   constexpr int NCP = NC + 16;  // padded stride of the staged far moments
   constexpr bool kGram = kGramNear<KT>;
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int P1 = ip.P1, q = ip.q;
   const int qpad = (q + 3) & ~3;
   float *F = reinterpret_cast<float *>(smem_raw);               // [D][P1][kRowsP]
   int *aidx = reinterpret_cast<int *>(F + D * P1 * kRowsP);     // [qpad] packed indices
   float *Un = reinterpret_cast<float *>(aidx + ((qpad + 3) & ~3));  // union region
   float *Ms = Un;                                  // far: [kFarChunk][NCP] moments
-  // near: [D][kChunk] source points, or with kGram [4][kChunk] rows of the
-  // distance MFMA's source operand
+  // near: [D][kChunk] source points, or with kGram [kDistGroups][kChunk]
+  // distance operands of the sources
   float *Ys = Un;
-  u16 *Xh = reinterpret_cast<u16 *>(Ys + 4 * kChunk);  // near: [NC][kChunkP] rhs, hi
+  bf16x8 *Yd = reinterpret_cast<bf16x8 *>(Un);
+  u16 *Xh = reinterpret_cast<u16 *>(Yd + kDistGroups * kChunk);  // near: [NC][kChunkP] rhs, hi
   u16 *Xl = Xh + NC * kChunkP;                         // near: [NC][kChunkP] rhs, lo
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -157,11 +343,11 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
   list_part(n0, n1);
   const int c = rows.leaves[li];
   const int b0 = rows.begin[c], sz = rows.size[c];
-  for (int e = threadIdx.x; e < qpad; e += blockDim.x)
+  for (int e = threadIdx.x; e < qpad; e += kThreads)
     aidx[e] = basis_index<float, D>(e < q ? e : 0, ip);
   for (int pbase = 0; pbase < sz; pbase += kRows) {
     __syncthreads();
-    {
+    if (do_far && threadIdx.x < kRows) {
       const int i = pbase + threadIdx.x;
       if (i < sz) {
 #pragma unroll
@@ -173,35 +359,37 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
           for (int a = 0; a < P1; ++a) F[(d * P1 + a) * kRowsP + threadIdx.x] = 0.f;
       }
     }
+    const int R = (min(kRows, sz - pbase) + 15) / 16;
+    const int kspl = k_split(R), wrows = kWaves / kspl, rg = wave % wrows, sg = wave / wrows;
     float x[kRT][D];
     bool tile_on[kRT];
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) {
-      const int tile_row0 = pbase + (wave + kWaves * rt) * 16;
+      const int tile_row0 = pbase + (rg + wrows * rt) * 16;
       tile_on[rt] = tile_row0 < sz;
       const int i = tile_row0 + lr;
 #pragma unroll
       for (int d = 0; d < D; ++d)
         x[rt][d] = i < sz ? rows.pts[(int64_t)d * rows.npts + b0 + i] : 0.f;
     }
-    // distance MFMA operands of the targets: xb = component lk of [x', 1]
-    // (x' = x - centre of the leaf), xx = |x'|^2
-    float ctr[D], xb[kRT], xx[kRT];
+    // distance operands of the targets, x' = sigma (x - centre of the leaf)
+    float ctr[D];
+    bf16x8 xb[kRT];
     const float sig = gram_sigma<KT>(kp);
 #pragma unroll
     for (int d = 0; d < D; ++d)
       ctr[d] = rows.bbmin[(int64_t)c * D + d] + 0.5f * rows.bbsize[(int64_t)c * D + d];
+    if constexpr (kGram) {
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) {
-      float s2 = 0.f, b = lk == 3 ? 1.f : 0.f;
+      for (int rt = 0; rt < kRT; ++rt) {
+        float s2 = 0.f, v[D];
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        const float v = (x[rt][d] - ctr[d]) * sig;
-        s2 = fmat(v, v, s2);
-        if (d == lk) b = v;
+        for (int d = 0; d < D; ++d) {
+          v[d] = (x[rt][d] - ctr[d]) * sig;
+          s2 = fmat(v[d], v[d], s2);
+        }
+        xb[rt] = target_operand<D>(v, s2, lk);
       }
-      xx[rt] = s2;
-      xb[rt] = b;
     }
     for (int rc = 0; rc < nrhs; rc += NC) {
       f32x4 acc[kRT][NT];
@@ -214,7 +402,7 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
       for (int a0 = 0; do_far && a0 < qpad; a0 += kFarChunk) {
         const int na = min(kFarChunk, qpad - a0);
         __syncthreads();
-        for (int e = threadIdx.x; e < kFarChunk * NC; e += blockDim.x) {
+        for (int e = threadIdx.x; e < kFarChunk * NC; e += kThreads) {
           const int al = e / NC, r = e % NC;
           const int alpha = a0 + al;
           Ms[al * NCP + r] = (alpha < q && rc + r < nrhs)
@@ -222,7 +410,7 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
                                  : 0.f;
         }
         __syncthreads();
-        for (int ks = 0; ks < na; ks += 4) {
+        for (int ks = 4 * sg; ks < na; ks += 4 * kspl) {
           const int al = ks + lk;
           const int pk = aidx[a0 + al];
           float b[NT];
@@ -231,7 +419,7 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
 #pragma unroll
           for (int rt = 0; rt < kRT; ++rt) {
             if (!tile_on[rt]) continue;
-            const int row = (wave + kWaves * rt) * 16 + lr;
+            const int row = (rg + wrows * rt) * 16 + lr;
             float v = F[(0 * P1 + unpack(pk, 0)) * kRowsP + row];
 #pragma unroll
             for (int d = 1; d < D; ++d) v *= F[(d * P1 + unpack(pk, d)) * kRowsP + row];
@@ -243,13 +431,14 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
       }
       // near field: chunks of kChunk sources fetched one chunk ahead into
       // registers, staged as coordinates Ys and the BF16 split of the rhs
-      constexpr int KX = kChunk * NC / 256;          // rhs values per thread
+      // (a thread takes two neighbouring sources of a column: 32-bit stores)
+      constexpr int KX = kChunk * NC / (2 * kThreads);  // rhs pairs per thread
       // coordinates per thread: with kGram thread jj < kChunk loads all D of
       // source jj (its row of the distance operand needs |y'|^2)
-      constexpr int KY = kGram ? D : (D * kChunk + 255) / 256;
-      static_assert(kChunk * NC % 256 == 0, "staging layout");
-      static_assert(kChunk <= 256, "one source per thread in the distance staging");
-      float py[KY], px[KX];
+      constexpr int KY = kGram ? D : (D * kChunk + kThreads - 1) / kThreads;
+      static_assert(kChunk * NC % (2 * kThreads) == 0, "staging layout");
+      static_assert(kChunk <= kThreads, "one source per thread in the distance staging");
+      float py[KY], px[KX][2];
       int nb = n0, j0 = 0, pnj = 0;
       auto fetch = [&]() {
         const int run = min(pat.near_run[nb], n1 - nb);
@@ -259,24 +448,31 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
         if constexpr (kGram) {
           const int jj = threadIdx.x;
 #pragma unroll
-          for (int d = 0; d < D; ++d)  // padding sources sit at the centre
-            py[d] = (jj < kChunk && jj < pnj) ? cols.pts[(int64_t)d * cols.npts + sb + j0 + jj]
-                                              : ctr[d];
+          for (int d = 0; d < D; ++d) {  // padding sources sit at the centre
+            const float *pt = cols.pts + ((int64_t)d * cols.npts + sb + j0);
+            py[d] = (jj < kChunk && jj < pnj) ? pt[(uint32_t)jj] : ctr[d];
+          }
         } else {
 #pragma unroll
           for (int k = 0; k < KY; ++k) {
-            const int e = threadIdx.x + 256 * k;
+            const int e = threadIdx.x + kThreads * k;
             const int d = e / kChunk, jj = e % kChunk;
             py[k] = (e < D * kChunk && jj < pnj)
                         ? cols.pts[(int64_t)d * cols.npts + sb + j0 + jj]
                         : 0.f;
           }
         }
+        // a uniform base and 32-bit offsets: no 64-bit address per load
+        const float *xt = xs + ((int64_t)(sb + j0) * nrhs + rc);
+        const int pr = threadIdx.x % NC, pj = 2 * (threadIdx.x / NC);
 #pragma unroll
         for (int k = 0; k < KX; ++k) {
-          const int e = threadIdx.x + 256 * k;
-          const int jj = e / NC, r = e % NC;
-          px[k] = (jj < pnj && rc + r < nrhs) ? xs[(int64_t)(sb + j0 + jj) * nrhs + rc + r] : 0.f;
+          const int jj = pj + 2 * (kThreads / NC) * k;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            px[k][u] = (jj + u < pnj && rc + pr < nrhs)
+                           ? xt[(uint32_t)((jj + u) * nrhs + pr)]
+                           : 0.f;
         }
         j0 += kChunk;
         if (j0 >= ss) {
@@ -292,195 +488,103 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
         if constexpr (kGram) {
           const int jj = threadIdx.x;
           if (jj < kChunk) {
-            float s2 = 0.f;
+            float s2 = 0.f, v[D];
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-              const float v = (py[d] - ctr[d]) * sig;
-              Ys[d * kChunk + jj] = -2.f * v;
-              s2 = fmat(v, v, s2);
+              v[d] = (py[d] - ctr[d]) * sig;
+              s2 = fmat(v[d], v[d], s2);
+              v[d] *= -2.f;
             }
+            bf16x8 op[kDistGroups];
+            source_operand<D>(v, s2, op);
 #pragma unroll
-            for (int d = D; d < 3; ++d) Ys[d * kChunk + jj] = 0.f;
-            Ys[3 * kChunk + jj] = s2;
+            for (int g = 0; g < kDistGroups; ++g) Yd[g * kChunk + jj] = op[g];
           }
         } else {
 #pragma unroll
           for (int k = 0; k < KY; ++k) {
-            const int e = threadIdx.x + 256 * k;
+            const int e = threadIdx.x + kThreads * k;
             if (e < D * kChunk) Ys[e] = py[k];
           }
         }
 #pragma unroll
         for (int k = 0; k < KX; ++k) {
-          const int e = threadIdx.x + 256 * k;
-          const int jj = e / NC, r = e % NC;
-          const int pos = kGram ? gram_pos(jj) : jj;
-          const uint32_t w = __builtin_bit_cast(uint32_t, px[k]);  // hi | lo << 16
-          Xh[r * kChunkP + pos] = (u16)(w & 0xffffu);
-          Xl[r * kChunkP + pos] = (u16)(w >> 16);
+          const int e = threadIdx.x + kThreads * k;
+          const int jj = 2 * (e / NC), r = e % NC;
+          store_pair(Xh, Xl, r * kChunkP + (kGram ? gram_pos(jj) : jj), px[k][0], px[k][1]);
         }
         __syncthreads();
         more = nb < n1;
         if (more) fetch();
         const int nsteps = (nj + kKB - 1) & ~(kKB - 1);
-        // all four row tiles valid and both column tiles used (the common
-        // case): no branches in a K-step, one basic block for the scheduler
+        // all row tiles valid and all column tiles used (the common case): no
+        // branches in a K-step, one basic block for the scheduler
         bool all_on = ntl == NT;
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt) all_on = all_on && tile_on[rt];
-        auto gram_steps = [&](auto all_t) {
-          constexpr bool ALL = decltype(all_t)::value;
-          for (int ks = 0; ks < nsteps; ks += kKB) {
-            const int j8 = ks + 8 * lk;  // this lane group's eight k-slots
-            // the distances of row tile rt + 1 are issued before the entries
-            // of row tile rt are formed, so the matrix core works under the VALU
-            const float ya = Ys[lk * kChunk + ks + lr], yb = Ys[lk * kChunk + ks + 16 + lr];
-            f32x4 g0 = f32x4{0, 0, 0, 0}, g1 = f32x4{0, 0, 0, 0};
-            if (ALL || tile_on[0]) {
-              g0 = mma_f32(ya, xb[0], splat4(xx[0]));
-              g1 = mma_f32(yb, xb[0], splat4(xx[0]));
-            }
-            // right operands of the K-step, shared by the row tiles
-            bf16x8 bh[NT], bl[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              bh[nt] = load8(Xh + (nt * 16 + lr) * kChunkP + j8);
-              bl[nt] = load8(Xl + (nt * 16 + lr) * kChunkP + j8);
-            }
-#pragma unroll
-            for (int rt = 0; rt < kRT; ++rt) {
-              f32x4 n0 = f32x4{0, 0, 0, 0}, n1 = f32x4{0, 0, 0, 0};
-              if (rt + 1 < kRT && (ALL || tile_on[rt + 1])) {
-                n0 = mma_f32(ya, xb[rt + 1], splat4(xx[rt + 1]));
-                n1 = mma_f32(yb, xb[rt + 1], splat4(xx[rt + 1]));
-              }
-              const f32x4 c0 = g0, c1 = g1;
-              g0 = n0;
-              g1 = n1;
-              if (!ALL && !tile_on[rt]) continue;
-              float ev[8];
-#pragma unroll
-              for (int v = 0; v < 4; ++v) {
-                ev[v] = gram_kernel<KT>(c0[v], kp);
-                ev[4 + v] = gram_kernel<KT>(c1[v], kp);
-              }
-              bf16x8 ah, al;
-              split8(ev, ah, al);
-#pragma unroll
-              for (int nt = 0; nt < NT; ++nt) {
-                if (!ALL && nt >= ntl) continue;
-                acc[rt][nt] = mma_bf16(ah, bh[nt], acc[rt][nt]);
-                acc[rt][nt] = mma_bf16(al, bh[nt], acc[rt][nt]);
-                acc[rt][nt] = mma_bf16(ah, bl[nt], acc[rt][nt]);
-              }
-            }
-          }
-        };
         if constexpr (kGram) {
-          if (all_on)
-            gram_steps(std::true_type{});
-          else
-            gram_steps(std::false_type{});
-        }
-        // kernels with a cusp at r = 0: differences on the VALU
-        auto direct_steps = [&](auto all_t) {
-          constexpr bool ALL = decltype(all_t)::value;
-          for (int ks = 0; ks < nsteps; ks += kKB) {
-            const int j8 = ks + 8 * lk;  // this lane group's eight sources
-            float y[D][8];
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-#pragma unroll
-              for (int i = 0; i < 8; ++i) y[d][i] = Ys[d * kChunk + j8 + i];
-            bf16x8 bh[NT], bl[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              bh[nt] = load8(Xh + (nt * 16 + lr) * kChunkP + j8);
-              bl[nt] = load8(Xl + (nt * 16 + lr) * kChunkP + j8);
+          const int gl = min(lk, kDistGroups - 1);  // group 3: zero in xb
+          auto steps = [&](auto all_t) {
+            for (int ks = kKB * sg; ks < nsteps; ks += kKB * kspl) {
+              const int off = lr * kChunkP + ks + 8 * lk;  // this lane group's eight k-slots
+              gram_step<KT, NT, decltype(all_t)::value>(
+                  Yd[gl * kChunk + ks + lr], Yd[gl * kChunk + ks + 16 + lr], Xh + off, Xl + off,
+                  xb, tile_on, ntl, kp, acc);
             }
+          };
+          if (all_on)
+            steps(std::true_type{});
+          else
+            steps(std::false_type{});
+        } else {
+          // kernels with a cusp at r = 0: differences on the VALU
+          auto steps = [&](auto all_t) {
+            constexpr bool ALL = decltype(all_t)::value;
+            for (int ks = kKB * sg; ks < nsteps; ks += kKB * kspl) {
+              const int j8 = ks + 8 * lk;  // this lane group's eight sources
+              float y[D][8];
 #pragma unroll
-            for (int rt = 0; rt < kRT; ++rt) {
-              if (!ALL && !tile_on[rt]) continue;
-              float ev[8];
+              for (int d = 0; d < D; ++d)
 #pragma unroll
-              for (int i = 0; i < 8; ++i) {
-                float r2 = 0.f;
+                for (int i = 0; i < 8; ++i) y[d][i] = Ys[d * kChunk + j8 + i];
+              bf16x8 ah[kRT], al[kRT];
 #pragma unroll
-                for (int d = 0; d < D; ++d) {
-                  const float dd = x[rt][d] - y[d][i];
-                  r2 = fmat(dd, dd, r2);
+              for (int rt = 0; rt < kRT; ++rt) {
+                if (!ALL && !tile_on[rt]) continue;
+                float ev[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                  float r2 = 0.f;
+#pragma unroll
+                  for (int d = 0; d < D; ++d) {
+                    const float dd = x[rt][d] - y[d][i];
+                    r2 = fmat(dd, dd, r2);
+                  }
+                  ev[i] = kernel_r2<KT, float>(r2, kp);
                 }
-                ev[i] = kernel_r2<KT, float>(r2, kp);
+                split8(ev, ah[rt], al[rt]);
               }
-              bf16x8 ah, al;
-              split8(ev, ah, al);
-#pragma unroll
-              for (int nt = 0; nt < NT; ++nt) {
-                if (!ALL && nt >= ntl) continue;
-                acc[rt][nt] = mma_bf16(ah, bh[nt], acc[rt][nt]);
-                acc[rt][nt] = mma_bf16(al, bh[nt], acc[rt][nt]);
-                acc[rt][nt] = mma_bf16(ah, bl[nt], acc[rt][nt]);
-              }
+              const int off = lr * kChunkP + j8;
+              contract<NT, ALL>(ah, al, Xh + off, Xl + off, tile_on, ntl, acc);
             }
-          }
-        };
-        // 32 columns: right operands loaded once per K-step for the four row
-        // tiles, and the branch-free K-step when all tiles are valid (13 %
-        // faster for EXPONENTIAL at 32 rhs); 16 columns and the run-time
-        // kernel switch (which would spill) keep the per-tile loads (5 %
-        // faster at 16 columns)
-        constexpr bool kHoist = !kGram && NT == 2 && KT >= 0;
-        if constexpr (kHoist) {
-          if (all_on)
-            direct_steps(std::true_type{});
+          };
+          if (all_on && KT >= 0)
+            steps(std::true_type{});
           else
-            direct_steps(std::false_type{});
-        }
-        for (int ks = 0; !kGram && !kHoist && ks < nsteps; ks += kKB) {
-          const int j8 = ks + 8 * lk;  // this lane group's eight sources
-          float y[D][8];
-#pragma unroll
-          for (int d = 0; d < D; ++d)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) y[d][i] = Ys[d * kChunk + j8 + i];
-#pragma unroll
-          for (int rt = 0; rt < kRT; ++rt) {
-            if (!tile_on[rt]) continue;
-            float ev[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              float r2 = 0.f;
-#pragma unroll
-              for (int d = 0; d < D; ++d) {
-                const float dd = x[rt][d] - y[d][i];
-                r2 = fmat(dd, dd, r2);
-              }
-              ev[i] = kernel_r2<KT, float>(r2, kp);
-            }
-            bf16x8 ah, al;
-            split8(ev, ah, al);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              if (nt >= ntl) continue;
-              const bf16x8 bh = load8(Xh + (nt * 16 + lr) * kChunkP + j8);
-              const bf16x8 bl = load8(Xl + (nt * 16 + lr) * kChunkP + j8);
-              acc[rt][nt] = mma_bf16(ah, bh, acc[rt][nt]);
-              acc[rt][nt] = mma_bf16(al, bh, acc[rt][nt]);
-              acc[rt][nt] = mma_bf16(ah, bl, acc[rt][nt]);
-            }
-          }
+            steps(std::false_type{});
         }
       }
-      // store: C row 4 lk + v of tile (wave + 4 rt), column lr of rhs tile nt
+      if (kspl > 1) add_groups<NT>(acc, Un, kspl, wrows, rg, sg, tile_on, lr, lk);
+      // store: C row 4 lk + v of tile (rg + wrows rt), column lr of rhs tile nt
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
-        if (!tile_on[rt]) continue;
+        if (!tile_on[rt] || sg != 0) continue;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const int col = rc + nt * 16 + lr;
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int i = pbase + (wave + kWaves * rt) * 16 + 4 * lk + v;
+            const int i = pbase + (rg + wrows * rt) * 16 + 4 * lk + v;
             if (i < sz && col < nrhs) {
               if (gridDim.y > 1) {
                 part[((int64_t)blockIdx.y * rows.npts + b0 + i) * nrhs + col] = acc[rt][nt][v];
@@ -506,26 +610,24 @@ __global__ __launch_bounds__(256, 2) void k_leaf_output_bf16(
 // K-steps of 32, N = 16 NT rhs columns.  A chunk of kChunk rows holds
 // G = kChunk / qpad whole sources when that is 2 or more, else kChunk nodes of
 // one source; rows past a source's q nodes or past the list carry zero
-// moments.  For q <= 64 every wave takes all row tiles and every fourth
-// K-step, and the partial sums are added in LDS in wave order.
+// moments.  With fewer than 9 row tiles the waves split the K-steps too.
 template <int D, int KT, int NT>
-__global__ __launch_bounds__(256, 2) void k_coupling_bf16(
+__global__ __launch_bounds__(kThreads, kOcc<NT>) void k_coupling_bf16(
     DevTreeView<float> rows, DevTreeView<float> cols, DevPatternView pat,
     InterpParams<float> ip, KernelParams<float> kp, int nrhs, const float *__restrict__ mom,
     float *__restrict__ tlhs, float *__restrict__ part) {
   constexpr int NC = 16 * NT;
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int q = ip.q;
   const int qpad = (q + 3) & ~3;
   float *U = reinterpret_cast<float *>(smem_raw);  // [D][qpad] unit node coordinates
-  // [4][kChunk] rows of the distance MFMA's source operand: -2 y' (k-slots
-  // 0..D-1), |y'|^2 (k-slot 3), y' = node - centre of the target cluster.
-  // Far blocks are separated (dist >= radius / eta), so the cancellation in
-  // |y'|^2 - 2 x'.y' + |x'|^2 stays at the rounding of the direct form.
-  float *Yc = U + D * qpad;
-  u16 *Mh = reinterpret_cast<u16 *>(Yc + 4 * kChunk);  // [NC][kChunkP] moments, hi
+  // [kDistGroups][kChunk] distance operands of the sources, y' = node - centre
+  // of the target cluster.  Far blocks are separated (dist >= radius / eta), so
+  // the cancellation in |y'|^2 - 2 x'.y' + |x'|^2 stays near the rounding of the
+  // direct form.
+  bf16x8 *Yd = reinterpret_cast<bf16x8 *>(U + D * qpad);  // qpad floats: 16-byte aligned
+  u16 *Mh = reinterpret_cast<u16 *>(Yd + kDistGroups * kChunk);  // [NC][kChunkP] moments, hi
   u16 *Ml = Mh + NC * kChunkP;                         // [NC][kChunkP] moments, lo
-  float *Red = reinterpret_cast<float *>(Ml + NC * kChunkP);  // [2 kRT 16][NC] K-split sums
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lk = lane >> 4;
@@ -537,18 +639,18 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
   // sums of this part: its slab, or the coupling sums themselves
   float *dst_all = gridDim.y > 1 ? part + (int64_t)blockIdx.y * rows.ncl * ip.q * nrhs : tlhs;
   const bool split = (pat.far_task[4 * task + 3] & kTaskSplit) != 0;
-  const int R = (q + 15) / 16;
-  const int kspl = R <= kRT ? 4 : (R <= 2 * kRT ? 2 : 1);
-  const int wrows = kWaves / kspl, rg = wave % wrows, sg = wave / wrows;
-  const int ks0 = kKB * sg, kstep = kKB * kspl;
+  const int kspl = k_split((q + 15) / 16), wrows = kWaves / kspl, rg = wave % wrows,
+            sg = wave / wrows;
   const int G = max(1, kChunk / qpad);
   const float rqpad = 1.0f / (float)qpad;  // bl / qpad = floor((bl + 0.5) / qpad), bl < 256
-  for (int e = threadIdx.x; e < D * qpad; e += blockDim.x) {
+  for (int e = threadIdx.x; e < D * qpad; e += kThreads) {
     const int d = e / qpad, b = e - d * qpad, bb = b < q ? b : 0;
     U[e] = ip.td ? ip.unodes[d * q + bb] : ip.xi[unpack(basis_index<float, D>(bb, ip), d)];
   }
-  float ctr[D], xb[kRT], xx[kRT];
+  float ctr[D];
+  bf16x8 xb[kRT];  // distance operands of the target nodes
   const float sig = gram_sigma<KT>(kp);
+  const int gl = min(lk, kDistGroups - 1);  // group 3: zero in xb
   bool tile_on[kRT];
 #pragma unroll
   for (int d = 0; d < D; ++d) ctr[d] = rows.bbmin[t * D + d] + 0.5f * rows.bbsize[t * D + d];
@@ -558,16 +660,14 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
     tile_on[rt] = tile_row0 < q;
     const int row = tile_row0 + lr < q ? tile_row0 + lr : 0;
     const int pk = basis_index<float, D>(row, ip);
-    float s2 = 0.f, b = lk == 3 ? 1.f : 0.f;
+    float s2 = 0.f, v[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const float u = ip.td ? ip.unodes[d * q + row] : ip.xi[unpack(pk, d)];
-      const float v = (u * rows.bbsize[t * D + d] + rows.bbmin[t * D + d] - ctr[d]) * sig;
-      s2 = fmat(v, v, s2);
-      if (d == lk) b = v;
+      v[d] = (u * rows.bbsize[t * D + d] + rows.bbmin[t * D + d] - ctr[d]) * sig;
+      s2 = fmat(v[d], v[d], s2);
     }
-    xx[rt] = s2;  // distance MFMA operands of the target nodes
-    xb[rt] = b;
+    xb[rt] = target_operand<D>(v, s2, lk);
   }
   __syncthreads();  // U
   // source slot and node of row bl of a chunk of nsrc whole sources (G >= 2);
@@ -588,64 +688,20 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
     bool all_on = ntl == NT;
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) all_on = all_on && tile_on[rt];
-    // all four row tiles valid and both column tiles used (the common case):
-    // no branches in a K-step, one basic block for the scheduler
+    // all row tiles valid and all column tiles used (the common case): no
+    // branches in a K-step, one basic block for the scheduler
     auto chunk_steps = [&](int nrows, auto all_t) {
-      constexpr bool ALL = decltype(all_t)::value;
-      for (int ks = ks0; ks < nrows; ks += kstep) {
-        const int j8 = ks + 8 * lk;  // this lane group's eight k-slots (gram_pos order)
-        const float ya = Yc[lk * kChunk + ks + lr], yb = Yc[lk * kChunk + ks + 16 + lr];
-        // distances of row tile rt + 1 issued before the entries of rt
-        f32x4 g0 = f32x4{0, 0, 0, 0}, g1 = f32x4{0, 0, 0, 0};
-        if (ALL || tile_on[0]) {
-          g0 = mma_f32(ya, xb[0], splat4(xx[0]));
-          g1 = mma_f32(yb, xb[0], splat4(xx[0]));
-        }
-        bf16x8 bh[NT], bl[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          bh[nt] = load8(Mh + (nt * 16 + lr) * kChunkP + j8);
-          bl[nt] = load8(Ml + (nt * 16 + lr) * kChunkP + j8);
-        }
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          f32x4 n0 = f32x4{0, 0, 0, 0}, n1 = f32x4{0, 0, 0, 0};
-          if (rt + 1 < kRT && (ALL || tile_on[rt + 1])) {
-            n0 = mma_f32(ya, xb[rt + 1], splat4(xx[rt + 1]));
-            n1 = mma_f32(yb, xb[rt + 1], splat4(xx[rt + 1]));
-          }
-          const f32x4 c0 = g0, c1 = g1;
-          g0 = n0;
-          g1 = n1;
-          if (!ALL && !tile_on[rt]) continue;
-          float ev[8];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            ev[v] = gram_kernel<KT>(c0[v], kp);
-            ev[4 + v] = gram_kernel<KT>(c1[v], kp);
-          }
-          bf16x8 ah, al;
-          split8(ev, ah, al);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) {
-            if (!ALL && nt >= ntl) continue;
-            acc[rt][nt] = mma_bf16(ah, bh[nt], acc[rt][nt]);
-            acc[rt][nt] = mma_bf16(al, bh[nt], acc[rt][nt]);
-            acc[rt][nt] = mma_bf16(ah, bl[nt], acc[rt][nt]);
-          }
-        }
+      for (int ks = kKB * sg; ks < nrows; ks += kKB * kspl) {
+        const int off = lr * kChunkP + ks + 8 * lk;  // eight k-slots (gram_pos order)
+        gram_step<KT, NT, decltype(all_t)::value>(
+            Yd[gl * kChunk + ks + lr], Yd[gl * kChunk + ks + 16 + lr], Mh + off, Ml + off, xb,
+            tile_on, ntl, kp, acc);
       }
     };
-    auto compute_chunk = [&](int nrows) {
-      if (all_on)
-        chunk_steps(nrows, std::true_type{});
-      else
-        chunk_steps(nrows, std::false_type{});
-    };
-    constexpr int KM = kChunk * NC / 256;  // staged moments per thread
-    static_assert(kChunk * NC % 256 == 0, "staging layout");
-    static_assert(kChunk <= 256, "one node per thread in the distance staging");
-    float py[D], pm[KM];  // py: the D coordinates of node threadIdx.x of the chunk
+    constexpr int KM = kChunk * NC / (2 * kThreads);  // staged moment pairs per thread
+    static_assert(kChunk * NC % (2 * kThreads) == 0, "staging layout");
+    static_assert(kChunk <= kThreads, "one node per thread in the distance staging");
+    float py[D], pm[KM][2];  // py: the D coordinates of node threadIdx.x of the chunk
     int f = f0, nbe = 0;
     int pn = 0;
     auto fetch = [&]() {
@@ -664,16 +720,23 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
         }
 #pragma unroll
         for (int k = 0; k < KM; ++k) {
-          const int e = threadIdx.x + 256 * k;
-          const int bl = e / NC, r = e % NC;
-          int slot, node;
+          const int e = threadIdx.x + kThreads * k;
+          const int bl = 2 * (e / NC), r = e % NC;
+          int slot, node;  // of both rows of the pair: qpad is even
           chunk_row(bl, nsrc, slot, node);
-          const float *ms = mom + (int64_t)pat.far_src[f + slot] * q * nrhs;
-          pm[k] = (node >= 0 && rc + r < nrhs) ? ms[node * nrhs + rc + r] : 0.f;
+          // from 32 columns on a wave's rows (4 or 2) lie in one source: qpad
+          // is a multiple of 4
+          if constexpr (NT >= 2) slot = __builtin_amdgcn_readfirstlane(slot);
+          const float *ms = mom + ((int64_t)pat.far_src[f + slot] * q * nrhs + rc);
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            pm[k][u] = (node >= 0 && node + u < q && rc + r < nrhs)
+                           ? ms[(uint32_t)((node + u) * nrhs + r)]
+                           : 0.f;
         }
       } else {
         const int s = pat.far_src[f];
-        const float *ms = mom + (int64_t)s * q * nrhs;
+        const float *ms = mom + ((int64_t)s * q * nrhs + rc);
         if (threadIdx.x < kChunk) {
           const int node = be + (int)threadIdx.x < q ? be + (int)threadIdx.x : 0;
 #pragma unroll
@@ -682,10 +745,15 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
         }
 #pragma unroll
         for (int k = 0; k < KM; ++k) {
-          const int e = threadIdx.x + 256 * k;
-          const int bl = e / NC, r = e % NC;
-          const int node = be + bl;
-          pm[k] = (bl < pn && node < q && rc + r < nrhs) ? ms[node * nrhs + rc + r] : 0.f;
+          const int e = threadIdx.x + kThreads * k;
+          const int bl = 2 * (e / NC), r = e % NC;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int node = be + bl + u;
+            pm[k][u] = (bl + u < pn && node < q && rc + r < nrhs)
+                           ? ms[(uint32_t)(node * nrhs + r)]
+                           : 0.f;
+          }
         }
       }
       if (G > 1) {
@@ -701,84 +769,56 @@ __global__ __launch_bounds__(256, 2) void k_coupling_bf16(
     auto stage = [&]() {
       if (threadIdx.x < kChunk) {
         const int bl = threadIdx.x;
-        float s2 = 0.f;
+        float s2 = 0.f, v[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-          const float v = (py[d] - ctr[d]) * sig;
-          Yc[d * kChunk + bl] = -2.f * v;
-          s2 = fmat(v, v, s2);
+          v[d] = (py[d] - ctr[d]) * sig;
+          s2 = fmat(v[d], v[d], s2);
+          v[d] *= -2.f;
         }
+        bf16x8 op[kDistGroups];
+        source_operand<D>(v, s2, op);
 #pragma unroll
-        for (int d = D; d < 3; ++d) Yc[d * kChunk + bl] = 0.f;
-        Yc[3 * kChunk + bl] = s2;
+        for (int g = 0; g < kDistGroups; ++g) Yd[g * kChunk + bl] = op[g];
       }
 #pragma unroll
       for (int k = 0; k < KM; ++k) {
-        const int e = threadIdx.x + 256 * k;
-        const int bl = e / NC, r = e % NC;
-        const uint32_t w = __builtin_bit_cast(uint32_t, pm[k]);  // hi | lo << 16
-        Mh[r * kChunkP + gram_pos(bl)] = (u16)(w & 0xffffu);
-        Ml[r * kChunkP + gram_pos(bl)] = (u16)(w >> 16);
+        const int e = threadIdx.x + kThreads * k;
+        const int bl = 2 * (e / NC), r = e % NC;
+        store_pair(Mh, Ml, r * kChunkP + gram_pos(bl), pm[k][0], pm[k][1]);
       }
     };
-    // no register lookahead of the next chunk here: its 18 values per thread
-    // push the 32-column form past 256 VGPRs (spills)
-    while (f < f1) {
-      fetch();
+    bool more = f < f1;
+    if (more) fetch();
+    while (more) {
       const int nrows = (pn + kKB - 1) & ~(kKB - 1);
       __syncthreads();
       stage();
       __syncthreads();
-      compute_chunk(nrows);
+      more = f < f1;
+      if (more) fetch();  // the next chunk's loads overlap this one's K-steps
+      if (all_on)
+        chunk_steps(nrows, std::true_type{});
+      else
+        chunk_steps(nrows, std::false_type{});
     }
-    if (kspl > 1) {
-      for (int g = 0; g < kspl; ++g) {
-        if (sg == g) {
+    if (kspl > 1)
+      add_groups<NT>(acc, reinterpret_cast<float *>(Mh), kspl, wrows, rg, sg, tile_on, lr, lk);
 #pragma unroll
-          for (int rt = 0; rt < kRT; ++rt) {
-            if (!tile_on[rt]) continue;
+    for (int rt = 0; rt < kRT; ++rt) {
+      if (!tile_on[rt] || sg != 0) continue;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              if (nt >= ntl) continue;
+      for (int nt = 0; nt < NT; ++nt) {
+        const int col = rc + nt * 16 + lr;
 #pragma unroll
-              for (int v = 0; v < 4; ++v) {
-                const int alpha = (rg + wrows * rt) * 16 + 4 * lk + v;
-                float *dst = Red + alpha * NC + nt * 16 + lr;
-                *dst = (g == 0 ? 0.f : *dst) + acc[rt][nt][v];
-              }
-            }
-          }
-        }
-        __syncthreads();
-      }
-      for (int e = threadIdx.x; e < q * NC; e += blockDim.x) {
-        const int alpha = e / NC, cc = e - alpha * NC;
-        if (cc < 16 * ntl && rc + cc < nrhs) {
-          float *p = dst_all + ((int64_t)t * q + alpha) * nrhs + rc + cc;
-          if (split)
-            atomic_accumulate(p, Red[e]);
-          else
-            *p = Red[e];
-        }
-      }
-      __syncthreads();
-    } else {
-#pragma unroll
-      for (int rt = 0; rt < kRT; ++rt) {
-        if (!tile_on[rt]) continue;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const int col = rc + nt * 16 + lr;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int alpha = (rg + wrows * rt) * 16 + 4 * lk + v;
-            if (alpha < q && col < nrhs) {
-              float *p = dst_all + ((int64_t)t * q + alpha) * nrhs + col;
-              if (split)
-                atomic_accumulate(p, acc[rt][nt][v]);
-              else
-                *p = acc[rt][nt][v];
-            }
+        for (int v = 0; v < 4; ++v) {
+          const int alpha = (rg + wrows * rt) * 16 + 4 * lk + v;
+          if (alpha < q && col < nrhs) {
+            float *p = dst_all + ((int64_t)t * q + alpha) * nrhs + col;
+            if (split)
+              atomic_accumulate(p, acc[rt][nt][v]);
+            else
+              *p = acc[rt][nt][v];
           }
         }
       }
@@ -791,7 +831,8 @@ size_t leaf_output_bf16_lds(int D, int P1, int q) {
   constexpr int NC = 16 * NT;
   const int qpad = (q + 3) & ~3;
   const size_t far = (size_t)kFarChunk * (NC + 16) * sizeof(float);
-  const size_t near = (size_t)4 * kChunk * sizeof(float) + (size_t)2 * NC * kChunkP * sizeof(u16);
+  const size_t near =
+      (size_t)kDistGroups * kChunk * 16 + (size_t)2 * NC * kChunkP * sizeof(u16);
   return (size_t)D * P1 * kRowsP * sizeof(float) + (size_t)((qpad + 3) & ~3) * sizeof(int) +
          (far > near ? far : near);
 }
@@ -800,9 +841,8 @@ template <int NT>
 size_t coupling_bf16_lds(int D, int q) {
   constexpr int NC = 16 * NT;
   const int qpad = (q + 3) & ~3;
-  const size_t red = q <= 2 * kRT * 16 ? (size_t)2 * kRT * 16 * NC * sizeof(float) : 0;
-  return (size_t)D * qpad * sizeof(float) + (size_t)4 * kChunk * sizeof(float) +
-         (size_t)2 * NC * kChunkP * sizeof(u16) + red;
+  return (size_t)D * qpad * sizeof(float) + (size_t)kDistGroups * kChunk * 16 +
+         (size_t)2 * NC * kChunkP * sizeof(u16);
 }
 
 template <int D, int NT>
@@ -814,11 +854,11 @@ hipError_t launch_bf16_nt(bool output, const MfmaLaunch<float> &a) {
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
 #define FMCA_BF16_LAUNCH(K)                                                                   \
   if (output)                                                                                 \
-    hipLaunchKernelGGL((k_leaf_output_bf16<D, K, NT>), grid, dim3(256), lds_out, a.stream,    \
+    hipLaunchKernelGGL((k_leaf_output_bf16<D, K, NT>), grid, dim3(kThreads), lds_out, a.stream,    \
                        a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs, a.tlhs, a.out, a.ldo, \
                        a.natural ? 1 : 0, slabs);                                             \
   else                                                                                        \
-    hipLaunchKernelGGL((k_coupling_bf16<D, K, NT>), grid, dim3(256), lds_cpl, a.stream,       \
+    hipLaunchKernelGGL((k_coupling_bf16<D, K, NT>), grid, dim3(kThreads), lds_cpl, a.stream,       \
                        a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs, slabs)
   switch (a.kp.kt) {
     case KT_EXPONENTIAL:
@@ -843,9 +883,26 @@ hipError_t launch_bf16_nt(bool output, const MfmaLaunch<float> &a) {
                                  a.ldo, a.natural, a.stream);
 }
 
+// Columns per pass: 16, 32, or 64 for more than 32 columns where the staging
+// fits: one evaluation of the entries for 64 columns (n = 1e6: 12.9 ms in the
+// leaf output against 2 x 7.7 ms).
+inline int bf16_nt(bool output, int D, int P1, int q, int nrhs) {
+  if (nrhs <= 16) return 1;
+  if (nrhs > 32 && (output ? leaf_output_bf16_lds<4>(D, P1, q) : coupling_bf16_lds<4>(D, q)) <=
+                       64 * 1024)
+    return 4;
+  return 2;
+}
+
 template <int D>
 hipError_t launch_bf16_d(bool output, const MfmaLaunch<float> &a) {
-  return a.nrhs <= 16 ? launch_bf16_nt<D, 1>(output, a) : launch_bf16_nt<D, 2>(output, a);
+  switch (bf16_nt(output, D, a.ip.P1, a.ip.q, a.nrhs)) {
+    case 1:
+      return launch_bf16_nt<D, 1>(output, a);
+    case 2:
+      return launch_bf16_nt<D, 2>(output, a);
+  }
+  return launch_bf16_nt<D, 4>(output, a);
 }
 
 }  // namespace
@@ -858,7 +915,7 @@ bool bf16_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vma
   if (output)
     return (nt == 1 ? leaf_output_bf16_lds<1>(D, P1, q) : leaf_output_bf16_lds<2>(D, P1, q)) <=
            limit;
-  if (q > kWaves * kRT * 16) return false;
+  if (q > kRows) return false;
   return (nt == 1 ? coupling_bf16_lds<1>(D, q) : coupling_bf16_lds<2>(D, q)) <= limit;
 }
 
