@@ -456,7 +456,19 @@ hipError_t dispatch_nr(bool output, const DevTreeView<T> &rows, const DevTreeVie
     if (kp.split_bf16 && bf16_supported(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask))
       return launch_bf16(output, a, buf.xs, buf.mom);
   }
-  if (!kp.geodesic && mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td))
+  // FP64 with at most 8 columns of one variant: an FP64 MFMA fills 16 columns
+  // and takes as long as the vector FMAs of 16 (neither overlaps the other), so
+  // the vector forms win while one source's nodes fill few passes of their
+  // workgroup.  8 columns, MFMA / vector (ms, leaf output and coupling): 2-D
+  // n = 2e5 degree 5 (q = 36) 0.54 + 0.74 / 0.33 + 0.48, 3-D n = 2e5 degree 3
+  // (q = 64) EXPONENTIAL 7.18 + 2.03 / 2.43 + 1.33; past q = 64 the coupling
+  // turns: degree 4 (q = 125) GAUSSIAN 4.82 + 1.94 / 4.48 + 3.56.  16 columns
+  // (q = 36): 0.54 + 0.75 / 0.53 + 0.89.  The bounds keep a full 8-column tile
+  // inside the vector forms' LDS.
+  const bool few = sizeof(T) == 8 && nrhs <= 8 && (kp.vmask & (kp.vmask - 1)) == 0 &&
+                   ip.q <= 64 && D * ip.P1 <= 20;
+  if (!few && !kp.geodesic &&
+      mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td))
     return launch_mfma<T>(output, a);
   return launch_valu<T>(output, a);
 }

@@ -45,11 +45,14 @@ constexpr int kAlphaTile = 128;  // far-field coefficients staged per step
 // Rows per thread, while the accumulators are few.  More rows share a source's
 // LDS reads and, in the coupling, the setup of a line; one row leaves the FP64
 // leaf output more waves.  Measured (us): FP64 leaf output n = 1e4, 1 rhs: 72
-// with one row, 79 with two; FP32 leaf output n = 123457, 5 rhs: 848 / 857
-// with two / one, 892 with four; FP32 coupling there: 547 with four, 608 with two.
-template <typename T, int NR, bool OUTPUT>
+// with one row, 79 with two; FP64 leaf output, 8 rhs, n = 2e5: 3-D degree 3
+// EXPONENTIAL 3600 / 2433 with one / two rows, degree 4 MATERN32 6497 / 5863,
+// but 2-D degree 5 333 / 362 (small leaves); FP32 leaf output n = 123457,
+// 5 rhs: 848 / 857 with two / one, 892 with four; FP32 coupling there: 547
+// with four, 608 with two.
+template <typename T, int D, int NR, bool OUTPUT>
 constexpr int kRowsPerThread = NR > 8 ? 1
-                               : OUTPUT ? (sizeof(T) == 8 ? 1 : 2)
+                               : OUTPUT ? (sizeof(T) == 8 && !(NR == 8 && D == 3) ? 1 : 2)
                                         : (sizeof(T) == 4 && NR <= 6 ? 4 : 2);
 
 // elements of a staged source (D coordinates, NR values), a multiple of 16 bytes
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(256) void k_leaf_output(DevTreeView<T> rows, DevTre
                                                      const T *__restrict__ tlhs,
                                                      double *__restrict__ out, int64_t ldo,
                                                      int natural, T *__restrict__ part) {
-  constexpr int RPT = kRowsPerThread<T, NR, true>;
+  constexpr int RPT = kRowsPerThread<T, D, NR, true>;
   constexpr int RS = kRecord<T, D, NR>;
   constexpr bool TAB = !GEO && kTableEntry<KT, T>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(256) void k_coupling(DevTreeView<T> rows, DevTreeVi
                                                   KernelParams<T> kp, int nrhs, int G,
                                                   const T *__restrict__ mom,
                                                   T *__restrict__ tlhs, T *__restrict__ part) {
-  constexpr int RPT = kRowsPerThread<T, NR, false>;
+  constexpr int RPT = kRowsPerThread<T, D, NR, false>;
   constexpr bool TAB = !GEO && kTableEntry<KT, T>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double tab[TAB ? 64 : 1];
@@ -465,7 +468,7 @@ size_t output_lds(int P1, int nt) {
   const size_t far = ((size_t)D * P1 * nt + (size_t)kAlphaTile * NR) * sizeof(T) +
                      kAlphaTile * sizeof(int);
   const size_t near = (size_t)nt * kRecord<T, D, NR> * sizeof(T);
-  const size_t red = (size_t)nt * kRowsPerThread<T, NR, true> * sizeof(T);
+  const size_t red = (size_t)nt * kRowsPerThread<T, D, NR, true> * sizeof(T);
   return std::max(far, std::max(near, red));
 }
 
@@ -475,7 +478,7 @@ template <typename T, int D, int NR>
 size_t coupling_lds(int P1, int q, bool single, int G, int nt) {
   const int p = single ? 1 : P1, nl = q / p;
   const size_t tile = (size_t)G * (q * NR + nl * D + p) * sizeof(T);
-  const size_t red = (size_t)nt * kRowsPerThread<T, NR, false> * sizeof(T);
+  const size_t red = (size_t)nt * kRowsPerThread<T, D, NR, false> * sizeof(T);
   return coupling_head<T, D>(p, nl, G) + std::max(tile, red);
 }
 
@@ -511,7 +514,7 @@ hipError_t valu_launch(bool output, const ValuLaunch<T> &a) {
   if (output) {
     if (a.pat.nnear_order <= 0) return hipSuccess;
     const int nt = valu_threads(a.rows.nleaves > 0 ? (double)a.rows.npts / a.rows.nleaves : 1,
-                                kRowsPerThread<T, NR, true>);
+                                kRowsPerThread<T, D, NR, true>);
     parts = phase_parts(a.pat.nnear_order, a.pat.nnear_split, nt / 64, a.pat.near_per_task, nt,
                         a.rows.npts * a.nrhs, a.part_cap);
     if (parts > 1 && !(slabs = a.part(parts * a.rows.npts * a.nrhs))) parts = 1;
@@ -521,7 +524,7 @@ hipError_t valu_launch(bool output, const ValuLaunch<T> &a) {
                        a.kp, a.nrhs, a.xs, a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);
   } else {
     if (a.pat.nfar_order <= 0) return hipSuccess;
-    const int nt = valu_threads(q, kRowsPerThread<T, NR, false>);
+    const int nt = valu_threads(q, kRowsPerThread<T, D, NR, false>);
     const bool single = GEO || a.ip.td;
     // whole sources per tile, up to 512 nodes of one column (fewer of more)
     const int want = NR == 1 ? 512 : (NR <= 4 ? 256 : 128);

@@ -45,7 +45,7 @@ def test_few_columns_match_the_oracle(dim, n, deg, eta):
 
 
 @pytest.mark.parametrize("interp", ["tensor_product", "total_degree"])
-@pytest.mark.parametrize("nrhs", [1, 6, 16, 40])
+@pytest.mark.parametrize("nrhs", [1, 6, 8, 16, 40])
 def test_parts_on_rectangular_and_transposed_sets(interp, nrhs):
     import torch
     import fmca_amd
