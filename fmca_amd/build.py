@@ -36,7 +36,7 @@ HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", f"-I{INCLUDE}", f"-I{CSRC}"
               "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]
 
 SOURCES_HIP = ["kernels.hip", "kernels_valu_f32.hip", "kernels_valu_f64.hip",
-               "kernels_mfma.hip", "kernels_bf16.hip", "kernels_grad.hip",
+               "kernels_mfma_f32.hip", "kernels_mfma_f64.hip", "kernels_bf16.hip", "kernels_grad.hip",
                "blas1.hip", "block_krylov.hip", "tree_device.hip", "assembled.hip", "pattern_device.hip",
                "samplets.hip"]
 SOURCES_CPP = ["plan.cpp", "actor.cpp", "projector.cpp", "samplets.cpp", "samplets_api.cpp"]

@@ -331,7 +331,7 @@ constexpr int kMfmaMinRhs = 8;
 template <typename T>
 bool mfma_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vmask, int td);
 
-// Leaf moments of the FP32 forms on the matrix cores (kernels_mfma.hip):
+// Leaf moments of the FP32 forms on the matrix cores (kernels_mfma_f32.hip):
 // q <= 128 and >= kMfmaMinRhs rhs where the LDS staging fits.
 bool upward_leaf_mfma_supported(int D, int P1, int q, int nrhs);
 hipError_t launch_upward_leaf_mfma(const DevTreeView<float> &tr, const InterpParams<float> &ip,

@@ -309,8 +309,9 @@ __device__ __forceinline__ T kernel_r2(T r2, const KernelParams<T> &kp) {
 // together, the three share the distance, square root and exponential.  A
 // variant outside kp.vmask (uniform over the launch) is not needed by any
 // column tile: where it costs extra work (a division, a separate evaluation)
-// it is skipped and left 0.
-template <int KT, typename T>
+// it is skipped and left 0.  PHI: phi is in the mask (1), is not (0), or the
+// mask tells (-1).
+template <int KT, typename T, int PHI = -1>
 __device__ __forceinline__ void kernel_r2_all(T r2, const KernelParams<T> &kp, const double *tab,
                                               T ev[3]) {
   using M = Math<T>;
@@ -333,7 +334,7 @@ __device__ __forceinline__ void kernel_r2_all(T r2, const KernelParams<T> &kp, c
     ev[KV_VALUE] = e;
     ev[KV_DL] = r * (kp.s * kp.s) * e;
     ev[KV_PHI] = T(0);
-    if (kp.vmask & (1 << KV_PHI))
+    if (PHI > 0 || (PHI < 0 && (kp.vmask & (1 << KV_PHI))))
       ev[KV_PHI] = r2 > kR2Start<KT, T> ? -M::div_(kp.s, r) * e : T(0);
   } else if constexpr (KT == KT_MATERN32 || KT == KT_MATERN52 || KT == KT_GAUSSIAN) {
     // the shared exponential; dk/dl = -(r^2 / l) phi for these f(r / l)

@@ -1,7 +1,7 @@
 // Matrix-core contractions of the FP32 precision form on BF16 inputs.
 //
 // The kernel entries are evaluated in FP32 exactly as in the FP32 MFMA forms
-// (kernels_mfma.hip), and so are the right operands (rhs rows, moments).  Each
+// (kernels_mfma.hpp), and so are the right operands (rhs rows, moments).  Each
 // FP32 operand v is split into two BF16 terms, hi = bf16(v) (round to nearest
 // even) and lo = bf16(v - hi), and a product a.b is formed as
 //     a_hi.b_hi + a_lo.b_hi + a_hi.b_lo

@@ -11,6 +11,11 @@
 // straight into the matrix core, with no LDS round trip and no shuffles --
 // while the right operand (rhs rows / moments) is staged in LDS once per
 // workgroup and read lane-parallel.
+//
+// The FP32 and FP64 instances are built apart (kernels_mfma_f32.hip,
+// kernels_mfma_f64.hip), side by side.
+#pragma once
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -69,12 +74,15 @@ constexpr int kYsRows = (sizeof(T) == 8 && D < 4) ? 4 : D;
 // three-variant run-time switch keep the default.
 template <typename T, int NT, int KT, bool MULTI>
 constexpr int kMinWaves = (sizeof(T) == 4 && NT <= 2 && !(MULTI && KT < 0)) ? 3 : 1;
-// The FP64 kernels with distances from the matrix cores ask for 2 waves per
-// SIMD (256 registers, a few spills at 32 columns): leaf output 45.3 ms at
-// n = 1e6, 32 rhs, against 56.7 ms with the default target
+// The FP64 kernels of one built-in variant ask for 2 waves per SIMD (256
+// registers, a few spills at 32 columns): leaf output 45.3 ms at n = 1e6, 32
+// rhs, against 56.7 ms with the default target; EXPONENTIAL (distances on the
+// vector ALU) at n = 2e5, degree 3, 16 rhs 4.26 ms against 7.21 ms; the
+// branch-free coupling of several variants (multi_step) needs 177 + 128
+// registers by default, which leaves one wave: 2-D degree 5 n = 2e5, 32
+// columns 1.80 ms against 1.04 ms
 template <typename T, int NT, int KT, bool MULTI>
-constexpr int kMinWavesGram =
-    (sizeof(T) == 8 && !MULTI && kGramNear<KT>) ? 2 : kMinWaves<T, NT, KT, MULTI>;
+constexpr int kMinWavesGram = (sizeof(T) == 8 && KT >= 0) ? 2 : kMinWaves<T, NT, KT, MULTI>;
 
 // The part of a task's list that this workgroup takes (grid.y parts).
 __device__ __forceinline__ void list_part(int &lo, int &hi) {
@@ -83,6 +91,144 @@ __device__ __forceinline__ void list_part(int &lo, int &hi) {
   const int lo0 = lo;
   lo = lo0 + (int)(cnt * blockIdx.y / gridDim.y);
   hi = lo0 + (int)(cnt * (blockIdx.y + 1) / gridDim.y);
+}
+
+// log2 of the wave groups that share the K-steps of a leaf pass of R row tiles
+// and ns sources.  FP32: as many as keep kRT tiles on a wave, whose B operands
+// are then read once (leaves of 62 rows, 16 columns: 1.3 times as fast).  FP64
+// reads few B operands for its MFMA time, so only where the tiles would not
+// spread evenly: the busiest wave's tiles / groups are 1/4, 1/2, 1, 1, 3/2,
+// 3/2, 2, 2 for R = 1..8 against 1, 1, 1, 1, 2, 2, 2, 2 without (2-D n = 2e5
+// degree 5, 16 columns: 0.50 / 0.56 ms).  A list of a few sources does not pay
+// for the addition of the groups (1-D n = 1e5, 3 sources a leaf, 16 columns:
+// 0.26 ms with it, 0.22 without).
+template <typename T>
+__device__ __forceinline__ int leaf_split(int R, int ns) {
+  if (ns < 8) return 0;
+  if constexpr (sizeof(T) == 8) return R == 1 ? 2 : (R == 2 || R == 5 || R == 6 ? 1 : 0);
+  return R <= kRT ? 2 : (R <= 2 * kRT ? 1 : 0);
+}
+
+// One K-step of 4 sources for the row tiles of a wave, squared distances from
+// coordinate differences: x are this lane's rows, y and b its source's
+// coordinates and right operands.
+template <typename T, int D, int KT, int NT, bool MULTI>
+__device__ __forceinline__ void direct_step(const T (&x)[kRT][D], const T (&y)[D],
+                                            const T (&b)[NT], const bool (&tile_on)[kRT], int ntl,
+                                            const int (&tv)[NT], const KernelParams<T> &kp,
+                                            const double *tab,
+                                            typename Mfma<T>::acc_t (&acc)[kRT][NT]) {
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    if (!tile_on[rt]) continue;
+    T r2 = kR2Start<KT, T>;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const T dd = x[rt][d] - y[d];
+      r2 = fmat(dd, dd, r2);
+    }
+    if constexpr (MULTI) {
+      T ev[3];
+      kernel_r2_all<KT, T>(r2, kp, tab, ev);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        if (nt < ntl) acc[rt][nt] = Mfma<T>::mma(pick_variant(ev, tv[nt]), b[nt], acc[rt][nt]);
+    } else {
+      const T e = entry_value<KT, T>(r2, kp, tab);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        if (nt < ntl) acc[rt][nt] = Mfma<T>::mma(e, b[nt], acc[rt][nt]);
+    }
+  }
+}
+
+// The same step of several variants with R tiles on and every column tile in
+// range: no branches, so the tiles' roots, exponentials and matrix products
+// overlap.  The empty asm keeps the variants' values from being sunk into a
+// branch on tv.  PHI: whether phi is among the variants.  FP32 EXPONENTIAL,
+// n = 1e6, value and dk/dl of 16 columns each: leaf output 24.2 -> 16.7 ms,
+// coupling 16.9 -> 11.3 ms.
+template <typename T, int D, int KT, int NT, int R, int PHI>
+__device__ __forceinline__ void multi_step(const T (&x)[kRT][D], const T (&y)[D], const T (&b)[NT],
+                                           const int (&tv)[NT], const KernelParams<T> &kp,
+                                           const double *tab,
+                                           typename Mfma<T>::acc_t (&acc)[kRT][NT]) {
+  T e[R][NT];
+#pragma unroll
+  for (int rt = 0; rt < R; ++rt) {
+    T r2 = kR2Start<KT, T>;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const T dd = x[rt][d] - y[d];
+      r2 = fmat(dd, dd, r2);
+    }
+    T ev[3];
+    kernel_r2_all<KT, T, PHI>(r2, kp, tab, ev);
+    T value = ev[KV_VALUE], dl = ev[KV_DL], phi = ev[KV_PHI];
+    asm("" : "+v"(value), "+v"(dl), "+v"(phi));
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      T v = tv[nt] == KV_DL ? dl : value;
+      if constexpr (PHI) v = tv[nt] == KV_PHI ? phi : v;
+      e[rt][nt] = v;
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = Mfma<T>::mma(e[rt][nt], b[nt], acc[rt][nt]);
+}
+
+// K-steps ks0, ks0 + step, .. < ks1 of the direct form: Y (D rows of stride
+// ys) holds the sources' coordinates, B (rows of stride bs) the right operands.
+template <typename T, int D, int KT, int NT, bool MULTI>
+__device__ __forceinline__ void direct_steps(int ks0, int ks1, int step, int lk, int lr,
+                                             const T *Y, int ys, const T *B, int bs,
+                                             const T (&x)[kRT][D], const bool (&tile_on)[kRT],
+                                             int ntl, const int (&tv)[NT],
+                                             const KernelParams<T> &kp, const double *tab,
+                                             typename Mfma<T>::acc_t (&acc)[kRT][NT]) {
+  auto operands = [&](int ks, T (&y)[D], T (&b)[NT]) {
+    const int s = ks + lk;
+#pragma unroll
+    for (int d = 0; d < D; ++d) y[d] = Y[d * ys + s];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) b[nt] = B[s * bs + nt * 16 + lr];
+  };
+  if constexpr (MULTI && KT >= 0) {
+    if (ntl == NT) {
+      auto run = [&](auto r, auto phi) {
+#pragma unroll 1
+        for (int ks = ks0; ks < ks1; ks += step) {
+          T y[D], b[NT];
+          operands(ks, y, b);
+          multi_step<T, D, KT, NT, decltype(r)::value, decltype(phi)::value>(x, y, b, tv, kp, tab,
+                                                                             acc);
+        }
+      };
+      auto tiles = [&](auto phi) {
+        if (tile_on[3])
+          run(std::integral_constant<int, 4>{}, phi);
+        else if (tile_on[2])
+          run(std::integral_constant<int, 3>{}, phi);
+        else if (tile_on[1])
+          run(std::integral_constant<int, 2>{}, phi);
+        else if (tile_on[0])
+          run(std::integral_constant<int, 1>{}, phi);
+      };
+      if (kp.vmask & (1 << KV_PHI))
+        tiles(std::integral_constant<int, 1>{});
+      else
+        tiles(std::integral_constant<int, 0>{});
+      return;
+    }
+  }
+#pragma unroll 2
+  for (int ks = ks0; ks < ks1; ks += step) {
+    T y[D], b[NT];
+    operands(ks, y, b);
+    direct_step<T, D, KT, NT, MULTI>(x, y, b, tile_on, ntl, tv, kp, tab, acc);
+  }
 }
 
 // Packed tensor index of every moment: a0 | a1 << 8 | a2 << 16.
@@ -94,7 +240,8 @@ __device__ __forceinline__ int unpack(int p, int d) { return (p >> (8 * d)) & 0x
 // fewer than 9 tiles the waves split the K-steps too) and 16*NT rhs columns.
 // MULTI: the rhs columns carry different kernel variants (kp.tv per 16-column
 // tile); every entry is evaluated once for all three variants.
-template <typename T, int D, int KT, int NT, bool MULTI>
+// KS: the launch may K-split (see leaf_split).
+template <typename T, int D, int KT, int NT, bool MULTI, bool KS>
 __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf_output_mfma(
     DevTreeView<T> rows, DevTreeView<T> cols, DevPatternView pat, InterpParams<T> ip,
     KernelParams<T> kp, int nrhs, const T *__restrict__ xs, const T *__restrict__ tlhs,
@@ -156,11 +303,10 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           for (int a = 0; a < P1; ++a) F[(d * P1 + a) * kRowsP + threadIdx.x] = T(0);
       }
     }
-    // K-split: with at most 8 row tiles, kspl groups of waves share the
-    // K-steps, so that every wave holds up to kRT row tiles (their B operands
-    // are read once); the groups' sums are added in LDS in group order
+    // K-split: kspl = 2^ksh groups of waves share the K-steps, each a run of
+    // them; the groups' sums are added in LDS in group order
     const int R = (min(kRows, sz - pbase) + 15) / 16;
-    const int kspl = R <= kRT ? 4 : (R <= 2 * kRT ? 2 : 1);
+    const int ksh = KS ? leaf_split<T>(R, n1 - n0) : 0, kspl = 1 << ksh;
     const int wrows = kWaves / kspl, rg = wave % wrows, sg = wave / wrows;
     // this lane's A rows: tile (rg + wrows rt), row lr
     T x[kRT][D];
@@ -340,43 +486,15 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
               }
             }
           };
-          int s0 = 16 * sg;
-          for (; s0 + 16 <= nj; s0 += 16 * kspl) group(s0, std::true_type{});
-          if (s0 < nj) group(s0, std::false_type{});
+          const int ng = (nj + 15) >> 4, s1 = min(nj, 16 * ((ng * (sg + 1)) >> ksh));
+          int s0 = 16 * ((ng * sg) >> ksh);
+          for (; s0 + 16 <= s1; s0 += 16) group(s0, std::true_type{});
+          if (s0 < s1) group(s0, std::false_type{});
         } else {
-          const int nsteps = (nj + 3) & ~3;
-#pragma unroll 2
-          for (int ks = 4 * sg; ks < nsteps; ks += 4 * kspl) {
-            const int sj = ks + lk;
-            T y[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) y[d] = Ys[d * kChunk + sj];
-            T b[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) b[nt] = Xs[sj * NCP + nt * 16 + lr];
-#pragma unroll
-            for (int rt = 0; rt < kRT; ++rt) {
-              if (!tile_on[rt]) continue;
-              T r2 = kR2Start<KT, T>;
-#pragma unroll
-              for (int d = 0; d < D; ++d) {
-                const T dd = x[rt][d] - y[d];
-                r2 = fmat(dd, dd, r2);
-              }
-              if constexpr (MULTI) {
-                T ev[3];
-                kernel_r2_all<KT, T>(r2, kp, tab, ev);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                  if (nt < ntl) acc[rt][nt] = M::mma(pick_variant(ev, tv[nt]), b[nt], acc[rt][nt]);
-              } else {
-                const T e = entry_value<KT, T>(r2, kp, tab);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                  if (nt < ntl) acc[rt][nt] = M::mma(e, b[nt], acc[rt][nt]);
-              }
-            }
-          }
+          const int ns = (nj + 3) >> 2, ks1 = 4 * ((ns * (sg + 1)) >> ksh);
+          const int ks0 = 4 * ((ns * sg) >> ksh);
+          direct_steps<T, D, KT, NT, MULTI>(ks0, ks1, 4, lk, lr, Ys, kChunk, Xs, NCP, x, tile_on,
+                                            ntl, tv, kp, tab, acc);
         }
       }
       if (kspl > 1) {
@@ -581,38 +699,8 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
         }
         return;
       }
-#pragma unroll 2
-      for (int ks = ks0; ks < nrows; ks += kstep) {
-        const int bl = ks + lk;
-        T y[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) y[d] = Yc[d * kChunk + bl];
-        T b[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) b[nt] = Ms[bl * NCP + nt * 16 + lr];
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          if (!tile_on[rt]) continue;
-          T r2 = kR2Start<KT, T>;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            const T dd = x[rt][d] - y[d];
-            r2 = fmat(dd, dd, r2);
-          }
-          if constexpr (MULTI) {
-            T ev[3];
-            kernel_r2_all<KT, T>(r2, kp, tab, ev);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-              if (nt < ntl) acc[rt][nt] = M::mma(pick_variant(ev, tv[nt]), b[nt], acc[rt][nt]);
-          } else {
-            const T e = entry_value<KT, T>(r2, kp, tab);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-              if (nt < ntl) acc[rt][nt] = M::mma(e, b[nt], acc[rt][nt]);
-          }
-        }
-      }
+      direct_steps<T, D, KT, NT, MULTI>(ks0, nrows, kstep, lk, lr, Yc, kChunk, Ms, NCP, x, tile_on,
+                                        ntl, tv, kp, tab, acc);
     };
     // Chunks are fetched into registers (coordinates py, moments pm) and then
     // written to LDS between two barriers.  FP32 fetches the next chunk right
@@ -957,11 +1045,20 @@ hipError_t launch_mfma_nt(bool output, const MfmaLaunch<T> &a) {
   T *slabs = nullptr;
   const int parts = launch_parts(output, a, &slabs);
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
+  // leaves of more than 8 row tiles are not split in FP32, whose kernels are
+  // then built without the split's registers (FP32 n = 1e6, 244 points a leaf,
+  // 16 columns of two variants: 25.0 ms with them, 24.2 ms without)
+  constexpr bool kAlways = sizeof(T) == 8;
+  const bool ks = kAlways || a.rows.npts <= (int64_t)128 * a.rows.nleaves;
 #define FMCA_MFMA_LAUNCH(K)                                                                   \
-  if (output)                                                                                 \
-    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI>), grid, dim3(256), lds_out,    \
-                       a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs, a.tlhs,     \
-                       a.out, a.ldo, a.natural ? 1 : 0, slabs);                               \
+  if (output && !ks)                                                                          \
+    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI, kAlways>), grid, dim3(256),    \
+                       lds_out, a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs,    \
+                       a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);                       \
+  else if (output)                                                                            \
+    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI, true>), grid, dim3(256),       \
+                       lds_out, a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs,    \
+                       a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);                       \
   else                                                                                        \
     hipLaunchKernelGGL((k_coupling_mfma<T, D, K, NT, MULTI>), grid, dim3(256), lds_cpl,       \
                        a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs,    \
@@ -1011,32 +1108,6 @@ hipError_t launch_mfma_d(bool output, const MfmaLaunch<T> &a) {
 
 }  // namespace
 
-// Leaf moments of the FP32 forms on the matrix cores (q <= 128, >= 8 rhs);
-// false: the caller takes the VALU kernel.
-bool upward_leaf_mfma_supported(int D, int P1, int q, int nrhs) {
-  return q <= 128 && nrhs >= kMfmaMinRhs && D >= 1 && D <= 3 &&
-         ((size_t)D * P1 * 68 + 64 * 36) * sizeof(float) <= 64 * 1024;
-}
-
-hipError_t launch_upward_leaf_mfma(const DevTreeView<float> &tr, const InterpParams<float> &ip,
-                                   const float *xs, int nrhs, float *mom, hipStream_t stream) {
-  const int D = tr.dim, P1 = ip.P1;
-  const int NT = nrhs > 16 ? 2 : 1;
-  const size_t lds = ((size_t)D * P1 * 68 + (size_t)64 * (16 * NT + 4)) * sizeof(float);
-#define FMCA_UPL(DV, NTV)                                                                   \
-  hipLaunchKernelGGL((k_upward_leaf_mfma<DV, NTV>), dim3(tr.nleaves), dim3(256), lds, stream, \
-                     tr, ip, xs, nrhs, mom)
-  if (D == 1) {
-    if (NT == 2) FMCA_UPL(1, 2); else FMCA_UPL(1, 1);
-  } else if (D == 2) {
-    if (NT == 2) FMCA_UPL(2, 2); else FMCA_UPL(2, 1);
-  } else {
-    if (NT == 2) FMCA_UPL(3, 2); else FMCA_UPL(3, 1);
-  }
-#undef FMCA_UPL
-  return hipGetLastError();
-}
-
 template <typename T>
 bool mfma_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vmask, int td) {
   if (nrhs < kMfmaMinRhs) return false;  // the VALU forms are faster there
@@ -1063,10 +1134,5 @@ hipError_t launch_mfma(bool output, const MfmaLaunch<T> &a) {
   }
   return hipErrorInvalidValue;
 }
-
-template bool mfma_supported<float>(bool, int, int, int, int, int, int, int);
-template bool mfma_supported<double>(bool, int, int, int, int, int, int, int);
-template hipError_t launch_mfma<float>(bool, const MfmaLaunch<float> &);
-template hipError_t launch_mfma<double>(bool, const MfmaLaunch<double> &);
 
 }  // namespace fmca_amd
