@@ -256,13 +256,18 @@ __device__ __forceinline__ void stream_item(const T *__restrict__ A, int K, int 
 // 4 / WS groups of WS waves: the groups take every (4 / WS)-th block of the
 // list, the WS waves of a group split the block's row tiles.  The groups'
 // sums are added in LDS in a fixed order, so the result is deterministic.
+// Where the targets are few the lists are cut into grid.y parts (phase_parts),
+// added from their slabs in order: n = 1e5, FP64, 32 rhs has 512 leaves, one
+// round of workgroups that waited for the longest list: output 3.68 -> 2.88 ms
+// in 6 parts, coupling 1.80 -> 1.52 ms (2.9 -> 3.7 TB/s).  Two waves per SIMD
+// are asked for (the FP64 coupling took 263 registers).
 template <typename T, int NT, int WS, int PF, bool OUTPUT>
-__global__ __launch_bounds__(kTB) void k_stream(DevTreeView<T> rows, DevTreeView<T> cols,
+__global__ __launch_bounds__(kTB, 2) void k_stream(DevTreeView<T> rows, DevTreeView<T> cols,
                                                 DevPatternView pat, StoredBlocks<T> st, int q,
                                                 int nrhs, const T *__restrict__ xs,
                                                 const T *__restrict__ mom, T *__restrict__ tlhs,
                                                 double *__restrict__ out, int64_t ldo,
-                                                int natural) {
+                                                int natural, T *__restrict__ part) {
   constexpr int NG = kWaves / WS;  // groups
   constexpr int NC = 16 * NT;      // columns per pass
   extern __shared__ unsigned char smem[];
@@ -283,13 +288,18 @@ __global__ __launch_bounds__(kTB) void k_stream(DevTreeView<T> rows, DevTreeView
     nitems = pat.far_ptr[t + 1] - pat.far_ptr[t];
   }
   const int RP = OUTPUT ? kStoredMaxRows : st.Rq;  // rows of an LDS slot
+  // this part's blocks of the list, and its slab
+  const int i0 = (int)((int64_t)nitems * blockIdx.y / gridDim.y);
+  const int i1 = (int)((int64_t)nitems * (blockIdx.y + 1) / gridDim.y);
+  const bool whole = gridDim.y == 1;
+  T *slab = part + (int64_t)blockIdx.y * (OUTPUT ? rows.npts : (int64_t)rows.ncl * q) * nrhs;
   for (int c0 = 0; c0 < nrhs; c0 += NC) {
     typename Mma<T>::acc_t acc[kMaxRT][NT];
 #pragma unroll
     for (int m = 0; m < kMaxRT; ++m)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[m][nt] = typename Mma<T>::acc_t{0, 0, 0, 0};
-    for (int it = grp; it < nitems; it += NG) {
+    for (int it = i0 + grp; it < i1; it += NG) {
       const T *A, *B;
       int K, brows;
       if (OUTPUT) {
@@ -370,12 +380,14 @@ __global__ __launch_bounds__(kTB) void k_stream(DevTreeView<T> rows, DevTreeView
             const int r = rt * 16 + Mma<T>::crow(lane >> 4, v);
             if (c >= nrhs) continue;
             if (OUTPUT) {
-              if (r < sz) {
+              if (r < sz && !whole) {
+                slab[(int64_t)(bt + r) * nrhs + c] = acc[m][nt][v];
+              } else if (r < sz) {
                 const int64_t row = natural ? (int64_t)rows.perm[bt + r] : (int64_t)(bt + r);
                 out[row + (int64_t)c * ldo] = (double)acc[m][nt][v];
               }
             } else if (r < q) {
-              tlhs[((int64_t)t * q + r) * nrhs + c] = acc[m][nt][v];
+              (whole ? tlhs : slab)[((int64_t)t * q + r) * nrhs + c] = acc[m][nt][v];
             }
           }
         }
@@ -428,10 +440,18 @@ hipError_t launch_assemble(const DevTreeView<T> &rows, const DevTreeView<T> &col
 template <typename T>
 hipError_t launch_stored(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                          const DevPatternView &pat, const StoredBlocks<T> &st, int q, int nrhs,
-                         const T *xs, const T *mom, T *tlhs, double *out, int64_t ldo,
-                         bool natural, hipStream_t stream) {
+                         const ActionBuffers<T> &buf, double *out, int64_t ldo, bool natural,
+                         hipStream_t stream) {
   if (st.Rq > kStoredMaxRows / 2) return hipErrorInvalidValue;
   const int nat = natural ? 1 : 0;
+  // as the matrix-core forms (launch_parts); a target's whole list is one task
+  const int64_t slab = (output ? rows.npts : (int64_t)rows.ncl * q) * (int64_t)nrhs;
+  int parts = output ? phase_parts(rows.nleaves, 0, kWaves, pat.near_per_task, 256, slab,
+                                   buf.part_cap, kFillWavesMfma)
+                     : phase_parts(rows.ncl, 0, kWaves, pat.far_per_task * q, 256, slab,
+                                   buf.part_cap, kFillWavesMfma);
+  T *slabs = nullptr;
+  if (parts > 1 && !(slabs = buf.part(parts * slab))) parts = 1;
   auto lds = [&](int slots, int rp, int nt) { return (size_t)slots * rp * 16 * nt * sizeof(T); };
   // Two column tiles: loads two groups ahead, and the coupling (q <= 128: 8
   // row tiles) spreads its list over 2 two-wave groups.  One column tile:
@@ -440,19 +460,23 @@ hipError_t launch_stored(bool output, const DevTreeView<T> &rows, const DevTreeV
   // waves on one block (16 row tiles).
 #define FMCA_STREAM(NTV, WSC, PFV)                                                           \
   if (output)                                                                                \
-    hipLaunchKernelGGL((k_stream<T, NTV, 4, PFV, true>), dim3(rows.nleaves), dim3(kTB), 0,   \
-                       stream, rows, cols, pat, st, q, nrhs, xs, mom, tlhs, out, ldo, nat);  \
+    hipLaunchKernelGGL((k_stream<T, NTV, 4, PFV, true>), dim3(rows.nleaves, parts), dim3(kTB), \
+                       0, stream, rows, cols, pat, st, q, nrhs, buf.xs, buf.mom, buf.tlhs,    \
+                       out, ldo, nat, slabs);                                                \
   else                                                                                       \
-    hipLaunchKernelGGL((k_stream<T, NTV, WSC, PFV, false>), dim3(rows.ncl), dim3(kTB),       \
+    hipLaunchKernelGGL((k_stream<T, NTV, WSC, PFV, false>), dim3(rows.ncl, parts), dim3(kTB), \
                        lds(WSC == 4 ? 0 : 1, st.Rq, NTV), stream, rows, cols, pat, st, q,    \
-                       nrhs, xs, mom, tlhs, out, ldo, nat);
+                       nrhs, buf.xs, buf.mom, buf.tlhs, out, ldo, nat, slabs);
   if (nrhs <= 16) {
     FMCA_STREAM(1, 4, 1)
   } else {
     FMCA_STREAM(2, 2, 2)
   }
 #undef FMCA_STREAM
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || parts == 1) return e;
+  return launch_add_parts<T>(output, rows, q, nrhs, parts, slabs, buf.tlhs, out, ldo, natural,
+                             stream);
 }
 
 template hipError_t launch_assemble<double>(const DevTreeView<double> &,
@@ -470,13 +494,13 @@ template hipError_t launch_assemble<float>(const DevTreeView<float> &, const Dev
                                            hipStream_t);
 template hipError_t launch_stored<double>(bool, const DevTreeView<double> &,
                                           const DevTreeView<double> &, const DevPatternView &,
-                                          const StoredBlocks<double> &, int, int, const double *,
-                                          const double *, double *, double *, int64_t, bool,
+                                          const StoredBlocks<double> &, int, int,
+                                          const ActionBuffers<double> &, double *, int64_t, bool,
                                           hipStream_t);
 template hipError_t launch_stored<float>(bool, const DevTreeView<float> &,
                                          const DevTreeView<float> &, const DevPatternView &,
-                                         const StoredBlocks<float> &, int, int, const float *,
-                                         const float *, float *, double *, int64_t, bool,
+                                         const StoredBlocks<float> &, int, int,
+                                         const ActionBuffers<float> &, double *, int64_t, bool,
                                          hipStream_t);
 
 }  // namespace fmca_amd

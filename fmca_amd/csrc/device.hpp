@@ -269,8 +269,8 @@ hipError_t launch_assemble(const DevTreeView<T> &rows, const DevTreeView<T> &col
 template <typename T>
 hipError_t launch_stored(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                          const DevPatternView &pat, const StoredBlocks<T> &st, int q, int nrhs,
-                         const T *xs, const T *mom, T *tlhs, double *out, int64_t ldo,
-                         bool natural, hipStream_t stream);
+                         const ActionBuffers<T> &buf, double *out, int64_t ldo, bool natural,
+                         hipStream_t stream);
 
 // Adds the slabs of a phase cut into parts (kernels.hip): the coupling sums of
 // all clusters, or the output rows (natural order through perm, or cluster

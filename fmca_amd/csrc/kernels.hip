@@ -620,8 +620,8 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
   if (tree && ip.td) basis_change(cols.ncl, 1, buf.mom);
   if (stored) {
     // stored coupling matrices; one workgroup per target writes all of it
-    if ((err = launch_stored<T>(false, rows, cols, pat, *stored, q, nrhs, buf.xs, buf.mom,
-                                buf.tlhs, out, ld_out, natural, stream)) != hipSuccess)
+    if ((err = launch_stored<T>(false, rows, cols, pat, *stored, q, nrhs, buf, out, ld_out,
+                                natural, stream)) != hipSuccess)
       return err;
   } else if (tree) {
     if (pat.nfar_split > 0)
@@ -677,8 +677,8 @@ hipError_t action_d(const DevTreeView<T> &rows, const DevTreeView<T> &cols,
     return err;
   }
   if (stored) {
-    err = launch_stored<T>(true, rows, cols, pat, *stored, q, nrhs, buf.xs, buf.mom, buf.tlhs,
-                           out, ld_out, natural, stream);
+    err = launch_stored<T>(true, rows, cols, pat, *stored, q, nrhs, buf, out, ld_out, natural,
+                           stream);
     mark(PH_COUNT);
     return err;
   }
