@@ -837,7 +837,7 @@ def main():
         bf16_flops = 3 * 2.0 * E_near * nrhs  # the three BF16 products of the near field
         entries = E_near
         kname = (f"k_leaf_output_bf16<3, 1, {nt}>" if bf
-                 else f"k_leaf_output_mfma<float, 3, 1, {nt}, false>")
+                 else f"k_leaf_output_mfma<float, 3, 1, {nt}, false, false>")
     else:
         flops = 2.0 * E_far * nrhs
         bf16_flops = 3 * 2.0 * E_far * nrhs
