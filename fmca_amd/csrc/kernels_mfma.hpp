@@ -520,6 +520,25 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           }
         }
       }
+      if (gridDim.y > 1) {  // this part's slab
+        // an opaque lane index keeps these offsets out of the registers of the
+        // loops above (31 spills, 2 % of the FP32 leaf output)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        T *slab = part + ((int64_t)blockIdx.y * rows.npts + b0 + pbase) * nrhs + rc;
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) {
+          if (!tile_on[rt] || sg != 0) continue;
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const int i = (rg + wrows * rt) * 16 + M::crow(ln >> 4, v), c = nt * 16 + (ln & 15);
+              if (pbase + i < sz && rc + c < nrhs) slab[(uint32_t)(i * nrhs + c)] = acc[rt][nt][v];
+            }
+        }
+        continue;
+      }
       // store: C row crow(lk, v) of tile (rg + wrows rt), column lr of rhs tile nt
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
@@ -531,10 +550,6 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           for (int v = 0; v < 4; ++v) {
             const int i = pbase + (rg + wrows * rt) * 16 + M::crow(lk, v);
             if (i < sz && col < nrhs) {
-              if (gridDim.y > 1) {
-                part[((int64_t)blockIdx.y * rows.npts + b0 + i) * nrhs + col] = acc[rt][nt][v];
-                continue;
-              }
               const int64_t row = natural ? (int64_t)rows.perm[b0 + i] : (int64_t)(b0 + i);
               double *p = out + row + (int64_t)col * ldo;
               if (split)
