@@ -67,6 +67,12 @@ void note_device_bytes(int64_t delta) {
   }
 }
 
+// Whether `bytes` more fit under the cap once `given_back` bytes are freed.
+bool device_room(size_t bytes, size_t given_back) {
+  const int64_t cap = g_dev_limit.load();
+  return cap <= 0 || g_dev_live.load() - (int64_t)given_back + (int64_t)bytes <= cap;
+}
+
 // A device allocation owned by the actor.
 struct DevBuf {
   void *p = nullptr;
@@ -84,12 +90,16 @@ struct DevBuf {
     p = nullptr;
     bytes = held = 0;
   }
+  void swap(DevBuf &o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+    std::swap(held, o.held);
+  }
   hipError_t alloc(size_t b) {
     if (b <= bytes && p) return hipSuccess;
     release();
     const size_t h = std::max<size_t>(b, 256);
-    const int64_t cap = g_dev_limit.load();
-    if (cap > 0 && g_dev_live.load() + (int64_t)h > cap) {
+    if (!device_room(h, 0)) {
       p = nullptr;
       return hipErrorOutOfMemory;
     }
@@ -184,10 +194,54 @@ struct DevPattern {
   }
 };
 
+// Most bytes of an action's slabs of partial sums (phases cut into parts).
+constexpr size_t kPartBytes = size_t(256) << 20;
+
+// The slabs of an actor and precision.  A phase that gets no room for them runs
+// uncut, so they are never a reason to refuse an action.  Their size is a
+// bound that grows with the columns only (part_bound), so that an action with
+// as many columns as an earlier one, or fewer, finds them in place.  Slabs that
+// a captured graph reads and writes stay allocated as long as the actor.
+struct PartBuf {
+  DevBuf buf;
+  bool captured = false;  // a graph holds the address of buf
+  std::vector<std::unique_ptr<DevBuf>> graphs;  // outgrown slabs of graphs
+  // Room for `want` bytes, of which the call needs `need`; null: no room.
+  void *get(size_t need, size_t want, bool capturing) {
+    if (buf.bytes < need && !capturing) {
+      auto next = std::make_unique<DevBuf>();
+      if (!captured) {
+        // the old slabs may make room for the new ones
+        if (!device_room(want, buf.held)) return nullptr;
+        buf.release();
+      }
+      if (next->alloc(want) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      buf.swap(*next);
+      if (captured) graphs.push_back(std::move(next));
+      captured = false;
+    }
+    if (buf.bytes < need) return nullptr;
+    captured = captured || capturing;
+    return buf.p;
+  }
+};
+
 template <typename T>
 struct Workspace {
-  DevBuf xs, mom, tlhs, part;
+  DevBuf xs, mom, tlhs;
+  PartBuf part;
 };
+
+// Elements of the slabs of an action with nrhs columns between these trees.
+template <typename T>
+int64_t part_bound(const Tree &a, const Tree &b, int q, int64_t nrhs) {
+  const int64_t slab = std::max(std::max<int64_t>(a.npts, b.npts),
+                                (int64_t)std::max(a.ncl, b.ncl) * q);
+  return std::min<int64_t>(kPartBytes / sizeof(T), kMaxParts * slab * nrhs);
+}
 
 }  // namespace
 
@@ -465,9 +519,6 @@ struct Region {
   size_t bytes;
 };
 
-// Most bytes of an action's slabs of partial sums.
-constexpr size_t kPartBytes = size_t(256) << 20;
-
 constexpr size_t align_up(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Enqueue one action on `stream`.  transpose swaps the roles of the trees.
@@ -476,7 +527,7 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
                     const DevTreeReals<T> &r_cols, const double *d_rhs, int64_t ld_rhs,
                     int64_t nrhs, double *d_out, int64_t ld_out, bool natural, bool transpose,
                     hipStream_t stream, const VariantGroups &groups, const Region *fixed,
-                    bool split_bf16 = false, const GradJob *grad = nullptr) {
+                    bool capturing, bool split_bf16, const GradJob *grad) {
   const Tree &tr_rows = a->rows();
   const Tree &tr_cols = a->cols();
   const DevTreeInts &i_cols = a->shared ? a->d_rows_i : a->d_cols_i;
@@ -525,11 +576,12 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
     buf.xs = ws.xs.template as<T>();
     buf.mom = ws.mom.template as<T>();
     buf.tlhs = ws.tlhs.template as<T>();
-    buf.part_cap = (int64_t)(kPartBytes / sizeof(T));
-    buf.part = [&ws](int64_t elems) -> T * {
-      if (ws.part.alloc((size_t)elems * sizeof(T)) == hipSuccess) return ws.part.template as<T>();
-      (void)hipGetLastError();  // no room: the phase runs uncut
-      return nullptr;
+    // a captured action allocates nothing: it is cut as far as the slabs of the
+    // actions before it allow
+    const size_t want = (size_t)part_bound<T>(tr_rows, tr_cols, q, nrhs) * sizeof(T);
+    buf.part_cap = (int64_t)((capturing ? std::min(want, ws.part.buf.bytes) : want) / sizeof(T));
+    buf.part = [&ws, want, capturing](int64_t elems) {
+      return static_cast<T *>(ws.part.get((size_t)elems * sizeof(T), want, capturing));
     };
   }
   PhaseEvents *pe = nullptr;
@@ -643,7 +695,7 @@ fmca_status enqueue_any_unordered(fmca_h2_actor *a, const double *d_rhs, int64_t
                                   int64_t nrhs, double *d_out, int64_t ld_out, int precision,
                                   bool natural, bool transpose, hipStream_t stream,
                                   const VariantGroups &groups, const Region *fixed,
-                                  const GradJob *grad);
+                                  const GradJob *grad, bool capturing);
 
 // One action on `stream`, ordered after the actor's previous action when that
 // ran on another stream: the workspaces (permuted rhs, moments, sums) are
@@ -659,7 +711,8 @@ fmca_status enqueue_any(fmca_h2_actor *a, const double *d_rhs, int64_t ld_rhs, i
   if (!captured && a->order_valid && a->order_stream != stream)
     HIP_TRY(hipStreamWaitEvent(stream, a->order_ev, 0));
   fmca_status st = enqueue_any_unordered(a, d_rhs, ld_rhs, nrhs, d_out, ld_out, precision,
-                                         natural, transpose, stream, groups, fixed, grad);
+                                         natural, transpose, stream, groups, fixed, grad,
+                                         captured);
   if (st != FMCA_OK || captured) return st;
   HIP_TRY(hipEventRecord(a->order_ev, stream));
   a->order_stream = stream;
@@ -671,7 +724,7 @@ fmca_status enqueue_any_unordered(fmca_h2_actor *a, const double *d_rhs, int64_t
                                   int64_t nrhs, double *d_out, int64_t ld_out, int precision,
                                   bool natural, bool transpose, hipStream_t stream,
                                   const VariantGroups &groups, const Region *fixed,
-                                  const GradJob *grad) {
+                                  const GradJob *grad, bool capturing) {
   if (a->geodesic) {
     // near the diagonal acos turns the rounding of an FP32 dot product into
     // an error of about 1e-7 / r in r, and the derivative in the points of a
@@ -693,11 +746,11 @@ fmca_status enqueue_any_unordered(fmca_h2_actor *a, const double *d_rhs, int64_t
   if (precision == FMCA_PRECISION_FP64)
     return enqueue<double>(a, a->ws64, a->d_rows_64, a->shared ? a->d_rows_64 : a->d_cols_64,
                            d_rhs, ld_rhs, nrhs, d_out, ld_out, natural, transpose, stream,
-                           groups, fixed, false, grad);
+                           groups, fixed, capturing, false, grad);
   if (precision == FMCA_PRECISION_FP32 || precision == FMCA_PRECISION_FP32_BF16)
     return enqueue<float>(a, a->ws32, a->d_rows_32, a->shared ? a->d_rows_32 : a->d_cols_32,
                           d_rhs, ld_rhs, nrhs, d_out, ld_out, natural, transpose, stream,
-                          groups, fixed, precision == FMCA_PRECISION_FP32_BF16, grad);
+                          groups, fixed, capturing, precision == FMCA_PRECISION_FP32_BF16, grad);
   return fail(FMCA_ERR_INVALID_ARGUMENT, "unknown precision");
 }
 
@@ -768,8 +821,7 @@ fmca_status scratch_on_device(int device, void **ptr) {
 namespace fmca_amd {
 int device_malloc(void **p, size_t bytes) {
   const size_t h = std::max<size_t>(bytes, 256);
-  const int64_t cap = g_dev_limit.load();
-  if (cap > 0 && g_dev_live.load() + (int64_t)h > cap) {
+  if (!device_room(h, 0)) {
     *p = nullptr;
     return (int)hipErrorOutOfMemory;
   }

@@ -197,7 +197,11 @@ fmca_status fmca_h2_action_cluster_order(fmca_h2_actor *actor, const double *rhs
  * actor's previous action first waits for that action (an event on the
  * previous stream); this holds for every device entry point below.  Work
  * captured into a HIP graph records no such event: while a stream captures
- * actions of an actor, no other stream may drive it. */
+ * actions of an actor, no other stream may drive it.
+ * Workspaces are sized by the largest column count so far.  An action can be
+ * captured after an eager one of the same precision and direction with as many
+ * columns or more, and its graph replayed until an action of more columns has
+ * outgrown them. */
 fmca_status fmca_h2_action_device(fmca_h2_actor *actor, const double *d_rhs, int64_t ld_rhs,
                                   int64_t nrhs, double *d_out, int64_t ld_out, int precision,
                                   int cluster_order, void *stream);
