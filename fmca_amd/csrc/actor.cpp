@@ -73,6 +73,33 @@ bool device_room(size_t bytes, size_t given_back) {
   return cap <= 0 || g_dev_live.load() - (int64_t)given_back + (int64_t)bytes <= cap;
 }
 
+// Bytes of slabs (PartBuf) that can be taken back, and their release: an
+// allocation that finds no room takes them back first, so that slabs kept for
+// later actions never refuse it.  True if any were freed.
+std::atomic<int64_t> g_slab_bytes{0};
+bool take_back_slabs();
+
+// hipMalloc under the cap; *p is null where it fails.
+hipError_t device_alloc_once(void **p, size_t bytes) {
+  *p = nullptr;
+  if (!device_room(bytes, 0)) return hipErrorOutOfMemory;
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess)
+    note_device_bytes((int64_t)bytes);
+  else
+    *p = nullptr;
+  return e;
+}
+hipError_t device_alloc(void **p, size_t bytes) {
+  hipError_t e = device_alloc_once(p, bytes);
+  if (e == hipErrorOutOfMemory && device_room(bytes, (size_t)g_slab_bytes.load()) &&
+      take_back_slabs()) {
+    (void)hipGetLastError();
+    e = device_alloc_once(p, bytes);
+  }
+  return e;
+}
+
 // A device allocation owned by the actor.
 struct DevBuf {
   void *p = nullptr;
@@ -95,21 +122,14 @@ struct DevBuf {
     std::swap(bytes, o.bytes);
     std::swap(held, o.held);
   }
-  hipError_t alloc(size_t b) {
+  hipError_t alloc(size_t b, bool slabs = false) {
     if (b <= bytes && p) return hipSuccess;
     release();
     const size_t h = std::max<size_t>(b, 256);
-    if (!device_room(h, 0)) {
-      p = nullptr;
-      return hipErrorOutOfMemory;
-    }
-    hipError_t e = hipMalloc(&p, h);
+    const hipError_t e = slabs ? device_alloc_once(&p, h) : device_alloc(&p, h);
     if (e == hipSuccess) {
       bytes = b;
       held = h;
-      note_device_bytes((int64_t)h);
-    } else {
-      p = nullptr;
     }
     return e;
   }
@@ -201,11 +221,19 @@ constexpr size_t kPartBytes = size_t(256) << 20;
 // uncut, so they are never a reason to refuse an action.  Their size is a
 // bound that grows with the columns only (part_bound), so that an action with
 // as many columns as an earlier one, or fewer, finds them in place.  Slabs that
-// a captured graph reads and writes stay allocated as long as the actor.
+// a captured graph reads and writes stay allocated as long as the actor; others
+// are given back when another allocation of the process finds no room.
 struct PartBuf {
   DevBuf buf;
   bool captured = false;  // a graph holds the address of buf
+  std::mutex in_use;      // held from get() to the last launch that uses the slabs
   std::vector<std::unique_ptr<DevBuf>> graphs;  // outgrown slabs of graphs
+  PartBuf();
+  ~PartBuf();
+  void give_back() {
+    if (!captured) g_slab_bytes -= (int64_t)buf.held;
+    buf.release();  // waits for the launches that use it
+  }
   // Room for `want` bytes, of which the call needs `need`; null: no room.
   void *get(size_t need, size_t want, bool capturing) {
     if (buf.bytes < need && !capturing) {
@@ -213,21 +241,51 @@ struct PartBuf {
       if (!captured) {
         // the old slabs may make room for the new ones
         if (!device_room(want, buf.held)) return nullptr;
-        buf.release();
+        give_back();
       }
-      if (next->alloc(want) != hipSuccess) {
+      if (next->alloc(want, true) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
       }
       buf.swap(*next);
       if (captured) graphs.push_back(std::move(next));
       captured = false;
+      g_slab_bytes += (int64_t)buf.held;
     }
     if (buf.bytes < need) return nullptr;
-    captured = captured || capturing;
+    if (capturing && !captured) {
+      captured = true;
+      g_slab_bytes -= (int64_t)buf.held;
+    }
     return buf.p;
   }
 };
+
+std::mutex g_parts_mtx;
+// every PartBuf of the process (never destroyed: actors may outlive statics)
+std::vector<PartBuf *> &g_parts = *new std::vector<PartBuf *>;
+
+PartBuf::PartBuf() {
+  std::lock_guard<std::mutex> lock(g_parts_mtx);
+  g_parts.push_back(this);
+}
+PartBuf::~PartBuf() {
+  std::lock_guard<std::mutex> lock(g_parts_mtx);
+  g_parts.erase(std::find(g_parts.begin(), g_parts.end(), this));
+  give_back();
+}
+
+bool take_back_slabs() {
+  std::lock_guard<std::mutex> lock(g_parts_mtx);
+  bool any = false;
+  for (PartBuf *b : g_parts) {
+    std::unique_lock<std::mutex> use(b->in_use, std::try_to_lock);
+    if (!use.owns_lock() || b->captured || !b->buf.p) continue;
+    b->give_back();
+    any = true;
+  }
+  return any;
+}
 
 template <typename T>
 struct Workspace {
@@ -552,6 +610,7 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
   const size_t b_tlhs = (size_t)t_tgt.ncl * q * nrhs * sizeof(T);
   const DevPatternView v_pat = dpat->view(*pat);
   ActionBuffers<T> buf;
+  std::unique_lock<std::mutex> use_slabs;
   if (fixed) {
     // the caller's region: xs | mom | tlhs, each start aligned to 256 bytes
     const size_t o_mom = align_up(b_xs), o_tlhs = o_mom + align_up(b_mom);
@@ -578,6 +637,7 @@ fmca_status enqueue(fmca_h2_actor *a, Workspace<T> &ws, const DevTreeReals<T> &r
     buf.tlhs = ws.tlhs.template as<T>();
     // a captured action allocates nothing: it is cut as far as the slabs of the
     // actions before it allow
+    use_slabs = std::unique_lock<std::mutex>(ws.part.in_use);
     const size_t want = (size_t)part_bound<T>(tr_rows, tr_cols, q, nrhs) * sizeof(T);
     buf.part_cap = (int64_t)((capturing ? std::min(want, ws.part.buf.bytes) : want) / sizeof(T));
     buf.part = [&ws, want, capturing](int64_t elems) {
@@ -820,14 +880,7 @@ fmca_status scratch_on_device(int device, void **ptr) {
 
 namespace fmca_amd {
 int device_malloc(void **p, size_t bytes) {
-  const size_t h = std::max<size_t>(bytes, 256);
-  if (!device_room(h, 0)) {
-    *p = nullptr;
-    return (int)hipErrorOutOfMemory;
-  }
-  const hipError_t e = hipMalloc(p, h);
-  if (e == hipSuccess) note_device_bytes((int64_t)h);
-  return (int)e;
+  return (int)device_alloc(p, std::max<size_t>(bytes, 256));
 }
 
 void device_free(void *p, size_t bytes) {
@@ -1623,7 +1676,8 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
     size_t budget = free_b / 2;
     const int64_t cap = g_dev_limit.load();
     if (cap > 0) {
-      const int64_t left = cap - g_dev_live.load() - (int64_t)(5 * vec * sizeof(double));
+      const int64_t left = cap - g_dev_live.load() + g_slab_bytes.load() -
+                           (int64_t)(5 * vec * sizeof(double));
       budget = std::min<size_t>(budget, left > 0 ? (size_t)left / 2 : 0);
     }
     m = (int)std::min<size_t>((size_t)kBasisMax, budget / pair_bytes);
@@ -1893,7 +1947,8 @@ fmca_status gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr,
     size_t budget = free_b / 2;
     const int64_t cap = g_dev_limit.load();
     if (cap > 0) {
-      const int64_t left = cap - g_dev_live.load() - (int64_t)(4 * vec * sizeof(double));
+      const int64_t left = cap - g_dev_live.load() + g_slab_bytes.load() -
+                           (int64_t)(4 * vec * sizeof(double));
       budget = std::min<size_t>(budget, left > 0 ? (size_t)left / 2 : 0);
     }
     m = (int)std::min<size_t>((size_t)kBasisMax, budget / pair_bytes);

@@ -69,3 +69,32 @@ def test_graph_keeps_its_slabs(precision, warm, nrhs):
         # captured with other parts than the eager call: another order of the sums
         tol = 1e-14 if precision == "FP64" else 4e-6
         assert (torch.linalg.norm(y - ref) / torch.linalg.norm(ref)).item() <= tol
+
+
+def test_slabs_make_room_for_other_allocations():
+    """Under a memory cap that holds the actor's blocks but not its slabs beside
+    them, the blocks are stored and the actions go on."""
+    import torch
+    import fmca_amd
+    print("[case] cap without room for slabs", flush=True)
+    n = 6000
+    x = _columns(n, 16)
+    H = _actor(n)
+    H.upload()
+    live = fmca_amd.device_memory()[0]
+    H.assemble(fmca_amd.FP64)
+    blocks = fmca_amd.device_memory()[0] - live
+    H.action_device(x)
+    H = _actor(n)
+    H.upload()
+    y = H.action_device(x)
+    live, _ = fmca_amd.device_memory(True)
+    slabs = 16 * n * 16 * 8
+    fmca_amd.set_device_memory_limit(live + blocks - slabs // 2)
+    try:
+        H.assemble(fmca_amd.FP64)
+        z = H.action_device(x)
+        assert fmca_amd.device_memory()[1] <= live + blocks - slabs // 2
+    finally:
+        fmca_amd.set_device_memory_limit(0)
+    assert (torch.linalg.norm(z - y) / torch.linalg.norm(y)).item() <= 1e-13
