@@ -2163,9 +2163,16 @@ fmca_status fmca_h2_cg_device(fmca_h2_actor *a, const double *d_b, int64_t ld_b,
   if (opts->method == FMCA_SOLVER_GCR) {
     *res = fmca_cg_result{};
     const bool f64 = opts->precision == FMCA_PRECISION_FP64;
-    if (nrhs > 1)
-      return f64 ? block_gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
-                 : block_gcr_solve<float>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0);
+    if (nrhs > 1) {
+      st = f64 ? block_gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
+               : block_gcr_solve<float>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0);
+      if (st != FMCA_ERR_OUT_OF_MEMORY) return st;
+      // the form of one space per column holds one vector and up to 16 MB of
+      // partial sums a block less; x is as it was
+      a->basis.clear();
+      for (DevBuf *b : {&a->cg_ws, &a->cg_scal, &a->basis_tab}) b->release();
+      *res = fmca_cg_result{};
+    }
     return f64 ? gcr_solve<double>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0)
                : gcr_solve<float>(a, d_b, ld_b, (int)nrhs, d_x, ld_x, opts, res, sm, t0);
   }

@@ -90,3 +90,26 @@ def test_start_vector_and_small_window():
                        max_basis=m, max_iter=3000)
         assert info["converged"] and info["iterations"] > m
         assert _resid(H, x, b, 0.5) <= 1e-9
+
+
+def test_without_room_for_the_shared_space():
+    """A memory cap that holds the vectors of one space per column but not the
+    block form's partial sums: the solve takes the former."""
+    import torch
+    import fmca_amd
+    H, b = _setup(3000, 8)
+    args = dict(ridge=0.5, tol=1e-9, method="gcr", precision=fmca_amd.FP32, max_basis=40)
+    x0 = torch.zeros_like(b)
+    H.action_device(b, precision=fmca_amd.FP64)
+    H.action_device(b, precision=fmca_amd.FP32)
+    live = fmca_amd.device_memory()[0]
+    # 4 vectors, 40 pairs in chunks of 8, scalars; the block form's sums take 16 MB
+    fmca_amd.set_device_memory_limit(live + (4 * 8 + 40 * 8) * 3000 * 8 + (3 << 20))
+    try:
+        x, info = H.cg(b, x0=x0, **args)
+    finally:
+        fmca_amd.set_device_memory_limit(0)
+    print("  ", info, flush=True)
+    assert info["converged"] and _resid(H, x, b, 0.5) <= 1e-9
+    y, info2 = H.cg(b, x0=x0, **args)
+    assert info2["converged"] and info2["iterations"] < info["iterations"]
