@@ -1564,6 +1564,10 @@ constexpr int kBasisChunk = 8;  // slot pairs per basis allocation
 // 10 more iterations, the same FP64 actions).
 constexpr double kInnerTarget = 0.5;
 
+// The larger of two relative residuals; not finite if one of them is not, as
+// that of a column with a NaN or an infinity, which no solve reaches.
+double worse(double a, double b) { return std::isnan(a) || b <= a ? a : b; }
+
 // T and T a of one block (32 x 32, row-major) from its Gram matrix G = Y^T Y
 // and H = Y^T R: with G = D L L^T D in pivoted order on its columns (D = diag
 // ||y_b||), T = D^-1 L^-T makes Y T orthonormal and a = T^T H are the
@@ -1795,7 +1799,7 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
     target[j] = opts->tol * std::sqrt(bn2[j]);
     active[j] = live[j] = rmax[j] > target[j];
     any = any || active[j];
-    worst = std::max(worst, rmax[j] / std::sqrt(bn2[j]));
+    worst = worse(worst, rmax[j] / std::sqrt(bn2[j]));
   }
   res->rel_residual = worst;
   GCR_TRY(push_flags());
@@ -1872,7 +1876,7 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
     any = false;
     for (int j = 0; j < nr; ++j) {
       const double rn = std::sqrt(rn2[j]);
-      worst = std::max(worst, rn / std::sqrt(bn2[j]));
+      worst = worse(worst, rn / std::sqrt(bn2[j]));
       if (active[j] && rn <= target[j]) active[j] = 0;
       live[j] = active[j];
       any = any || active[j];
@@ -1887,11 +1891,11 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
     for (int j = 0; j < nr; ++j)
       if (active[j]) rmax[j] = std::sqrt(rn2[j]);
   }
-  res->converged = !any;
+  res->converged = !any && std::isfinite(res->rel_residual);
   if (any) {  // stopped by a cap: report the FP64 residual of the returned x
     if ((st = residual()) != FMCA_OK) return st;
     worst = 0;
-    for (int j = 0; j < nr; ++j) worst = std::max(worst, std::sqrt(rn2[j] / bn2[j]));
+    for (int j = 0; j < nr; ++j) worst = worse(worst, std::sqrt(rn2[j] / bn2[j]));
     res->rel_residual = worst;
   }
   if (cl)
@@ -2051,7 +2055,7 @@ fmca_status gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr,
     target[j] = opts->tol * std::sqrt(bn2[j]);
     active[j] = rmax[j] > target[j];
     any = any || active[j];
-    worst = std::max(worst, rmax[j] / std::sqrt(bn2[j]));
+    worst = worse(worst, rmax[j] / std::sqrt(bn2[j]));
   }
   res->rel_residual = worst;
   GCR_TRY(push_active());
@@ -2098,7 +2102,7 @@ fmca_status gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr,
     any = false;
     for (int j = 0; j < nr; ++j) {
       const double rn = std::sqrt(rn2[j]);
-      worst = std::max(worst, rn / std::sqrt(bn2[j]));
+      worst = worse(worst, rn / std::sqrt(bn2[j]));
       if (active[j] && rn <= target[j]) active[j] = 0;
       any = any || active[j];
     }
@@ -2113,14 +2117,14 @@ fmca_status gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr,
     for (int j = 0; j < nr; ++j)
       if (active[j]) rmax[j] = std::sqrt(rn2[j]);
   }
-  res->converged = !any;
+  res->converged = !any && std::isfinite(res->rel_residual);
   if (any) {  // stopped by a cap: report the FP64 residual of the returned x
     if ((st = matvec(X, Y, FMCA_PRECISION_FP64)) != FMCA_OK) return st;
     GCR_TRY(blas1_residual(n, nr, ridge, B, n, Y, n, X, n, R, n, sm));
     GCR_TRY(blas1_dot(n, nr, R, n, R, n, d_rr, d_scratch, sm));
     if ((st = read_rr()) != FMCA_OK) return st;
     worst = 0;
-    for (int j = 0; j < nr; ++j) worst = std::max(worst, std::sqrt(rn2[j] / bn2[j]));
+    for (int j = 0; j < nr; ++j) worst = worse(worst, std::sqrt(rn2[j] / bn2[j]));
     res->rel_residual = worst;
   }
   if (cl)
@@ -2264,7 +2268,7 @@ fmca_status fmca_h2_cg_device(fmca_h2_actor *a, const double *d_b, int64_t ld_b,
     target[j] = opts->tol * std::sqrt(bn2[j]);
     active[j] = rmax[j] > target[j];
     any = any || active[j];
-    worst = std::max(worst, rmax[j] / std::sqrt(bn2[j]));
+    worst = worse(worst, rmax[j] / std::sqrt(bn2[j]));
   }
   res->rel_residual = worst;
   CG_TRY(hipMemcpyAsync(Pv, R, vec * sizeof(double), hipMemcpyDeviceToDevice, sm));
@@ -2316,7 +2320,7 @@ fmca_status fmca_h2_cg_device(fmca_h2_actor *a, const double *d_b, int64_t ld_b,
       for (int j = 0; j < nr; ++j) {
         const double rn = std::sqrt(rn2[j]);
         rmax[j] = rn;
-        worst = std::max(worst, rn / std::sqrt(bn2[j]));
+        worst = worse(worst, rn / std::sqrt(bn2[j]));
         if (active[j] && rn <= target[j]) active[j] = 0;
       }
       res->rel_residual = worst;
@@ -2338,13 +2342,13 @@ fmca_status fmca_h2_cg_device(fmca_h2_actor *a, const double *d_b, int64_t ld_b,
     CG_TRY(upload(d_beta, h_beta));
     CG_TRY(blas1_xpby(n, nr, d_beta, R, n, Pv, n, sm));
   }
-  res->converged = !any;
+  res->converged = !any && std::isfinite(res->rel_residual);
   if (any) {  // stopped by a cap: report the FP64 residual of the returned x
     if ((st = matvec(X, Y, FMCA_PRECISION_FP64)) != FMCA_OK) return st;
     CG_TRY(blas1_residual(n, nr, ridge, B, n, Y, n, X, n, R, n, sm));
     if ((st = dot(R, R, rn2.data())) != FMCA_OK) return st;
     worst = 0;
-    for (int j = 0; j < nr; ++j) worst = std::max(worst, std::sqrt(rn2[j] / bn2[j]));
+    for (int j = 0; j < nr; ++j) worst = worse(worst, std::sqrt(rn2[j] / bn2[j]));
     res->rel_residual = worst;
   }
   if (cl)

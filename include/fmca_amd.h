@@ -276,7 +276,8 @@ typedef struct {
   int matvecs_fp32;     /* FP32 actions */
   double rel_residual;  /* max over columns of ||b - (K + ridge I) x|| / ||b||, FP64 action,
                            at the last replacement, or of the returned x when a cap
-                           stopped the solve */
+                           stopped the solve; not finite (and converged 0) if a column
+                           of b or x is not */
   double seconds;       /* wall time of the solve */
   int indefinite;       /* 1 if a column met p.(K + ridge I)p <= 0 (the H2 matrix plus ridge
                            is not positive definite); the solve then stops */

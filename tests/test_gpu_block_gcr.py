@@ -49,7 +49,8 @@ def test_block_sizes(n, nrhs, precision):
 def test_dependent_zero_and_non_finite_columns():
     """Equal and linearly dependent columns leave the block with fewer new
     directions than columns; zero columns stay zero; a column of NaN is
-    neither solved nor lets its values into the others."""
+    neither solved nor lets its values into the others, which are, and the
+    solve reports that not every column reached tol."""
     import torch
     import fmca_amd
     H, b = _setup(3000, 7)
@@ -61,7 +62,8 @@ def test_dependent_zero_and_non_finite_columns():
     for prec in (fmca_amd.FP64, fmca_amd.FP32_BF16):
         x, info = H.cg(b, x0=torch.zeros_like(b), ridge=0.3, tol=1e-9, method="gcr",
                        precision=prec, max_iter=300)
-        assert info["converged"]
+        assert not info["converged"] and np.isnan(info["rel_residual"])
+        assert info["iterations"] < 300
         assert _resid(H, x[:, good].t().contiguous().t(), b[:, good].t().contiguous().t(),
                       0.3) <= 1e-9
         assert torch.all(x[:, 4] == 0) and torch.all(x[:, 5] == 0)
@@ -113,3 +115,22 @@ def test_without_room_for_the_shared_space():
     assert info["converged"] and _resid(H, x, b, 0.5) <= 1e-9
     y, info2 = H.cg(b, x0=x0, **args)
     assert info2["converged"] and info2["iterations"] < info["iterations"]
+
+
+@pytest.mark.parametrize("method,nrhs", [("cg", 3), ("gcr", 1), ("gcr", 3)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_non_finite_column_is_reported(method, nrhs, bad):
+    """No solver reports convergence when a column of b (or, as NaN, of the
+    start vector) is not finite."""
+    import torch
+    import fmca_amd
+    H, b = _setup(500, nrhs)
+    x0 = torch.zeros_like(b)
+    for where in (b, x0) if np.isnan(bad) else (b,):
+        v = where[7, nrhs - 1].item()
+        where[7, nrhs - 1] = bad
+        x, info = H.cg(b, x0=x0, ridge=0.5, method=method, precision=fmca_amd.FP64)
+        assert not info["converged"] and not np.isfinite(info["rel_residual"])
+        where[7, nrhs - 1] = v
+    x, info = H.cg(b, x0=x0, ridge=0.5, method=method, precision=fmca_amd.FP64)
+    assert info["converged"]
