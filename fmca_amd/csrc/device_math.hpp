@@ -149,9 +149,14 @@ __constant__ double kExp2Table[64] = {
 //          r2 > 1e-284 as it was and makes k(0) its value at r = 1e-150.
 //   2^(-t / 64): k = rint(t), f = k - t in [-1/2, 1/2], 2^(f / 64) - 1 by its
 //          Taylor polynomial of degree 5 (remainder < 4e-17), times the table
-//          value of -k mod 64 (LDS), scaled by ldexp; 10 operations instead
+//          value of -k mod 64 (LDS), scaled by ldexp; 11 operations instead
 //          of 21 for the reduction by ln 2 and a degree-12 polynomial.  The
 //          result carries the rounding of one fma and of the table value.
+//          t stops at 64 * 1100, where the result is 0: an infinite t would
+//          leave f NaN, one past 2^31 a k outside of an int (0.2-1.6 % of an
+//          FP64 action; rounding by an added constant instead of rint and the
+//          conversion gains that back in the direct forms and loses it in the
+//          Gram forms).
 // FP64 action, n = 1e4, 1 rhs: 42 -> 27 vector operations per entry.
 constexpr double kTinyR2 = 1e-300;
 
@@ -163,6 +168,7 @@ __device__ __forceinline__ double sqrt_pos(double x) {
 }
 
 __device__ __forceinline__ double exp2_neg64(double t, const double *tab) {
+  t = __builtin_fmin(t, 64.0 * 1100);
   const double k = __builtin_rint(t);
   const int n = (int)(-k);
   const double f = k - t;

@@ -65,3 +65,23 @@ def test_fp32_exp_sqrt():
     s32 = s.astype(np.float32).astype(np.float64)
     ys = _run(3, s)
     assert (np.abs(ys - np.sqrt(s32)) / np.maximum(np.sqrt(s32), 1e-30)).max() < 3e-7
+
+
+@pytest.mark.parametrize("ktype,ratio", [
+    (k, r) for k in ("EXPONENTIAL", "MATERN32", "MATERN52", "GAUSSIAN") for r in (2e3, 1e5, 1e9, 1e30)
+] + [("GAUSSIAN", 1e160)])
+@pytest.mark.parametrize("nrhs", [1, 8, 16])
+def test_far_entries_are_exactly_zero(ktype, ratio, nrhs):
+    """FP64 entries of points many lengthscales apart, up to a squared distance
+    that overflows, are 0."""
+    import torch
+    import fmca_amd
+    print(f"[case] {ktype} {ratio:g} lengthscales, {nrhs} columns", flush=True)
+    P = np.array([[0.0, ratio * 0.3]])
+    H = fmca_amd.H2kernelActor(fmca_amd.CovarianceKernel(ktype, 0.3), P, P, 2, 0.8)
+    x = torch.zeros(nrhs, 2, dtype=torch.float64, device="cuda").t()
+    x[1] = 1.0
+    y = H.action_device(x).cpu().numpy()
+    assert np.all(y[0] == 0)
+    if nrhs <= 8:  # vector forms: exact distances of equal points
+        assert np.all(y[1] == 1)
