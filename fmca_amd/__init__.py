@@ -260,7 +260,9 @@ class H2kernelActor:
         at most 256), the residual minimised over the window, with the same
         replacement rule; a replaced residual is projected on the window.  The
         pairs stay consistent under lower-precision matvecs, so FP32 forms
-        converge in about as many iterations as FP64.
+        converge in about as many iterations as FP64.  Two columns or more
+        share their directions, up to 32 at a time (block GCR): fewer
+        iterations, but a column's iterates depend on those beside it.
 
         b, x0: float64 CUDA tensors (n,) or (n, nrhs); x0 defaults to b as in
         pCG.  Returns (x, info) with info['rel_residual'] measured with the

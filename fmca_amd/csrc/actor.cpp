@@ -1568,6 +1568,16 @@ constexpr double kInnerTarget = 0.5;
 // that of a column with a NaN or an infinity, which no solve reaches.
 double worse(double a, double b) { return std::isnan(a) || b <= a ? a : b; }
 
+// Stall of a block's recurrence: its worst column has not halved for
+// kStallShort iterations once it has dropped to kStallDrop since the last
+// replacement, or for kStallLong without that.  The directions are then the
+// rounding of the stored pairs and of the matvec, and only the FP64 residual
+// brings new ones.  NumPy model, n = 1000, ridge 1e-7 n, refine_factor 3e-5, 8
+// columns: no end without the rule, 136 iterations and 8 replacements with it,
+// 177 and 14 with 8 iterations for the longer one, 115 and 17 with 4.
+constexpr double kStallDrop = 0.1;
+constexpr int kStallShort = 4, kStallLong = 12;
+
 // T and T a of one block (32 x 32, row-major) from its Gram matrix G = Y^T Y
 // and H = Y^T R: with G = D L L^T D in pivoted order on its columns (D = diag
 // ||y_b||), T = D^-1 L^-T makes Y T orthonormal and a = T^T H are the
@@ -1642,7 +1652,7 @@ int block_factor(const double *G, const double *H, const double *sq, double lost
 // block as well), makes it orthonormal through its Gram matrix, and removes
 // from every residual of the block its component on the whole new image
 // block: ||r|| is minimised over the directions of all columns, so the
-// iterations fall with the block size (n = 1e6, 32 columns: 58 -> 14; one
+// iterations fall with the block size (n = 1e6, 32 columns: 58 -> 12; one
 // iteration costs one action either way).  Pairs stay consistent with their
 // own matvec as in gcr_solve, and the residual replacement is the same.
 // A block whose columns are all below their target, or have dropped by
@@ -1650,8 +1660,10 @@ int block_factor(const double *G, const double *H, const double *sq, double lost
 // recurrence with FP32 pairs stalls at about 3e-8 of a cycle's start, and pairs
 // made from there on are rounding.  When no column has a new direction left (rank 0: the window
 // spans the space to rounding) the residual is replaced and projected, which
-// still reduces it by the rounding of the stored pairs; the solve stops when
-// that no longer halves it.  One column is served by gcr_solve, whose kernels
+// still reduces it by the rounding of the stored pairs; when that no longer
+// halves it, a new window is begun, and the solve stops when a new window does
+// not halve it either.  A block whose recurrence stalls counts as ready, and
+// pairs after which the FP64 residual has grown are dropped.  One column is served by gcr_solve, whose kernels
 // read each stored pair once in vector form.
 template <typename S>
 fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, int nr, double *d_x,
@@ -1805,6 +1817,12 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
   GCR_TRY(push_flags());
   int first = 0, count = 0;
   double stuck_at = std::numeric_limits<double>::infinity();  // residual of the last rank 0
+  // largest FP64 residual at the last replacement, at the last restart of a
+  // window that was spent
+  double replaced = std::numeric_limits<double>::infinity(), restarted = replaced;
+  // least drop of a block's worst column since its last halving, iterations since
+  std::vector<double> low(ng, std::numeric_limits<double>::infinity());
+  std::vector<int> idle(ng, 0);
   while (any && res->iterations < max_iter && res->outer < max_updates) {
     // the image block (K + ridge I) r of the unit residuals, orthogonal to the
     // window (Y), and its directions (W)
@@ -1840,6 +1858,7 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
     double top = 0;
     for (int g = 0; g < ng; ++g) {
       bool ready = true;  // every column of the block
+      double drop = 0;    // of its worst column, since the last replacement
       const int c0 = g * bs, c1 = std::min(nr, c0 + bs);
       for (int j = c0; j < c1; ++j) {
         if (!active[j]) continue;
@@ -1850,6 +1869,12 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
         all_done = all_done && done;
         ready = ready && (done || (prec != FMCA_PRECISION_FP64 && rn < delta * rmax[j]));
         top = std::max(top, rn / std::sqrt(bn2[j]));
+        if (!done) drop = std::max(drop, rn / rmax[j]);
+      }
+      if (prec != FMCA_PRECISION_FP64 && !ready) {
+        idle[g] = drop < 0.5 * low[g] ? 0 : idle[g] + 1;
+        if (idle[g] == 0) low[g] = drop;
+        ready = idle[g] >= (drop < kStallDrop ? kStallShort : kStallLong);
       }
       all_ready = all_ready && ready;
       // a block that is ready waits for the others: further directions would
@@ -1865,39 +1890,56 @@ fmca_status block_gcr_solve(fmca_h2_actor *a, const double *d_b, int64_t ld_b, i
       if (changed) GCR_TRY(push_flags());
       continue;
     }
+    bool spent = false;  // the window spans all that the matvec resolves
     if (rank == 0) {
-      if (!(top < 0.5 * stuck_at)) break;
-      stuck_at = top;
+      spent = !(top < 0.5 * stuck_at);
+      stuck_at = spent ? std::numeric_limits<double>::infinity() : top;
     }
     // FP64 residual; columns that meet tol stop, the others are projected
     if ((st = residual()) != FMCA_OK) return st;
     res->outer++;
     worst = 0;
     any = false;
+    double left = 0;  // of the columns that go on
     for (int j = 0; j < nr; ++j) {
       const double rn = std::sqrt(rn2[j]);
       worst = worse(worst, rn / std::sqrt(bn2[j]));
       if (active[j] && rn <= target[j]) active[j] = 0;
       live[j] = active[j];
       any = any || active[j];
+      if (active[j]) left = std::max(left, rn / std::sqrt(bn2[j]));
     }
     res->rel_residual = worst;
     GCR_TRY(push_flags());
     if (!any) break;
+    // a replaced residual no smaller than the last one: the pairs made since
+    // are rounding, and so are further ones next to them; start a new window
+    if (spent || !(left < replaced)) count = 0;
+    replaced = left;
+    if (spent) {
+      if (!(left < 0.5 * restarted)) break;
+      restarted = left;
+    }
     GCR_TRY(block_dots<S>(ld, nr, R, d_qtab, first, count, m, d_active, d_coef, d_scratch, sm));
     GCR_TRY(block_combine<S>(ld, nr, d_qtab, d_ptab, first, count, m, d_coef, d_active, R, -1.0,
                              X, 1.0, sm));
     if ((st = read_norms(R)) != FMCA_OK) return st;
     for (int j = 0; j < nr; ++j)
       if (active[j]) rmax[j] = std::sqrt(rn2[j]);
+    std::fill(low.begin(), low.end(), std::numeric_limits<double>::infinity());
+    std::fill(idle.begin(), idle.end(), 0);
   }
-  res->converged = !any && std::isfinite(res->rel_residual);
-  if (any) {  // stopped by a cap: report the FP64 residual of the returned x
+  if (any) {  // stopped: the FP64 residual of the returned x decides
     if ((st = residual()) != FMCA_OK) return st;
     worst = 0;
-    for (int j = 0; j < nr; ++j) worst = worse(worst, std::sqrt(rn2[j] / bn2[j]));
+    any = false;
+    for (int j = 0; j < nr; ++j) {
+      worst = worse(worst, std::sqrt(rn2[j] / bn2[j]));
+      any = any || std::sqrt(rn2[j]) > target[j];
+    }
     res->rel_residual = worst;
   }
+  res->converged = !any && std::isfinite(res->rel_residual);
   if (cl)
     GCR_TRY(blas1_permute(n, nr, perm, false, X, ld, d_x, ld_x, sm));
   else

@@ -251,9 +251,15 @@ fmca_status fmca_h2_action_transpose_device(fmca_h2_actor *actor, const double *
  *                    them.  Each stored pair is consistent as its matvec
  *                    computed it, so lower-precision matvecs do not delay
  *                    convergence as they do CG's; a replaced residual is
- *                    projected on the window.  Holds 2 max_basis vectors
- *                    of n x nrhs (FP64 for FP64 matvecs, FP32 otherwise)
- *                    during the solve.
+ *                    projected on the window.  With two columns or more the
+ *                    columns of a block of up to 32 share their directions
+ *                    (one Krylov space for the block; a column's iterates then
+ *                    depend on those beside it), the residual is also replaced
+ *                    when the iterated one stalls before it has dropped by
+ *                    refine_factor, and one that has grown since the last
+ *                    replacement starts a new window.  Holds 2 max_basis
+ *                    vectors of n x nrhs (FP64 for FP64 matvecs, FP32
+ *                    otherwise) during the solve.
  * Convergence is always decided on the FP64 residual. */
 enum { FMCA_SOLVER_CG = 0, FMCA_SOLVER_GCR = 1 };
 typedef struct {

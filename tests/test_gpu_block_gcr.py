@@ -134,3 +134,36 @@ def test_a_non_finite_column_is_reported(method, nrhs, bad):
         where[7, nrhs - 1] = v
     x, info = H.cg(b, x0=x0, ridge=0.5, method=method, precision=fmca_amd.FP64)
     assert info["converged"]
+
+
+@pytest.mark.parametrize("precision,n,nrhs", [("FP32", 5000, 32), ("FP32", 1000, 2),
+                                              ("FP32_BF16", 1000, 8), ("FP32_BF16", 1000, 32)])
+def test_a_stalled_recurrence_is_replaced(precision, n, nrhs):
+    """Ridge 1e-7 n and a refine_factor below what the stored pairs of lower
+    precision reach: the block's recurrence stalls before its columns have
+    dropped by the factor, and goes on from the FP64 residual."""
+    import torch
+    import fmca_amd
+    from fmca_amd import workloads as W
+    print(f"[case] {precision} n={n} nrhs={nrhs}", flush=True)
+    P = W.uniform(n, 3, 1)
+    H = fmca_amd.H2kernelActor(fmca_amd.CovarianceKernel("MATERN32", 0.4), P, P, 4, 0.8)
+    b = torch.from_numpy(np.random.default_rng(1).standard_normal((n, nrhs))).cuda()
+    x, info = H.cg(b, x0=torch.zeros_like(b), ridge=1e-7 * n, tol=1e-8, method="gcr",
+                   precision=getattr(fmca_amd, precision), refine_factor=3e-5, max_iter=1000)
+    print("  ", info, flush=True)
+    assert info["converged"] and info["rel_residual"] <= 1e-8
+
+
+def test_a_solve_stopped_at_its_cap_is_judged_by_its_residual():
+    """The last iteration allowed meets tol: converged, as the FP64 residual
+    of the returned x says."""
+    import torch
+    import fmca_amd
+    H, b = _setup(2000, 4)
+    args = dict(x0=torch.zeros_like(b), ridge=0.5, tol=1e-8, method="gcr",
+                precision=fmca_amd.FP64)
+    _, full = H.cg(b, **args)
+    for k in (full["iterations"], full["iterations"] - 1):
+        _, info = H.cg(b, max_iter=k, **args)
+        assert info["converged"] == (info["rel_residual"] <= 1e-8)
