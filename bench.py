@@ -843,7 +843,7 @@ def main():
         bf16_flops = 3 * 2.0 * E_far * nrhs
         entries = E_far
         kname = (f"k_coupling_bf16<3, 1, {nt}>" if bf
-                 else f"k_coupling_mfma<float, 3, 1, {nt}, false>")
+                 else f"k_coupling_mfma<float, 3, 1, {nt}, false, false>")
     achieved = flops / t_dom / 1e12
     roofline = {
         # the products are FP32-accurate (FP32 entries; BF16 three-term split or

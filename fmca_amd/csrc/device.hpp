@@ -152,18 +152,20 @@ struct ActionBuffers {
 // Parts of a phase's lists.  A launch of few or of long workgroups leaves CUs
 // idle, at its end above all (n = 1e6, 1 rhs: 16 leaf workgroups per CU, 8 of
 // them resident, kept the CUs 65 % busy).  So the workgroups take grid.y
-// contiguous parts of every task's list, until the launch has about
-// kFillWaves waves (8 rounds of 8 waves per SIMD) or a part has fewer than
-// `least` sources on average.  Part k writes slab k and the slabs are added
-// in order.  Launches with split tasks (nsplit) already add atomically and
-// are not cut further.
+// contiguous parts of every task's list, as many as keep the launch within
+// kFillWaves waves (8 rounds of 8 waves per SIMD) and a part at `least` sources
+// or more on average.  Part k writes slab k and the slabs are added in order:
+// a pass over memory and a launch more, which a launch that fills half the
+// chip or more does not get back (FP32, 64 columns, 2048 leaves of 98 rows and
+// 1767 sources: 0.97 ms whole, 1.18 ms in two parts).  Launches with split
+// tasks (nsplit) already add atomically and are not cut further.
 constexpr int kFillWaves = 65536;
 constexpr int kFillWavesMfma = 12288;  // the matrix-core forms: fewer waves per SIMD
 constexpr int kMaxParts = 16;
 inline int phase_parts(int tasks, int nsplit, int waves, double sources, double least,
                        int64_t slab, int64_t cap, int fill = kFillWaves) {
   if (nsplit > 0 || tasks <= 0 || slab <= 0) return 1;
-  const double want = std::ceil((double)fill / ((double)tasks * waves));
+  const double want = std::floor((double)fill / ((double)tasks * waves));
   const double most = std::min(sources / least, (double)(cap / slab));
   const int k = (int)std::min(std::min(want, most), (double)kMaxParts);
   return k < 2 ? 1 : k;
@@ -305,18 +307,21 @@ using MfmaLaunch = PhaseLaunch<T>;
 template <typename T>
 hipError_t launch_valu(bool output, const ValuLaunch<T> &a);
 
-// Parts of a matrix-core launch (256 threads per task) and their slabs.
+// Parts of a matrix-core launch of `waves` waves per task, and their slabs.
+// 3 rounds of the 4 resident waves per SIMD.  A part has at least 1024 sources
+// (FP64, whose entries take twice the time: 512): 512 leaves of 68 rows and
+// 1171 sources, FP32, 32 columns, take 109 us whole, 120 us in two parts.
+// Fewer than two tasks per CU are cut down to 256 sources (n = 4000, 3-D degree
+// 3, 16 columns: 69 us an action, 99 us with 1024).
 template <typename T>
-inline int launch_parts(bool output, const MfmaLaunch<T> &a, T **slabs) {
-  // a part has at least two staged chunks of 128 sources; 3 rounds of the 4
-  // resident waves per SIMD
+inline int launch_parts(bool output, const MfmaLaunch<T> &a, int waves, T **slabs) {
+  const int tasks = output ? a.pat.nnear_order : a.pat.nfar_order;
+  const double least = tasks < 512 ? 256 : (sizeof(T) == 8 ? 512 : 1024);
   const int64_t slab =
       (output ? a.rows.npts : (int64_t)a.rows.ncl * a.ip.q) * (int64_t)a.nrhs;
-  int parts = output ? phase_parts(a.pat.nnear_order, a.pat.nnear_split, 4, a.pat.near_per_task,
-                                   256, slab, a.part_cap, kFillWavesMfma)
-                     : phase_parts(a.pat.nfar_order, a.pat.nfar_split, 4,
-                                   a.pat.far_per_task * a.ip.q, 256, slab, a.part_cap,
-                                   kFillWavesMfma);
+  int parts = phase_parts(tasks, output ? a.pat.nnear_split : a.pat.nfar_split, waves,
+                          output ? a.pat.near_per_task : a.pat.far_per_task * a.ip.q, least, slab,
+                          a.part_cap, kFillWavesMfma);
   if (parts > 1 && !(*slabs = a.part(parts * slab))) parts = 1;
   return parts;
 }

@@ -850,7 +850,7 @@ hipError_t launch_bf16_nt(bool output, const MfmaLaunch<float> &a) {
   const size_t lds_out = leaf_output_bf16_lds<NT>(D, a.ip.P1, a.ip.q);
   const size_t lds_cpl = coupling_bf16_lds<NT>(D, a.ip.q);
   float *slabs = nullptr;
-  const int parts = launch_parts(output, a, &slabs);
+  const int parts = launch_parts(output, a, 4, &slabs);
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
 #define FMCA_BF16_LAUNCH(K)                                                                   \
   if (output)                                                                                 \

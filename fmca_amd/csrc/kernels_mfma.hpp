@@ -93,20 +93,30 @@ __device__ __forceinline__ void list_part(int &lo, int &hi) {
   hi = lo0 + (int)(cnt * (blockIdx.y + 1) / gridDim.y);
 }
 
-// log2 of the wave groups that share the K-steps of a leaf pass of R row tiles
-// and ns sources.  FP32: as many as keep kRT tiles on a wave, whose B operands
-// are then read once (leaves of 62 rows, 16 columns: 1.3 times as fast).  FP64
-// reads few B operands for its MFMA time, so only where the tiles would not
-// spread evenly: the busiest wave's tiles / groups are 1/4, 1/2, 1, 1, 3/2,
-// 3/2, 2, 2 for R = 1..8 against 1, 1, 1, 1, 2, 2, 2, 2 without (2-D n = 2e5
-// degree 5, 16 columns: 0.50 / 0.56 ms).  A list of a few sources does not pay
-// for the addition of the groups (1-D n = 1e5, 3 sources a leaf, 16 columns:
-// 0.26 ms with it, 0.22 without).
+// log2 of the wave groups that share the K-steps of a leaf pass of R row tiles.
+// FP32: as many as keep kRT tiles on a wave, whose B operands are then read
+// once (leaves of 62 rows, 16 columns: 1.3 times as fast).  FP64 reads few B
+// operands for its MFMA time, so only where the tiles would not spread evenly:
+// the busiest wave's tiles / groups are 1/4, 1/2, 1, 1, 3/2, 3/2, 2, 2 for
+// R = 1..8 against 1, 1, 1, 1, 2, 2, 2, 2 without.
 template <typename T>
-__device__ __forceinline__ int leaf_split(int R, int ns) {
-  if (ns < 8) return 0;
+__device__ __forceinline__ int leaf_split(int R) {
   if constexpr (sizeof(T) == 8) return R == 1 ? 2 : (R == 2 || R == 5 || R == 6 ? 1 : 0);
   return R <= kRT ? 2 : (R <= 2 * kRT ? 1 : 0);
+}
+
+// Whether the leaf output splits its K-steps: the groups' sums cost up to five
+// barriers a column tile, which a short list does not pay for.  `rows`: mean
+// rows of a leaf, `sources`: mean sources of a part's list.  FP32, 16 columns,
+// split / not (us): 2-D degree 1 (6 rows, 77 sources, n = 2e5) 464 / 353;
+// degree 2 (12 rows, 172) 288 / 251; 3-D degree 1 (11 rows, 675) 196 / 222;
+// total degree 3 (24 rows, 2031) 770 / 883; but 2-D degree 5 (49 rows, 831)
+// 249 / 219, 3-D degree 2 (49 rows, 3429) 812 / 808 and on clusters (49 rows,
+// 6491) 839 / 1012.  Leaves of more than 8 row tiles have nothing to split.
+template <typename T>
+inline bool leaf_split_pays(double rows, double sources) {
+  if (sizeof(T) == 8) return rows <= 48 && sources >= 300;
+  return rows <= 128 && sources >= (rows <= 48 ? 600 : 1000);
 }
 
 // One K-step of 4 sources for the row tiles of a wave, squared distances from
@@ -240,12 +250,12 @@ __device__ __forceinline__ int unpack(int p, int d) { return (p >> (8 * d)) & 0x
 // fewer than 9 tiles the waves split the K-steps too) and 16*NT rhs columns.
 // MULTI: the rhs columns carry different kernel variants (kp.tv per 16-column
 // tile); every entry is evaluated once for all three variants.
-// KS: the launch may K-split (see leaf_split).
-template <typename T, int D, int KT, int NT, bool MULTI, bool KS>
+// CUT: the launch may K-split (see leaf_split) or is cut into parts.
+template <typename T, int D, int KT, int NT, bool MULTI, bool CUT>
 __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf_output_mfma(
     DevTreeView<T> rows, DevTreeView<T> cols, DevPatternView pat, InterpParams<T> ip,
     KernelParams<T> kp, int nrhs, const T *__restrict__ xs, const T *__restrict__ tlhs,
-    double *__restrict__ out, int64_t ldo, int natural, T *__restrict__ part) {
+    double *__restrict__ out, int64_t ldo, int natural, int ksplit, T *__restrict__ part) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int NC = 16 * NT;
@@ -274,8 +284,8 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
   const int li = pat.near_task[4 * task], flags = pat.near_task[4 * task + 3];
   int n0 = pat.near_task[4 * task + 1], n1 = pat.near_task[4 * task + 2];
   const bool split = (flags & kTaskSplit) != 0;
-  const bool do_far = (flags & kTaskFar) != 0 && pat.has_far && blockIdx.y == 0;
-  list_part(n0, n1);
+  const bool do_far = (flags & kTaskFar) != 0 && tlhs && (!CUT || blockIdx.y == 0);
+  if constexpr (CUT) list_part(n0, n1);
   const int c = rows.leaves[li];
   const int b0 = rows.begin[c], sz = rows.size[c];
   for (int e = threadIdx.x; e < qpad; e += blockDim.x)
@@ -306,8 +316,8 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
     // K-split: kspl = 2^ksh groups of waves share the K-steps, each a run of
     // them; the groups' sums are added in LDS in group order
     const int R = (min(kRows, sz - pbase) + 15) / 16;
-    const int ksh = KS ? leaf_split<T>(R, n1 - n0) : 0, kspl = 1 << ksh;
-    const int wrows = kWaves / kspl, rg = wave % wrows, sg = wave / wrows;
+    const int ksh = CUT && ksplit ? leaf_split<T>(R) : 0, kspl = 1 << ksh;
+    const int wrows = kWaves / kspl, rg = CUT ? wave % wrows : wave, sg = CUT ? wave / wrows : 0;
     // this lane's A rows: tile (rg + wrows rt), row lr
     T x[kRT][D];
     bool tile_on[kRT];
@@ -393,7 +403,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
       int nb = n0, j0 = 0, pnj = 0;
       // a run of sources with adjacent point ranges is staged as one source
       auto fetch = [&]() {
-        const int run = min(pat.near_run[nb], n1 - nb);
+        const int run = CUT ? min(pat.near_run[nb], n1 - nb) : pat.near_run[nb];
         const int s = pat.near_src[nb], sl = pat.near_src[nb + run - 1];
         const int sb = cols.begin[s], ss = cols.begin[sl] + cols.size[sl] - sb;
         pnj = min(kChunk, ss - j0);
@@ -520,7 +530,7 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
           }
         }
       }
-      if (gridDim.y > 1) {  // this part's slab
+      if (CUT && gridDim.y > 1) {  // this part's slab
         // an opaque lane index keeps these offsets out of the registers of the
         // loops above (31 spills, 2 % of the FP32 leaf output)
         int ln = lane;
@@ -571,12 +581,12 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_leaf
 // most kRT row tiles) every wave takes all row tiles and a quarter of the
 // K-steps, and the four partial sums are added in LDS (in wave order, so the
 // result does not depend on scheduling): all waves stay busy.
-template <typename T, int D, int KT, int NT, bool MULTI>
-__global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coupling_mfma(DevTreeView<T> rows, DevTreeView<T> cols,
-                                                       DevPatternView pat, InterpParams<T> ip,
-                                                       KernelParams<T> kp, int nrhs,
-                                                       const T *__restrict__ mom,
-                                                       T *__restrict__ tlhs, T *__restrict__ part) {
+// CUT: the launch is cut into parts.
+template <typename T, int D, int KT, int NT, bool MULTI, bool CUT>
+__global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coupling_mfma(
+    DevTreeView<T> rows, DevTreeView<T> cols, DevPatternView pat, InterpParams<T> ip,
+    KernelParams<T> kp, int nrhs, const T *__restrict__ mom, T *__restrict__ tlhs,
+    T *__restrict__ part) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int NC = 16 * NT;
@@ -603,9 +613,12 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
   if (task < 0) return;
   const int t = pat.far_task[4 * task];
   int f0 = pat.far_task[4 * task + 1], f1 = pat.far_task[4 * task + 2];
-  list_part(f0, f1);
   // sums of this part: its slab, or the coupling sums themselves
-  T *dst_all = gridDim.y > 1 ? part + (int64_t)blockIdx.y * rows.ncl * ip.q * nrhs : tlhs;
+  T *dst_all = tlhs;
+  if constexpr (CUT) {
+    list_part(f0, f1);
+    if (gridDim.y > 1) dst_all = part + (int64_t)blockIdx.y * rows.ncl * ip.q * nrhs;
+  }
   const bool split = (pat.far_task[4 * task + 3] & kTaskSplit) != 0;
   // K-split: with R row tiles, kspl groups of waves (4 for R <= kRT, 2 for
   // R <= 2 kRT, else 1) share the K-steps, so that every wave holds up to kRT
@@ -1058,26 +1071,32 @@ hipError_t launch_mfma_nt(bool output, const MfmaLaunch<T> &a) {
   // (a derivative variant there goes to the run-time switch, K = -1)
   const int key = MULTI ? base : a.kp.kt;
   T *slabs = nullptr;
-  const int parts = launch_parts(output, a, &slabs);
+  const int parts = launch_parts(output, a, kWaves, &slabs);
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
-  // leaves of more than 8 row tiles are not split in FP32, whose kernels are
-  // then built without the split's registers (FP32 n = 1e6, 244 points a leaf,
-  // 16 columns of two variants: 25.0 ms with them, 24.2 ms without)
-  constexpr bool kAlways = sizeof(T) == 8;
-  const bool ks = kAlways || a.rows.npts <= (int64_t)128 * a.rows.nleaves;
+  const double per_part = a.pat.near_per_task / parts;
+  const int ksplit = output && leaf_split_pays<T>((double)a.rows.npts / a.rows.nleaves, per_part);
+  // an uncut launch takes kernels without the parts' and the split's registers
+  // (FP32 leaf output, 32 columns: 95 spilled SGPRs with them, 56 without; 49
+  // rows of 816 sources, n = 25000: 79 / 71 us)
+  const bool cut = parts > 1 || ksplit;
+  const T *far = a.pat.has_far ? a.tlhs : nullptr;  // null: no far field to add
+#define FMCA_MFMA_OUTPUT(K, C)                                                                \
+  hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI, C>), grid, dim3(256), lds_out,   \
+                     a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs, far,          \
+                     a.out, a.ldo, a.natural ? 1 : 0, ksplit, slabs)
+#define FMCA_MFMA_COUPLING(K, C)                                                              \
+  hipLaunchKernelGGL((k_coupling_mfma<T, D, K, NT, MULTI, C>), grid, dim3(256), lds_cpl,      \
+                     a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs,      \
+                     slabs)
 #define FMCA_MFMA_LAUNCH(K)                                                                   \
-  if (output && !ks)                                                                          \
-    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI, kAlways>), grid, dim3(256),    \
-                       lds_out, a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs,    \
-                       a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);                       \
+  if (output && !cut)                                                                         \
+    FMCA_MFMA_OUTPUT(K, false);                                                             \
   else if (output)                                                                            \
-    hipLaunchKernelGGL((k_leaf_output_mfma<T, D, K, NT, MULTI, true>), grid, dim3(256),       \
-                       lds_out, a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.xs,    \
-                       a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);                       \
+    FMCA_MFMA_OUTPUT(K, true);                                                                \
+  else if (!cut)                                                                              \
+    FMCA_MFMA_COUPLING(K, false);                                                           \
   else                                                                                        \
-    hipLaunchKernelGGL((k_coupling_mfma<T, D, K, NT, MULTI>), grid, dim3(256), lds_cpl,       \
-                       a.stream, a.rows, a.cols, a.pat, a.ip, a.kp, a.nrhs, a.mom, a.tlhs,    \
-                       slabs)
+    FMCA_MFMA_COUPLING(K, true)
   switch (key) {
     case KT_EXPONENTIAL:
       FMCA_MFMA_LAUNCH(KT_EXPONENTIAL);
@@ -1095,6 +1114,8 @@ hipError_t launch_mfma_nt(bool output, const MfmaLaunch<T> &a) {
       FMCA_MFMA_LAUNCH(-1);
   }
 #undef FMCA_MFMA_LAUNCH
+#undef FMCA_MFMA_OUTPUT
+#undef FMCA_MFMA_COUPLING
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || parts == 1) return e;
   return launch_add_parts<T>(output, a.rows, a.ip.q, a.nrhs, parts, slabs, a.tlhs, a.out, a.ldo,
