@@ -112,11 +112,13 @@ __device__ __forceinline__ int leaf_split(int R) {
 // degree 2 (12 rows, 172) 288 / 251; 3-D degree 1 (11 rows, 675) 196 / 222;
 // total degree 3 (24 rows, 2031) 770 / 883; but 2-D degree 5 (49 rows, 831)
 // 249 / 219, 3-D degree 2 (49 rows, 3429) 812 / 808 and on clusters (49 rows,
-// 6491) 839 / 1012.  Leaves of more than 8 row tiles have nothing to split.
+// 6491) 839 / 1012.  Fewer than two leaves per CU leave it idle otherwise
+// (n = 4000, 2-D degree 2, 256 leaves, 211 sources: 19 / 24; degree 4, 128, 475:
+// 28 / 35).  Leaves of more than 8 row tiles have nothing to split.
 template <typename T>
-inline bool leaf_split_pays(double rows, double sources) {
+inline bool leaf_split_pays(double rows, double sources, int leaves) {
   if (sizeof(T) == 8) return rows <= 48 && sources >= 300;
-  return rows <= 128 && sources >= (rows <= 48 ? 600 : 1000);
+  return rows <= 128 && sources >= (rows > 48 ? 1000 : (leaves < 512 ? 200 : 600));
 }
 
 // One K-step of 4 sources for the row tiles of a wave, squared distances from
@@ -1074,7 +1076,8 @@ hipError_t launch_mfma_nt(bool output, const MfmaLaunch<T> &a) {
   const int parts = launch_parts(output, a, kWaves, &slabs);
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
   const double per_part = a.pat.near_per_task / parts;
-  const int ksplit = output && leaf_split_pays<T>((double)a.rows.npts / a.rows.nleaves, per_part);
+  const int ksplit = output && leaf_split_pays<T>((double)a.rows.npts / a.rows.nleaves, per_part,
+                                                  a.rows.nleaves);
   // an uncut launch takes kernels without the parts' and the split's registers
   // (FP32 leaf output, 32 columns: 95 spilled SGPRs with them, 56 without; 49
   // rows of 816 sources, n = 25000: 79 / 71 us)
