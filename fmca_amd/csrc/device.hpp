@@ -345,6 +345,7 @@ hipError_t launch_upward_leaf_mfma(const DevTreeView<float> &tr, const InterpPar
 // BF16 three-term forms of the FP32 leaf output / coupling (kernels_bf16.hip):
 // kernel values only, >= kMfmaMinRhs rhs, where the LDS staging fits.
 bool bf16_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vmask);
+bool bf16_pays(bool output, const MfmaLaunch<float> &a);
 // The right operand the launch reads (xs for the leaf output, mom for the
 // coupling) is split into BF16 halves in place first, so it holds hi | lo << 16
 // words afterwards.

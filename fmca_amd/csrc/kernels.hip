@@ -453,7 +453,9 @@ hipError_t dispatch_nr(bool output, const DevTreeView<T> &rows, const DevTreeVie
                          out,  ldo,  natural, buf.part, buf.part_cap, stream};
   if constexpr (sizeof(T) == 4) {
     if (kp.geodesic) return hipErrorInvalidValue;
-    if (kp.split_bf16 && bf16_supported(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask))
+    if (kp.split_bf16 && bf16_supported(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask) &&
+        (bf16_pays(output, a) ||
+         !mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td)))
       return launch_bf16(output, a, buf.xs, buf.mom);
   }
   // FP64 with at most 8 columns of one variant: an FP64 MFMA fills 16 columns

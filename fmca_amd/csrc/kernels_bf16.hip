@@ -14,6 +14,9 @@
 // squared distances come from the same instruction on three-term splits (24
 // bits, see source_operand).
 //
+// Used where leaves and node sets are large enough (bf16_pays); the FP32 form
+// takes the others.
+//
 // What bounds them: the vector ALU work of an entry (root, exponential,
 // polynomial, split: about 60 cycles per 64 entries) plus the part of the
 // matrix-core time that it does not hide.  Measured (ms, n = 1e6, MATERN32,
@@ -148,29 +151,33 @@ template <int NT>
 constexpr int kOcc = NT <= 2 ? 4 : 2;
 
 // K-split of R row tiles: with fewer than 9 tiles, groups of waves share the
-// K-steps, so that every wave holds up to kRT row tiles; the groups' sums are
-// added in LDS in group order.  wave = rg + wrows sg.
+// K-steps, at most four groups, as a chunk has four; so that no wave holds more
+// than kRT row tiles, and one where there are at most two.  The groups' sums
+// are added in LDS in group order.  wave = rg + wrows sg.  Against no split
+// (us, 16 / 64 columns): leaf output of 49 rows (3-D degree 2, n = 2e5) 709 /
+// 1945 against 878 / 2810, coupling of q = 64 (3-D degree 3, n = 2e5) 610 / 2093
+// against 817 / 3080.
 __device__ __forceinline__ int k_split(int R) {
-  return R <= kRT ? 8 : (R <= 2 * kRT ? 4 : (R <= 4 * kRT ? 2 : 1));
+  return R <= 2 * kRT ? 4 : (R <= 4 * kRT ? 2 : 1);
 }
 
-// Adds the wave groups' accumulators over LDS, one column tile at a time; the
-// sums end in group 0.  Red: [16 R][16].
+// Adds the wave groups' accumulators over LDS; the sums end in group 0.
+// Red: [16 R][16 NT] (R <= 8: at most the staged right operand's room).
 template <int NT>
 __device__ __forceinline__ void add_groups(f32x4 (&acc)[kRT][NT], float *Red, int kspl, int wrows,
                                            int rg, int sg, const bool (&tile_on)[kRT], int lr,
                                            int lk) {
+  for (int g = 1; g <= kspl; ++g) {
+    __syncthreads();
+    if (sg != g % kspl) continue;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    for (int g = 1; g <= kspl; ++g) {
-      __syncthreads();
-      if (sg != g % kspl) continue;
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
         if (!tile_on[rt]) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          float *dst = Red + ((rg + wrows * rt) * 16 + 4 * lk + v) * 16 + lr;
+          float *dst = Red + (((rg + wrows * rt) * 16 + 4 * lk + v) * NT + nt) * 16 + lr;
           const float sum = (g == 1 ? 0.f : *dst) + acc[rt][nt][v];
           if (g < kspl)
             *dst = sum;
@@ -178,7 +185,6 @@ __device__ __forceinline__ void add_groups(f32x4 (&acc)[kRT][NT], float *Red, in
             acc[rt][nt][v] = sum;
         }
       }
-    }
   }
 }
 
@@ -850,7 +856,7 @@ hipError_t launch_bf16_nt(bool output, const MfmaLaunch<float> &a) {
   const size_t lds_out = leaf_output_bf16_lds<NT>(D, a.ip.P1, a.ip.q);
   const size_t lds_cpl = coupling_bf16_lds<NT>(D, a.ip.q);
   float *slabs = nullptr;
-  const int parts = launch_parts(output, a, 4, &slabs);
+  const int parts = launch_parts(output, a, kWaves, &slabs);
   const dim3 grid(output ? a.pat.nnear_order : a.pat.nfar_order, (unsigned)parts);
 #define FMCA_BF16_LAUNCH(K)                                                                   \
   if (output)                                                                                 \
@@ -906,6 +912,27 @@ hipError_t launch_bf16_d(bool output, const MfmaLaunch<float> &a) {
 }
 
 }  // namespace
+
+// Where the BF16 form is the faster one.  A chunk of 128 sources or nodes is
+// staged by eight waves between two barriers; small row counts leave most of a
+// K-step's tiles empty and short lists most of a chunk, and the FP32 form, of
+// four waves and smaller tiles, is faster there.  FP32 / BF16 (us):
+//   leaf output, 16 / 64 columns: 6 rows (2-D degree 1, n = 2e5) 465 / 1087 and
+//     1266 / 3487; 24 rows (2-D degree 3, n = 2e5) 218 / 333 and 699 / 983; 49
+//     rows with 831 sources (2-D degree 5, n = 2e5) 216 / 266 and 682 / 822, with
+//     3429 (3-D degree 2, n = 2e5) 804 / 709 and 2246 / 1945; 62 rows with 869,
+//     but only 64 leaves (n = 4000) 30 / 28 and 58 / 39;
+//   coupling: q = 16 (2-D degree 3, n = 2e5) 207 / 307 and 647 / 1152; q = 36
+//     with 663 nodes (2-D degree 5, n = 2e5) 253 / 306 and 908 / 1147, with 1132
+//     (clusters) 242 / 226 and 946 / 907; q = 27 with 2335 (3-D degree 2,
+//     n = 2e5) 817 / 702 and 2844 / 2844; few clusters (n = 4000, q = 25) 29 / 23.
+bool bf16_pays(bool output, const MfmaLaunch<float> &a) {
+  if (output)
+    return a.rows.npts > (int64_t)48 * a.rows.nleaves &&
+           (a.pat.near_per_task >= 1000 || a.rows.nleaves < 512);
+  const int q = a.ip.q;
+  return q > 48 || (q > 16 && (a.pat.far_per_task * q >= 700 || a.rows.ncl < 512));
+}
 
 bool bf16_supported(bool output, int D, int P1, int q, int nrhs, int kt, int vmask) {
   if (nrhs < kMfmaMinRhs) return false;

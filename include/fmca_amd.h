@@ -42,7 +42,9 @@ enum {
    * (hi = bf16(v), lo = bf16(v - hi)), products hi.hi + lo.hi + hi.lo with
    * FP32 accumulation -- the error class of FP32 entries at 3/16 of the FP32
    * matrix-core cycles.  Used where the FP32 form would use the matrix cores
-   * for kernel values (>= 8 rhs); every other phase is the FP32 form's. */
+   * for kernel values (>= 8 rhs) on leaves of more than 48 points and node
+   * sets of more than 16, where it is the faster of the two; every other phase
+   * is the FP32 form's. */
   FMCA_PRECISION_FP32_BF16 = 2
 };
 

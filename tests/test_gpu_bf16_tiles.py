@@ -1,6 +1,7 @@
-"""The BF16 matrix-core form against FP64: leaves of one to sixteen and more row
+"""The BF16 precision form against FP64: leaves of one to sixteen and more row
 tiles (wave groups that share the sources), node counts around the same edges,
-passes of 16, 32 and 64 columns with remainders, every distance form."""
+passes of 16, 32 and 64 columns with remainders, every distance form.  The
+smallest leaves and node sets take the FP32 form's kernels."""
 import numpy as np
 import pytest
 
