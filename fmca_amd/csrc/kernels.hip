@@ -444,6 +444,29 @@ __global__ __launch_bounds__(kBlock) void k_add_parts_out(int64_t n, int nrhs, i
 
 constexpr size_t kLdsLimit = 64 * 1024;
 
+// FP64 with at most 8 columns of one variant: an FP64 MFMA fills 16 columns and
+// takes as long as the vector FMAs of 16 (neither overlaps the other), so the
+// vector forms win while one source's nodes fill few passes of their workgroup
+// (q <= 64; D P1 <= 20 keeps a full 8-column tile inside their LDS).  8
+// columns, MFMA / vector (us):
+//   leaf output  2-D n = 2e5 degree 5 (q = 36) 563 / 317, 3-D n = 25000 degree 2
+//     643 / 367, degree 3 on clusters 2452 / 1587; but 2-D on clusters, whose
+//     split tasks are not cut into parts and take one row a thread, degree 6
+//     1110 / 1527 and 7 1207 / 2979;
+//   coupling  2-D n = 2e5 degree 5 997 / 420, 3-D degree 3 2207 / 1364; but with
+//     lines of two nodes (3-D degree 1, n = 25000) 188 / 261, nodes taken singly
+//     (total degree, q = 20, n = 25000) 274 / 293, launches of few entries
+//     (2-D degree 4, n = 4000, 1.7e6 entries) 37 / 51, split tasks at q = 64
+//     (degree 3, clusters) 377 / 473.
+// Past q = 64 the coupling turns: degree 4 (q = 125), n = 2e5, 1.94 / 3.56 ms.
+template <typename T>
+bool few_columns_pay(bool output, int D, const InterpParams<T> &ip, const DevPatternView &pat) {
+  if (output) return !(pat.nnear_split > 0 && D < 3 && ip.q > 36);
+  const double entries = pat.far_per_task * pat.nfar_order * ip.q * ip.q;
+  return entries >= 2e6 && !(pat.nfar_split > 0 && ip.q > 56) &&
+         (ip.td ? ip.q >= 32 : ip.P1 >= 3);
+}
+
 template <typename T, int D>
 hipError_t dispatch_nr(bool output, const DevTreeView<T> &rows, const DevTreeView<T> &cols,
                        const DevPatternView &pat, const InterpParams<T> &ip,
@@ -458,17 +481,8 @@ hipError_t dispatch_nr(bool output, const DevTreeView<T> &rows, const DevTreeVie
          !mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td)))
       return launch_bf16(output, a, buf.xs, buf.mom);
   }
-  // FP64 with at most 8 columns of one variant: an FP64 MFMA fills 16 columns
-  // and takes as long as the vector FMAs of 16 (neither overlaps the other), so
-  // the vector forms win while one source's nodes fill few passes of their
-  // workgroup.  8 columns, MFMA / vector (ms, leaf output and coupling): 2-D
-  // n = 2e5 degree 5 (q = 36) 0.54 + 0.74 / 0.33 + 0.48, 3-D n = 2e5 degree 3
-  // (q = 64) EXPONENTIAL 7.18 + 2.03 / 2.43 + 1.33; past q = 64 the coupling
-  // turns: degree 4 (q = 125) GAUSSIAN 4.82 + 1.94 / 4.48 + 3.56.  16 columns
-  // (q = 36): 0.54 + 0.75 / 0.53 + 0.89.  The bounds keep a full 8-column tile
-  // inside the vector forms' LDS.
   const bool few = sizeof(T) == 8 && nrhs <= 8 && (kp.vmask & (kp.vmask - 1)) == 0 &&
-                   ip.q <= 64 && D * ip.P1 <= 20;
+                   ip.q <= 64 && D * ip.P1 <= 20 && few_columns_pay(output, D, ip, pat);
   if (!few && !kp.geodesic &&
       mfma_supported<T>(output, D, ip.P1, ip.q, nrhs, kp.kt, kp.vmask, ip.td))
     return launch_mfma<T>(output, a);
