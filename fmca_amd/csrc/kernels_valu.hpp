@@ -41,6 +41,11 @@ namespace {
 using namespace dev;
 
 constexpr int kAlphaTile = 128;  // far-field coefficients staged per step
+// Nodes of a source from which the coupling stages one source at a time; below,
+// all sources of a tile at once, as most threads would idle and a list of a few
+// nodes wait for a loop over the tile's sources (coupling, FP32, 1 rhs, n = 2e5:
+// 1-D degree 1 247 -> 142 us, 2-D degree 1 228 -> 100, degree 3 120 -> 91).
+constexpr int kWholeSources = 32;
 
 // Rows per thread, while the accumulators are few.  More rows share a source's
 // LDS reads and, in the coupling, the setup of a line; one row leaves the FP64
@@ -104,7 +109,8 @@ __global__ __launch_bounds__(256) void k_leaf_output(DevTreeView<T> rows, DevTre
                                                      const T *__restrict__ xs,
                                                      const T *__restrict__ tlhs,
                                                      double *__restrict__ out, int64_t ldo,
-                                                     int natural, T *__restrict__ part) {
+                                                     int natural, int smax,
+                                                     T *__restrict__ part) {
   constexpr int RPT = kRowsPerThread<T, D, NR, true>;
   constexpr int RS = kRecord<T, D, NR>;
   constexpr bool TAB = !GEO && kTableEntry<KT, T>;
@@ -137,7 +143,7 @@ __global__ __launch_bounds__(256) void k_leaf_output(DevTreeView<T> rows, DevTre
     for (int pbase = 0; pbase < sz; pbase += nt) {
       const int nrow = min(nt, sz - pbase);
       const int nh = (nrow + RPT - 1) / RPT;
-      const int S = min(nt / nh, 32);
+      const int S = min(nt / nh, smax);
       const int slice = threadIdx.x / nh, tr = threadIdx.x - slice * nh;
       const bool act = slice < S;
       T x[RPT][D], acc[RPT][NR];
@@ -297,10 +303,11 @@ __host__ __device__ inline int coupling_head(int P1, int NL, int G) {
 // other axes is formed once per line, which leaves 2 + 4 / P1 operations of
 // distance per entry instead of 6 in 3-D.  Total-degree nodes and geodesic
 // entries take one node at a time ("lines" of one node).
-template <typename T, int D, int KT, int NR, bool GEO>
+// FEW: q < kWholeSources (see there).
+template <typename T, int D, int KT, int NR, bool GEO, bool FEW>
 __global__ __launch_bounds__(256) void k_coupling(DevTreeView<T> rows, DevTreeView<T> cols,
                                                   DevPatternView pat, InterpParams<T> ip,
-                                                  KernelParams<T> kp, int nrhs, int G,
+                                                  KernelParams<T> kp, int nrhs, int G, int smax,
                                                   const T *__restrict__ mom,
                                                   T *__restrict__ tlhs, T *__restrict__ part) {
   constexpr int RPT = kRowsPerThread<T, D, NR, false>;
@@ -340,14 +347,20 @@ __global__ __launch_bounds__(256) void k_coupling(DevTreeView<T> rows, DevTreeVi
     for (int d = 0; d < D; ++d) Ul[l * D + d] = unit(l * P1, d);
   if (lines)
     for (int b = threadIdx.x; b < P1; b += nt) U0[b] = ip.xi[b];
-  for (int g = 0; g < G; ++g)
-    for (int l = threadIdx.x; l < NL; l += nt) gl[g * NL + l] = g * P1;
+  // e / q and e / NL of a tile's nodes and lines (at most 2^15)
+  [[maybe_unused]] const float rq = 1.0f / (float)q, rl = 1.0f / (float)NL;
+  if constexpr (FEW) {
+    for (int e = threadIdx.x; e < G * NL; e += nt) gl[e] = (int)(((float)e + 0.5f) * rl) * P1;
+  } else {
+    for (int g = 0; g < G; ++g)
+      for (int l = threadIdx.x; l < NL; l += nt) gl[g * NL + l] = g * P1;
+  }
   for (int rc = 0; rc < nrhs; rc += NR) {
     const int nr = min(NR, nrhs - rc);
     for (int abase = 0; abase < q; abase += nt) {
       const int nrow = min(nt, q - abase);
       const int nh = (nrow + RPT - 1) / RPT;
-      const int S = min(nt / nh, 32);
+      const int S = min(nt / nh, smax);
       const int slice = threadIdx.x / nh, tr = threadIdx.x - slice * nh;
       const bool act = slice < S;
       T x[RPT][D], acc[RPT][NR];
@@ -363,24 +376,44 @@ __global__ __launch_bounds__(256) void k_coupling(DevTreeView<T> rows, DevTreeVi
       for (int f = f0; f < f1; f += G) {
         const int ns = min(G, f1 - f);
         __syncthreads();
-        for (int g = 0; g < ns; ++g) {
-          const int64_t s = pat.far_src[f + g];
-          T bs[D], bm[D];
+        if constexpr (FEW) {  // threads over the nodes and lines of all sources
+          for (int e = threadIdx.x; e < ns * q; e += nt) {
+            const int g = (int)(((float)e + 0.5f) * rq);
+            const T *ms = mom + ((int64_t)pat.far_src[f + g] * q + (e - g * q)) * nrhs + rc;
 #pragma unroll
-          for (int d = 0; d < D; ++d) {
-            bs[d] = cols.bbsize[s * D + d];
-            bm[d] = cols.bbmin[s * D + d];
+            for (int r = 0; r < NR; ++r) Mv[e * NR + r] = r < nr ? ms[r] : T(0);
           }
-          const T *ms = mom + s * q * nrhs + rc;
-          for (int j = threadIdx.x; j < q; j += nt)
+          for (int e = threadIdx.x; e < ns * NL; e += nt) {
+            const int g = (int)(((float)e + 0.5f) * rl), l = e - g * NL;
+            const int64_t s = pat.far_src[f + g];
 #pragma unroll
-            for (int r = 0; r < NR; ++r)
-              Mv[(g * q + j) * NR + r] = r < nr ? ms[(int64_t)j * nrhs + r] : T(0);
-          for (int l = threadIdx.x; l < NL; l += nt)
+            for (int d = 0; d < D; ++d)
+              Yl[e * D + d] = Ul[l * D + d] * cols.bbsize[s * D + d] + cols.bbmin[s * D + d];
+            if (lines)
+              for (int b = l; b < P1; b += NL)
+                Y0[g * P1 + b] = U0[b] * cols.bbsize[s * D] + cols.bbmin[s * D];
+          }
+        } else {
+          for (int g = 0; g < ns; ++g) {
+            const int64_t s = pat.far_src[f + g];
+            T bs[D], bm[D];
 #pragma unroll
-            for (int d = 0; d < D; ++d) Yl[(g * NL + l) * D + d] = Ul[l * D + d] * bs[d] + bm[d];
-          if (lines)
-            for (int b = threadIdx.x; b < P1; b += nt) Y0[g * P1 + b] = U0[b] * bs[0] + bm[0];
+            for (int d = 0; d < D; ++d) {
+              bs[d] = cols.bbsize[s * D + d];
+              bm[d] = cols.bbmin[s * D + d];
+            }
+            const T *ms = mom + s * q * nrhs + rc;
+            for (int j = threadIdx.x; j < q; j += nt)
+#pragma unroll
+              for (int r = 0; r < NR; ++r)
+                Mv[(g * q + j) * NR + r] = r < nr ? ms[(int64_t)j * nrhs + r] : T(0);
+            for (int l = threadIdx.x; l < NL; l += nt)
+#pragma unroll
+              for (int d = 0; d < D; ++d)
+                Yl[(g * NL + l) * D + d] = Ul[l * D + d] * bs[d] + bm[d];
+            if (lines)
+              for (int b = threadIdx.x; b < P1; b += nt) Y0[g * P1 + b] = U0[b] * bs[0] + bm[0];
+          }
         }
         __syncthreads();
         if (!act) continue;
@@ -484,16 +517,27 @@ size_t coupling_lds(int P1, int q, bool single, int G, int nt) {
 
 constexpr size_t kValuLds = 63 * 1024;  // with the static table at most 64 KB
 
+// Most slices of a workgroup whose list has `sources` sources: a slice of fewer
+// than four costs more in add_slices than it saves (FP32 leaf output, 7 columns,
+// against one row a thread: at worst 0.77 of its speed with up to 32 slices
+// whatever the list, 1.07 with four sources a slice, 0.83 with sixteen).
+inline int valu_slices(double sources) {
+  return (int)std::max(1.0, std::min(32.0, sources / 4));
+}
+
 // Workgroup size for targets of `rows` rows: the one of 64, 128 and 256
 // threads whose lanes the slices use best; of nearly equal ones (4 %) the
-// smaller (cheaper barriers, finer scheduling).
-inline int valu_threads(double rows, int rpt) {
+// smaller (cheaper barriers, finer scheduling).  `whole`: split tasks, whose
+// launch is not cut into parts, take 256 threads for more than 64 rows (2-D
+// degree 7, clusters, FP64 leaf output, 1 rhs: 64 threads 2.39 ms, 256 0.74).
+inline int valu_threads(double rows, int rpt, int smax, bool whole) {
   int best = 256;
   double top = -1;
   for (int nt : {64, 128, 256}) {
+    if (whole && nt < 256 && rows > 64) continue;
     const int r = std::max(1, (int)std::min<double>(nt, std::ceil(rows)));
     const int nh = (r + rpt - 1) / rpt;
-    const int S = std::min(nt / nh, 32);
+    const int S = std::min(nt / nh, smax);
     // passes of nt rows: the last one is partly filled
     const double passes = std::ceil(std::max(1.0, rows) / nt);
     const double use = passes > 1 ? rows / (passes * nt) * ((double)S * nh / nt)
@@ -513,29 +557,39 @@ hipError_t valu_launch(bool output, const ValuLaunch<T> &a) {
   T *slabs = nullptr;
   if (output) {
     if (a.pat.nnear_order <= 0) return hipSuccess;
+    const int smax = valu_slices(a.pat.near_per_task);
     const int nt = valu_threads(a.rows.nleaves > 0 ? (double)a.rows.npts / a.rows.nleaves : 1,
-                                kRowsPerThread<T, D, NR, true>);
+                                kRowsPerThread<T, D, NR, true>, smax, a.pat.nnear_split > 0);
     parts = phase_parts(a.pat.nnear_order, a.pat.nnear_split, nt / 64, a.pat.near_per_task, nt,
                         a.rows.npts * a.nrhs, a.part_cap);
     if (parts > 1 && !(slabs = a.part(parts * a.rows.npts * a.nrhs))) parts = 1;
     hipLaunchKernelGGL((k_leaf_output<T, D, KT, NR, GEO>),
                        dim3(a.pat.nnear_order, (unsigned)parts), dim3(nt),
                        (output_lds<T, D, NR>(P1, nt)), a.stream, a.rows, a.cols, a.pat, a.ip,
-                       a.kp, a.nrhs, a.xs, a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, slabs);
+                       a.kp, a.nrhs, a.xs, a.tlhs, a.out, a.ldo, a.natural ? 1 : 0, smax, slabs);
   } else {
     if (a.pat.nfar_order <= 0) return hipSuccess;
-    const int nt = valu_threads(q, kRowsPerThread<T, D, NR, false>);
+    const int smax = valu_slices(a.pat.far_per_task * q);
+    const int nt = valu_threads(q, kRowsPerThread<T, D, NR, false>, smax, false);
     const bool single = GEO || a.ip.td;
     // whole sources per tile, up to 512 nodes of one column (fewer of more)
     const int want = NR == 1 ? 512 : (NR <= 4 ? 256 : 128);
+    // (and no more than a usual list has)
     int G = std::max(1, std::min(want / std::max(1, q), 64));
+    G = std::max(1, std::min(G, (int)std::ceil(2 * a.pat.far_per_task)));
     while (G > 1 && coupling_lds<T, D, NR>(P1, q, single, G, nt) > kValuLds / 2) --G;
     parts = phase_parts(a.pat.nfar_order, a.pat.nfar_split, nt / 64, a.pat.far_per_task * q, nt,
                         (int64_t)a.rows.ncl * q * a.nrhs, a.part_cap);
     if (parts > 1 && !(slabs = a.part(parts * (int64_t)a.rows.ncl * q * a.nrhs))) parts = 1;
-    hipLaunchKernelGGL((k_coupling<T, D, KT, NR, GEO>), dim3(a.pat.nfar_order, (unsigned)parts),
-                       dim3(nt), (coupling_lds<T, D, NR>(P1, q, single, G, nt)), a.stream, a.rows,
-                       a.cols, a.pat, a.ip, a.kp, a.nrhs, G, a.mom, a.tlhs, slabs);
+#define FMCA_COUPLING(F)                                                                        \
+  hipLaunchKernelGGL((k_coupling<T, D, KT, NR, GEO, F>), dim3(a.pat.nfar_order, (unsigned)parts), \
+                     dim3(nt), (coupling_lds<T, D, NR>(P1, q, single, G, nt)), a.stream, a.rows,  \
+                     a.cols, a.pat, a.ip, a.kp, a.nrhs, G, smax, a.mom, a.tlhs, slabs)
+    if (q < kWholeSources)
+      FMCA_COUPLING(true);
+    else
+      FMCA_COUPLING(false);
+#undef FMCA_COUPLING
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || parts == 1) return e;
