@@ -1,7 +1,9 @@
 // Matrix-core contractions of the FP32 precision form on BF16 inputs.
 //
-// The kernel entries are evaluated in FP32 exactly as in the FP32 MFMA forms
-// (kernels_mfma.hpp), and so are the right operands (rhs rows, moments).  Each
+// The kernel entries are evaluated in FP32, from squared distances that the BF16
+// matrix cores form from three-term splits (24 bits, see source_operand; the
+// leaf output of kernels with a cusp at 0: from FP32 differences), and so are the
+// right operands (rhs rows, moments).  Each
 // FP32 operand v is split into two BF16 terms, hi = bf16(v) (round to nearest
 // even) and lo = bf16(v - hi), and a product a.b is formed as
 //     a_hi.b_hi + a_lo.b_hi + a_hi.b_lo
@@ -213,13 +215,19 @@ __device__ __forceinline__ void contract(const bf16x8 (&ah)[kRT], const bf16x8 (
 
 // Distance operands.  r^2 = |y|^2 - 2 x.y + |x|^2 of 16 sources and 16 targets
 // comes from one v_mfma_f32_16x16x32_bf16: every coordinate and squared norm is
-// split into three BF16 terms (24 bits), and its k-slots hold, per axis, the
-// six products down to 2^-16 (slots 6 d .. 6 d + 5: y1x1 y1x2 y2x1 y2x2 y1x3
-// y3x1), then |y|^2 against 1 (18-20) and 1 against |x|^2 (21-23); the last
-// eight are zero on the target side.  FP32 products and sums of the
-// instruction: error 0.9-1.0 of 2^-24 (|x|^2 + |y|^2) rms, against 0.7-0.8 for
-// v_mfma_f32_16x16x4, whose 41 cycles do not overlap with the vector ALU (19
-// cycles here, partly hidden).
+// split into three BF16 terms (24 bits), and its k-slots hold 24 products, per
+// axis those down to 2^-16 (y1x1; y1x2 y2x1; y2x2 y1x3 y3x1), |y|^2 against 1 and
+// 1 against |x|^2; the last eight are zero on the target side.  The instruction
+// drops what lies below the last place of its running sum, so the products
+// stand in rising order.  Error of r^2 in units of 2^-24 (|x|^2 + |y|^2), rms,
+// sources around the targets / one / three box widths off: 0.75 / 0.80 / 0.93
+// (mean -0.2 to -0.3), axis by axis 0.90 / 0.93 / 1.04, v_mfma_f32_16x16x4 0.84 /
+// 0.82 / 0.77, whose 41 cycles do not overlap with the vector ALU (19 cycles here,
+// partly hidden).  y2x3 and y3x2 in the free slots change no bit; 32 slots with
+// zeros between the orders give 0.72 / 0.76 / 0.86 and a leaf output of 8.0
+// instead of 7.8 ms (n = 1e6, 32 columns).  The split of the entries and right
+// operands dominates the action's error: 4.1e-6 at n = 5e4, 32 columns, in every
+// one of these layouts (4.4e-6 with the FP32 instruction and its order of sums).
 struct Split3 {
   __bf16 t[3];
   __device__ __forceinline__ explicit Split3(float v) {
@@ -230,27 +238,41 @@ struct Split3 {
     }
   }
 };
-constexpr int kDistGroups = 3;  // eight k-slots each; the fourth group is zero
+constexpr int kDistGroups = 3;         // eight k-slots each; the fourth group is zero
+constexpr int kSlot[3] = {19, 11, 0};  // first slot of the products of 1, 2^-8, 2^-16
+
+// The k-slots of the source operand (SOURCE: of -2 y' and |y'|^2) or of the
+// target operand (of x' and |x'|^2).
+template <int D, bool SOURCE>
+__device__ __forceinline__ void distance_slots(const float (&v)[D], float s2, __bf16 (&k)[24]) {
+  const __bf16 one = (__bf16)1.f;
+#pragma unroll
+  for (int i = 0; i < 24; ++i) k[i] = (__bf16)0.f;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const Split3 u(v[d]);
+    k[kSlot[0] + d] = u.t[0];
+    k[kSlot[1] + 2 * d] = u.t[SOURCE ? 0 : 1];
+    k[kSlot[1] + 2 * d + 1] = u.t[SOURCE ? 1 : 0];
+    k[kSlot[2] + 3 * d] = u.t[1];
+    k[kSlot[2] + 3 * d + 1] = u.t[SOURCE ? 0 : 2];
+    k[kSlot[2] + 3 * d + 2] = u.t[SOURCE ? 2 : 0];
+  }
+  const Split3 u(s2);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int at = kSlot[i] + (i == 0 ? 3 : (i == 1 ? 6 : 9));
+    k[at + (SOURCE ? 0 : 1)] = u.t[i];
+    k[at + (SOURCE ? 1 : 0)] = one;
+  }
+}
 
 // the source operand of -2 y' and |y'|^2: group g of this source
 template <int D>
 __device__ __forceinline__ void source_operand(const float (&y)[D], float s2,
                                                bf16x8 (&out)[kDistGroups]) {
-  const __bf16 zero = (__bf16)0.f, one = (__bf16)1.f;
   __bf16 a[24];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const Split3 u(d < D ? y[d < D ? d : 0] : 0.f);
-    a[6 * d] = a[6 * d + 1] = a[6 * d + 4] = d < D ? u.t[0] : zero;
-    a[6 * d + 2] = a[6 * d + 3] = d < D ? u.t[1] : zero;
-    a[6 * d + 5] = d < D ? u.t[2] : zero;
-  }
-  const Split3 u(s2);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    a[18 + i] = u.t[i];
-    a[21 + i] = one;
-  }
+  distance_slots<D, true>(y, s2, a);
 #pragma unroll
   for (int g = 0; g < kDistGroups; ++g)
 #pragma unroll
@@ -260,27 +282,12 @@ __device__ __forceinline__ void source_operand(const float (&y)[D], float s2,
 // the target operand of x' and |x'|^2: the k-slots of lane group lk
 template <int D>
 __device__ __forceinline__ bf16x8 target_operand(const float (&x)[D], float s2, int lk) {
-  const __bf16 zero = (__bf16)0.f, one = (__bf16)1.f;
-  __bf16 b[32];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const Split3 v(d < D ? x[d < D ? d : 0] : 0.f);
-    b[6 * d] = b[6 * d + 2] = b[6 * d + 5] = d < D ? v.t[0] : zero;
-    b[6 * d + 1] = b[6 * d + 3] = d < D ? v.t[1] : zero;
-    b[6 * d + 4] = d < D ? v.t[2] : zero;
-  }
-  const Split3 v(s2);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    b[18 + i] = one;
-    b[21 + i] = v.t[i];
-  }
-#pragma unroll
-  for (int i = 24; i < 32; ++i) b[i] = zero;
+  __bf16 b[24];
+  distance_slots<D, false>(x, s2, b);
   bf16x8 out;
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    out[i] = lk == 0 ? b[i] : (lk == 1 ? b[8 + i] : (lk == 2 ? b[16 + i] : zero));
+    out[i] = lk == 0 ? b[i] : (lk == 1 ? b[8 + i] : (lk == 2 ? b[16 + i] : (__bf16)0.f));
   return out;
 }
 

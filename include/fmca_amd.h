@@ -38,7 +38,8 @@ enum {
   FMCA_PRECISION_FP64 = 0, /* plain form: every phase in FP64 */
   FMCA_PRECISION_FP32 = 1, /* precision form: FP32 kernel entries and contractions */
   /* precision form with the contractions of the kernel entries on BF16 matrix
-   * cores: FP32 entries and right operands, each split into two BF16 terms
+   * cores: FP32 entries (their squared distances from three-term BF16 products,
+   * about FP32's rounding) and right operands, each split into two BF16 terms
    * (hi = bf16(v), lo = bf16(v - hi)), products hi.hi + lo.hi + hi.lo with
    * FP32 accumulation -- the error class of FP32 entries at 3/16 of the FP32
    * matrix-core cycles.  Used where the FP32 form would use the matrix cores
