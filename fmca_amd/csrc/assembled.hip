@@ -259,8 +259,9 @@ __device__ __forceinline__ void stream_item(const T *__restrict__ A, int K, int 
 // Where the targets are few the lists are cut into grid.y parts (phase_parts),
 // added from their slabs in order: n = 1e5, FP64, 32 rhs has 512 leaves, one
 // round of workgroups that waited for the longest list: output 3.68 -> 2.88 ms
-// in 6 parts, coupling 1.80 -> 1.52 ms (2.9 -> 3.7 TB/s).  Two waves per SIMD
-// are asked for (the FP64 coupling took 263 registers).
+// in 6 parts, coupling 1.80 -> 1.52 ms, the whole product 5.47 -> 4.66 ms (2.9
+// -> 3.4 TB/s).  Two waves per SIMD are asked for (the FP64 coupling took 263
+// registers).
 template <typename T, int NT, int WS, int PF, bool OUTPUT>
 __global__ __launch_bounds__(kTB, 2) void k_stream(DevTreeView<T> rows, DevTreeView<T> cols,
                                                 DevPatternView pat, StoredBlocks<T> st, int q,

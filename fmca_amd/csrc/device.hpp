@@ -308,9 +308,10 @@ template <typename T>
 hipError_t launch_valu(bool output, const ValuLaunch<T> &a);
 
 // Parts of a matrix-core launch of `waves` waves per task, and their slabs.
-// 3 rounds of the 4 resident waves per SIMD.  A part has at least 1024 sources
-// (FP64, whose entries take twice the time: 512): 512 leaves of 68 rows and
-// 1171 sources, FP32, 32 columns, take 109 us whole, 120 us in two parts.
+// kFillWavesMfma is 3 rounds of 4 resident waves per SIMD (BF16, up to 32
+// columns; 4 of the 3 of FP32, 6 of the 2 of FP64).  A part has at least 1024
+// sources (FP64, whose entries take twice the time: 512): 512 leaves of 68 rows
+// and 1171 sources, FP32, 32 columns, take 109 us whole, 120 us in two parts.
 // Fewer than two tasks per CU are cut down to 256 sources (n = 4000, 3-D degree
 // 3, 16 columns: 69 us an action, 99 us with 1024).
 template <typename T>
@@ -407,7 +408,9 @@ hipError_t basis_project(int64_t n, int nrhs, const double *coef, const S *const
 // from n on zero.  Small matrices are 32 x 32, row-major.
 constexpr int kBlockCols = 32;
 // blocks, and columns of a block: blocks of about equal size (33 columns: 17
-// and 16, not 32 and 1, whose single column would converge four times slower)
+// and 16, not 32 and 1, whose single column would converge four times slower).
+// All blocks but the last have block_cols columns, so the last one is short by
+// up to block_groups - 1: it has one column first at 993 = 32 * 31 + 1.
 __host__ __device__ inline int block_groups(int nrhs) {
   return (nrhs + kBlockCols - 1) / kBlockCols;
 }

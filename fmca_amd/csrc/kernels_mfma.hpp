@@ -735,8 +735,9 @@ __global__ __launch_bounds__(256, (kMinWavesGram<T, NT, KT, MULTI>)) void k_coup
     // Chunks are fetched into registers (coordinates py, moments pm) and then
     // written to LDS between two barriers.  FP32 fetches the next chunk right
     // after the barriers, so its global loads overlap the MFMA work of the
-    // current one; FP64 (one wave per SIMD) fetches just before staging, as a
-    // lookahead measured slower there.
+    // current one; FP64 fetches just before staging: its registers are short,
+    // and a lookahead measured slower there (when the kernel ran at one wave per
+    // SIMD; not measured again at the two that it runs at now).
     constexpr int KM = kChunk * NC / 256;          // staged moments per thread
     // staged coordinates per thread (kGram: thread bl < kChunk holds the D
     // coordinates of row bl)
